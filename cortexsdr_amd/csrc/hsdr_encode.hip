@@ -18,6 +18,11 @@
 // Each D element loaded is used for every tile of the workgroup. Then one wave per tile scans
 // the scores (first maximum), and the residuals are updated with one fused multiply-add per
 // element.
+//
+// mp_gram_kernel makes the same picks without a projection per pick: scores start as tile . D^T
+// and follow the residual through D . D^T, an error bound says which atoms can be the
+// reference's pick, and only where that leaves more than one are the exact projections taken
+// (see the comment there). launch_mp chooses between the two.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -26,6 +31,7 @@
 #include <cstring>
 #include <random>
 #include <string>
+#include <type_traits>
 #include <unordered_map>
 #include <vector>
 
@@ -58,6 +64,8 @@ struct MpArgs {
     uint16_t* codes;     // n x S*k, packIndexSign
     long long n;
     int C, K, S, k, tt;
+    const int* list;   // NULL: tiles 0 .. n - 1; else *count tiles by number (TT = 1)
+    const int* count;
     float gamma[kMaxStages];
 };
 
@@ -84,11 +92,9 @@ __device__ __forceinline__ void load_tiles(const float* rc, float* rv) {
 }
 
 template <int TT>
-__global__ __launch_bounds__(kEThreads) void mp_kernel(MpArgs a) {
+__device__ __forceinline__ void mp_tiles(const MpArgs& a, long long t0, int nt) {
     extern __shared__ float smem[];
     const int tt = TT, C = a.C, K = a.K;
-    const long long t0 = (long long)blockIdx.x * tt;
-    const int nt = (int)min((long long)tt, a.n - t0);
     float* r = smem;                                                    // C x TT residuals
     float* proj = r + (size_t)tt * C;                                   // nt x K scores
     uint8_t* used = reinterpret_cast<uint8_t*>(proj + (size_t)tt * K);  // nt x K
@@ -226,8 +232,458 @@ __global__ __launch_bounds__(kEThreads) void mp_kernel(MpArgs a) {
     }
 }
 
+template <int TT>
+__global__ __launch_bounds__(kEThreads) void mp_kernel(MpArgs a) {
+    const long long t0 = (long long)blockIdx.x * TT;
+    mp_tiles<TT>(a, t0, (int)min((long long)TT, a.n - t0));
+}
+
+// The tiles that mp_gram_kernel leaves (list, count).
+__global__ __launch_bounds__(kEThreads) void mp_list_kernel(MpArgs a) {
+    const int n = *a.count;
+    for (int b = blockIdx.x; b < n; b += gridDim.x) mp_tiles<1>(a, a.list[b], 1);
+}
+
 size_t mp_lds_bytes(int tt, int C, int K) {
     return (size_t)tt * ((size_t)C + K) * 4 + csdr::align_up((size_t)tt * K, 16);
+}
+
+// ---------------------------------------------------------------- picks through the Gram matrix
+
+// mp_kernel's K x C projections per tile and pick bound it (36% of the fp32 vector rate). The
+// scores of the next residual are the last ones minus gamma sign (D . D^T)[best], K operations
+// instead of K x C, so here a pick is one row of D . D^T per tile. The picks stay the
+// reference's because its rounding is bounded. With u = 2^-24, N_t the residual's norm, dmax
+// the longest atom's:
+//   * the reference's projection: at most c1 = C / 16 + 16 roundings on any element's way, so
+//     within c1 u dmax N_t of the true dot product with its residual;
+//   * its residual: one rounding per element and pick, t u max N off the true one;
+//   * the scores here: sums in double rounded to float once (u dmax N_0 and, through the Gram
+//     entries, u dmax sum gamma |D_b|), one rounding per pick (t u dmax max N).
+// Their sum is eps. An atom whose score is more than 2 eps below the largest cannot be the
+// pick; a single one left is, with the sign of its score once that exceeds eps. Otherwise
+// (about one pick in 500 on Gaussian tiles, more where D holds an atom twice) the wave brings
+// the residual up to date in LDS with the reference's own fused updates and takes the left
+// atoms' projections in its order, as mp_kernel does. A tile whose norm or atoms are outside
+// [1e-12, 1e12], NaN or infinite, or with more than kGramMaxCand atoms left, goes to a list
+// that mp_list_kernel encodes.
+// One wave per tile: the scores (KPL per lane) stay in registers, a Gram row is KPL coalesced
+// loads from L2, and a pick is bound by that one round trip and the wave's maximum.
+// 4864 x 896, K = 512, 24 picks, with both products: 3.9 ms -> 0.30 ms (picks 119 us, scores
+// about 115, D . D^T about 40); 896 x 896, K = 256, 15 picks: 807 -> 155 us; 3000 x 4096,
+// K = 1024, 8 picks: 12.2 -> 1.0 ms; 300 x 39, K = 48: 74 -> 44 us.
+constexpr int kGramMaxK = 2048;      // 32 scores per lane
+constexpr int kGramMaxC = 8192;      // residual in LDS: 32 KiB per wave
+constexpr int kGramMaxCand = 64;
+constexpr size_t kGramScoreBytes = 64u << 20;  // scores of one chunk of tiles
+
+struct GramArgs {
+    const float* tiles;   // n x C
+    const float* D;       // K x C
+    const float* scores;  // n x K: tile . D^T
+    const float* gram;    // K x K: D . D^T
+    const float* sq;      // K: its diagonal
+    uint16_t* codes;      // n x S*k
+    int* list;            // tiles left to mp_list_kernel, and their count
+    int* count;
+    int C, K, S, k;
+    float gamma[kMaxStages];
+};
+
+// out (M x R) = X (M x C) . W^T (W R x C) with the sums in double (v_mfma_f64_16x16x4_f64),
+// rounded to float. A 64 x 64 tile per 2 x 2 waves, 32-deep stages through LDS with the next
+// stage's loads in flight; the k order within a stage is permuted (step s of lane group g takes
+// k = 8 g + s) so that a lane reads its eight values as one 32-byte run.
+constexpr int kPLd = 36;
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef double doublex4 __attribute__((ext_vector_type(4)));
+
+template <bool VEC>
+__device__ __forceinline__ floatx4 load4(const float* p, int k, int C) {
+    if constexpr (VEC)
+        return k < C ? *reinterpret_cast<const floatx4*>(p + k) : floatx4{0.f, 0.f, 0.f, 0.f};
+    floatx4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = k + i < C ? p[k + i] : 0.f;
+    return v;
+}
+
+template <bool VEC>
+__global__ __launch_bounds__(kEThreads) void dots_f64_kernel(const float* __restrict__ X,
+                                                             long long M,
+                                                             const float* __restrict__ W, int R,
+                                                             int C, float* __restrict__ out,
+                                                             float* diag, int* zero) {
+    __shared__ __attribute__((aligned(16))) float xs[64 * kPLd];
+    __shared__ __attribute__((aligned(16))) float ws[64 * kPLd];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    if (zero && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *zero = 0;
+    const int li = lane & 15, lg = lane >> 4;
+    const long long m0 = (long long)blockIdx.x * 64;
+    const int r0 = blockIdx.y * 64;
+    const int wm = (wave >> 1) * 32, wr = (wave & 1) * 32;
+    const int row = tid >> 3, kq = (tid & 7) * 4;  // and row + 32
+    const float* xp[2];
+    const float* wp[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {  // rows past the end repeat the last one (not stored)
+        xp[j] = X + (size_t)min(m0 + row + 32 * j, M - 1) * C;
+        wp[j] = W + (size_t)min(r0 + row + 32 * j, R - 1) * C;
+    }
+    floatx4 px[2], pw[2];
+    auto load = [&](int k0) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            px[j] = load4<VEC>(xp[j], k0 + kq, C);
+            pw[j] = load4<VEC>(wp[j], k0 + kq, C);
+        }
+    };
+    doublex4 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) acc[a][b] = doublex4{0., 0., 0., 0.};
+    const int nst = (C + 31) / 32;
+    load(0);
+    for (int s = 0; s < nst; ++s) {
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            *reinterpret_cast<floatx4*>(xs + (row + 32 * j) * kPLd + kq) = px[j];
+            *reinterpret_cast<floatx4*>(ws + (row + 32 * j) * kPLd + kq) = pw[j];
+        }
+        __syncthreads();
+        if (s + 1 < nst) load((s + 1) * 32);
+        floatx4 xf[2][2], wf[2][2];
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                xf[a][h] = *reinterpret_cast<const floatx4*>(xs + (wm + a * 16 + li) * kPLd +
+                                                             lg * 8 + 4 * h);
+                wf[a][h] = *reinterpret_cast<const floatx4*>(ws + (wr + a * 16 + li) * kPLd +
+                                                             lg * 8 + 4 * h);
+            }
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+            const double x0 = xf[0][q >> 2][q & 3], x1 = xf[1][q >> 2][q & 3];
+            const double w0 = wf[0][q >> 2][q & 3], w1 = wf[1][q >> 2][q & 3];
+            acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, w0, acc[0][0], 0, 0, 0);
+            acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x0, w1, acc[0][1], 0, 0, 0);
+            acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, w0, acc[1][0], 0, 0, 0);
+            acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(x1, w1, acc[1][1], 0, 0, 0);
+        }
+    }
+    // the f64 form: lane holds D[4 v + l / 16][l % 16], X rows along the MFMA's rows
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int r = r0 + wr + b * 16 + li;
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const long long m = m0 + wm + a * 16 + 4 * v + lg;
+                if (m < M && r < R) {
+                    out[(size_t)m * R + r] = (float)acc[a][b][v];
+                    if (diag && m == r) diag[r] = (float)acc[a][b][v];
+                }
+            }
+        }
+}
+
+// max over the wave of values >= 0 (NaN dropped), in every lane: DPP rows, then broadcasts
+__device__ __forceinline__ float wave_max(float v) {
+    const auto step = [&](auto ctrl, auto rows) {
+        const int o = __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v),
+                                                  decltype(ctrl)::value, decltype(rows)::value,
+                                                  0xf, false);
+        v = fmaxf(v, __builtin_bit_cast(float, o));
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr 1, 2, 4, 8
+    step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
+    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row 0 / 2 into 1 / 3
+    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row 1 into 2, 3
+    return __builtin_bit_cast(float,
+                              __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
+}
+
+template <int KPL>
+__global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
+    extern __shared__ float smem[];
+    const int C = a.C, K = a.K, lane = threadIdx.x, slots = a.S * a.k;
+    float* r = smem;                                           // C: the exact residual, when needed
+    float* hgam = r + C;                                       // slots: gamma * sign of the picks
+    uint16_t* hist = reinterpret_cast<uint16_t*>(hgam + slots);  // and their atoms
+    uint16_t* cand = hist + ((slots + 1) & ~1);                // kGramMaxCand: atoms left
+    const int tile = blockIdx.x;
+    const float* x = a.tiles + (size_t)tile * C;
+    float s[KPL];
+    uint32_t out_of = 0;  // atoms past K
+    int jc[KPL];          // this lane's atoms, clamped
+#pragma unroll
+    for (int i = 0; i < KPL; ++i) {
+        const int j = lane + 64 * i;
+        jc[i] = min(j, K - 1);
+        s[i] = a.scores[(size_t)tile * K + jc[i]];
+        if (j >= K) out_of |= 1u << i;
+    }
+    float dm = 0.f;
+    bool odd = false;  // NaN or infinite (fmaxf would drop a NaN)
+    for (int j = lane; j < K; j += 64) {
+        const float g = a.sq[j];
+        dm = fmaxf(dm, g);
+        odd |= !(g >= 0.f);
+    }
+    const float dmax = __builtin_amdgcn_sqrtf(wave_max(dm)) * 1.01f;
+    // the tile's norm, scaled by its largest magnitude
+    float mx = 0.f;
+    for (int c = lane; c < C; c += 64) {
+        mx = fmaxf(mx, fabsf(x[c]));
+        odd |= !(fabsf(x[c]) < INFINITY);
+    }
+    mx = wave_max(mx);
+    float n2 = 0.f;
+    if (mx > 0.f)
+        for (int c = lane; c < C; c += 64) {
+            const float v = x[c] / mx;
+            n2 = fmaf(v, v, n2);
+        }
+    const float n0 = mx > 0.f ? mx * __builtin_amdgcn_sqrtf(csdr::wave_sum(n2)) * 1.01f : 0.f;
+    const auto leave = [&] {
+        if (lane == 0) a.list[atomicAdd(a.count, 1)] = tile;
+    };
+    if (__any(odd) || !(dmax >= 1e-12f && dmax <= 1e12f) ||
+        !(n0 == 0.f || (n0 >= 1e-12f && n0 <= 1e12f))) {
+        leave();
+        return;
+    }
+    const float u = 1.25f * 5.9604645e-8f * dmax;
+    float rn2 = n0 * n0, nmax2 = rn2, len = 0.f;
+    int upto = -1;  // picks applied to r (-1: r not loaded)
+    int t = 0;
+    for (int l = 0; l < a.S; ++l) {
+        uint32_t used = out_of;
+        const float gl = a.gamma[l];
+        for (int st = 0; st < a.k; ++st, ++t) {
+            float v[KPL];  // |score|, -1 for atoms used in this stage
+            float m = 0.f;
+#pragma unroll
+            for (int i = 0; i < KPL; ++i) {
+                v[i] = used >> i & 1 ? -1.f : fabsf(s[i]);
+                m = fmaxf(m, v[i]);
+            }
+            m = wave_max(m);
+            const float nmax = __builtin_amdgcn_sqrtf(nmax2) * 1.01f;
+            const float nt =
+                __builtin_amdgcn_sqrtf(rn2 + (1e-4f + 1e-6f * (float)t) * nmax2) * 1.01f;
+            const float eps =
+                u * ((float)(C / 16 + 16) * nt + (float)(2 * t) * nmax + n0 + len) + 1e-38f;
+            if (!(m <= 1e30f && len <= 1e15f && eps < 1e30f)) {
+                leave();
+                return;
+            }
+            const float thr = m - 2.f * eps;
+            // the atoms left: NaN stays in; a used one's -1 may only come in with thr < -1,
+            // where eps is far past any score
+            uint64_t left[KPL];
+            int nc = 0;
+#pragma unroll
+            for (int i = 0; i < KPL; ++i) {
+                left[i] = __ballot(!(v[i] < thr) && !(used >> i & 1));
+                nc += __popcll(left[i]);
+            }
+            int bi = 0, sg = 1;
+            if (nc == 1 && m > eps) {
+                float sv = 0.f;
+#pragma unroll
+                for (int i = 0; i < KPL; ++i)
+                    if (left[i]) {  // one of them
+                        const int src = __ffsll((unsigned long long)left[i]) - 1;
+                        bi = 64 * i + src;
+                        sv = __builtin_bit_cast(
+                            float,
+                            __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[i]), src));
+                    }
+                sg = sv >= 0.f ? 1 : -1;
+            } else if (n0 == 0.f && t == 0) {
+                // a zero tile: every projection is 0, atom 0 stands
+            } else if (nc > kGramMaxCand) {
+                leave();
+                return;
+            } else {
+                // the residual up to date, as the reference updates it; four elements a lane
+                // at a time, so that every pick's loads are independent of the last one's
+                for (int c0 = lane; c0 < C; c0 += 256) {
+                    float rv[4];
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        rv[e] = upto < 0 ? x[min(c0 + 64 * e, C - 1)] : r[min(c0 + 64 * e, C - 1)];
+#pragma unroll 4
+                    for (int q = max(upto, 0); q < t; ++q) {
+                        const uint16_t h = hist[q];
+                        const float sc = hgam[q];
+                        const float* d = a.D + (size_t)h * C;
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            rv[e] = fmaf(-d[min(c0 + 64 * e, C - 1)], sc, rv[e]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (c0 + 64 * e < C) r[c0 + 64 * e] = rv[e];
+                }
+                upto = t;
+                int n = 0;  // the atoms left, in ascending order
+#pragma unroll
+                for (int i = 0; i < KPL; ++i) {
+                    if (left[i] >> lane & 1)
+                        cand[n + __popcll(left[i] & ((1ull << lane) - 1))] =
+                            (uint16_t)(lane + 64 * i);
+                    n += __popcll(left[i]);
+                }
+                __syncthreads();
+                // their projections in the reference's order, one per 16 lanes
+                const int l16 = lane & 15, grp = lane >> 4;
+                const int C16 = C & ~15, C8 = C & ~7;
+                float bv = 0.f;  // sg: atom 0 used in this stage scores 0, a positive sign
+                for (int q = 0; q < nc; q += 4) {
+                    const int j = cand[min(q + grp, nc - 1)];
+                    const float* d = a.D + (size_t)j * C;
+                    float p = 0.f;
+#pragma unroll 8
+                    for (int c = l16; c < C16; c += 16) p = fmaf(d[c], r[c], p);
+                    if (C8 > C16 && l16 < 8) p = fmaf(d[C16 + l16], r[C16 + l16], p);
+                    p += __shfl_xor(p, 8, 16);
+                    p += __shfl_xor(p, 4, 16);
+                    p += __shfl_xor(p, 1, 16);
+                    p += __shfl_xor(p, 2, 16);
+                    for (int c = C8; c < C; ++c) p = fmaf(d[c], r[c], p);
+                    if (fabsf(p) > bv) {  // ascending within a group: the first maximum
+                        bv = fabsf(p);
+                        bi = j;
+                        sg = p >= 0.f ? 1 : -1;
+                    } else if (j == 0 && bv == 0.f) {
+                        sg = p >= 0.f ? 1 : -1;
+                    }
+                }
+                // group 0 holds atom 0 when it is left: with no score above 0 its sign stands
+#pragma unroll
+                for (int off = 16; off <= 32; off <<= 1) {
+                    const float ov = __shfl_xor(bv, off, 64);
+                    const int oi = __shfl_xor(bi, off, 64), os = __shfl_xor(sg, off, 64);
+                    if (ov > bv || (ov == bv && (oi < bi || (ov == 0.f && os < sg)))) {
+                        bv = ov;
+                        bi = oi;
+                        sg = os;
+                    }
+                }
+                bi = __builtin_amdgcn_readfirstlane(bi);
+                sg = __builtin_amdgcn_readfirstlane(sg);
+            }
+            const float sc = gl * (float)sg;
+            const float* g = a.gram + (size_t)bi * K;
+            const float gb = a.sq[bi];
+            float sb = 0.f;
+#pragma unroll
+            for (int i = 0; i < KPL; ++i) {
+                if (i == bi >> 6)
+                    sb = __builtin_bit_cast(
+                        float,
+                        __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[i]), bi & 63));
+                s[i] = fmaf(-sc, g[jc[i]], s[i]);
+            }
+            if (lane == (bi & 63)) used |= 1u << (bi >> 6);
+            if (lane == 0) {
+                a.codes[(size_t)tile * slots + t] =
+                    (uint16_t)((bi & 0x7FFF) | (sg < 0 ? 0x8000 : 0));
+                hist[t] = (uint16_t)bi;
+                hgam[t] = sc;
+            }
+            rn2 += sc * (sc * gb - 2.f * sb);
+            rn2 = rn2 >= 0.f ? rn2 : rn2 < 0.f ? 0.f : INFINITY;  // NaN: the tile leaves
+            len += fabsf(sc) * __builtin_amdgcn_sqrtf(gb) * 1.01f;
+            nmax2 = fmaxf(nmax2, rn2);
+            __syncthreads();  // hist and cand before the next pick's reads and writes
+        }
+    }
+}
+
+// Workspace of the Gram path: the scores of a chunk of tiles, the Gram matrix, its
+// diagonal, the numbers of a chunk's tiles left to mp_list_kernel and their count.
+long long gram_chunk(long long n, int K) {
+    return std::min<long long>(n, std::max<long long>(64, (long long)(kGramScoreBytes / 4) / K));
+}
+size_t gram_ws_bytes(long long n, int K) {
+    const size_t chunk = (size_t)gram_chunk(n, K);
+    return csdr::align_up(chunk * K * 4, 256) + csdr::align_up((size_t)K * K * 4, 256) +
+           ((size_t)K + chunk + 1) * 4;
+}
+
+// The Gram path does 2 (n + K) K C operations where mp_kernel does 2 n picks K C.
+bool gram_pays(long long n, int C, int K, int S, int k) {
+    return K <= kGramMaxK && C <= kGramMaxC && 2 * n * S * k >= n + K &&
+           !std::getenv("CSDR_HSDR_TILES_PER_WG");  // that override names mp_kernel's form
+}
+
+int launch_dots(const float* X, long long M, const float* W, int R, int C, float* out,
+                float* diag, int* zero, hipStream_t st) {
+    const dim3 grid((unsigned)((M + 63) / 64), (unsigned)((R + 63) / 64));
+    if (C % 4 == 0 && reinterpret_cast<uintptr_t>(X) % 16 == 0 &&
+        reinterpret_cast<uintptr_t>(W) % 16 == 0)
+        dots_f64_kernel<true><<<grid, kEThreads, 0, st>>>(X, M, W, R, C, out, diag, zero);
+    else
+        dots_f64_kernel<false><<<grid, kEThreads, 0, st>>>(X, M, W, R, C, out, diag, zero);
+    CSDR_LAUNCH_CHECK("hsdr_encode products");
+    return CSDR_OK;
+}
+
+int launch_mp_gram(const float* tiles, long long n, int C, const float* D, int K, int S, int k,
+                   const float* gamma, uint16_t* codes, void* ws, hipStream_t st) {
+    const long long chunk = gram_chunk(n, K);
+    char* w = static_cast<char*>(ws);
+    float* scores = reinterpret_cast<float*>(w);
+    w += csdr::align_up((size_t)chunk * K * 4, 256);
+    float* gram = reinterpret_cast<float*>(w);
+    w += csdr::align_up((size_t)K * K * 4, 256);
+    float* sq = reinterpret_cast<float*>(w);
+    int* count = reinterpret_cast<int*>(sq + K);
+    int rc = launch_dots(D, K, D, K, C, gram, sq, nullptr, st);
+    if (rc != CSDR_OK) return rc;
+    GramArgs a{};
+    MpArgs b{};
+    a.D = b.D = D;
+    a.scores = scores;
+    a.gram = gram;
+    a.sq = sq;
+    a.C = b.C = C;
+    a.K = b.K = K;
+    a.S = b.S = S;
+    a.k = b.k = k;
+    a.count = count;
+    a.list = count + 1;
+    b.count = count;
+    b.list = count + 1;
+    for (int l = 0; l < S; ++l) a.gamma[l] = b.gamma[l] = gamma[l];
+    const size_t lds = (size_t)(C + S * k) * 4 + (size_t)(((S * k + 1) & ~1) + kGramMaxCand) * 2;
+    const size_t list_lds = mp_lds_bytes(1, C, K);
+    for (long long t0 = 0; t0 < n; t0 += chunk) {
+        const long long nt = std::min(chunk, n - t0);
+        a.tiles = b.tiles = tiles + (size_t)t0 * C;
+        a.codes = b.codes = codes + (size_t)t0 * S * k;
+        b.n = nt;
+        rc = launch_dots(a.tiles, nt, D, K, C, scores, nullptr, count, st);
+        if (rc != CSDR_OK) return rc;
+        const unsigned grid = (unsigned)nt;
+        if (K <= 256) mp_gram_kernel<4><<<grid, 64, lds, st>>>(a);
+        else if (K <= 512) mp_gram_kernel<8><<<grid, 64, lds, st>>>(a);
+        else if (K <= 1024) mp_gram_kernel<16><<<grid, 64, lds, st>>>(a);
+        else mp_gram_kernel<32><<<grid, 64, lds, st>>>(a);
+        mp_list_kernel<<<(unsigned)std::min<long long>(nt, 1024), kEThreads, list_lds, st>>>(b);
+        CSDR_LAUNCH_CHECK("hsdr_encode");
+    }
+    return CSDR_OK;
 }
 
 // Tiles per workgroup: about n / 1024, at least 2 (measured on the Qwen2-0.5B shapes, 1-row
@@ -255,9 +711,11 @@ int check_mp_shape(long long n, int C, int K, int S, int k) {
     return CSDR_OK;
 }
 
+// gram_ws: gram_ws_bytes(n, K) of device memory, or NULL for mp_kernel.
 int launch_mp(const float* tiles, long long n, int C, const float* D, int K, int S, int k,
-              const float* gamma, uint16_t* codes, hipStream_t st) {
+              const float* gamma, uint16_t* codes, void* gram_ws, hipStream_t st) {
     if (n == 0) return CSDR_OK;
+    if (gram_ws) return launch_mp_gram(tiles, n, C, D, K, S, k, gamma, codes, gram_ws, st);
     MpArgs a{};
     a.tiles = tiles;
     a.D = D;
@@ -559,7 +1017,9 @@ int fit_tiles(const std::vector<float>& tiles, uint32_t n_tiles, uint32_t tile_d
     csdr::hsdr_init_dictionary(tiles.data(), n_tiles, tile_dim, K, (uint32_t)S * k, D.data(),
                                &rng);
     const size_t ncodes = (size_t)n_tiles * S * k;
-    DevBuf d_tiles, d_D, d_codes;
+    DevBuf d_tiles, d_D, d_codes, d_gram;
+    if (gram_pays(n_tiles, (int)tile_dim, K, S, k))
+        CSDR_HIP_CHECK(hipMalloc(&d_gram.p, gram_ws_bytes(n_tiles, K)));
     CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, std::max<size_t>(tiles.size(), 1) * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_D.p, D.size() * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
@@ -567,7 +1027,7 @@ int fit_tiles(const std::vector<float>& tiles, uint32_t n_tiles, uint32_t tile_d
                                   hipMemcpyHostToDevice, st));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_D.p, D.data(), D.size() * 4, hipMemcpyHostToDevice, st));
     rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
-                   d_codes.u16(), st);
+                   d_codes.u16(), d_gram.p, st);
     if (rc != CSDR_OK) return rc;
     if (ksvd_iters) {
         Refine rf;
@@ -577,7 +1037,7 @@ int fit_tiles(const std::vector<float>& tiles, uint32_t n_tiles, uint32_t tile_d
             rc = rf.pass(g, tiles, gamma, d_tiles.f(), d_D.f(), d_codes.u16(), rng, st);
             if (rc != CSDR_OK) return rc;
             rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
-                           d_codes.u16(), st);
+                           d_codes.u16(), d_gram.p, st);
             if (rc != CSDR_OK) return rc;
         }
         CSDR_HIP_CHECK(hipMemcpyAsync(D.data(), d_D.p, D.size() * 4, hipMemcpyDeviceToHost, st));
@@ -601,7 +1061,9 @@ int encode_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, const 
     int rc = check_mp_shape(n_tiles, (int)tile_dim, K, S, k);
     if (rc != CSDR_OK) return rc;
     const size_t ncodes = (size_t)n_tiles * S * k;
-    DevBuf d_tiles, d_D, d_codes;
+    DevBuf d_tiles, d_D, d_codes, d_gram;
+    if (gram_pays(n_tiles, (int)tile_dim, K, S, k))
+        CSDR_HIP_CHECK(hipMalloc(&d_gram.p, gram_ws_bytes(n_tiles, K)));
     CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, std::max<size_t>((size_t)n_tiles * tile_dim, 1) * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_D.p, D.size() * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
@@ -609,7 +1071,7 @@ int encode_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, const 
                                   hipMemcpyHostToDevice, st));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_D.p, D.data(), D.size() * 4, hipMemcpyHostToDevice, st));
     rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
-                   d_codes.u16(), st);
+                   d_codes.u16(), d_gram.p, st);
     if (rc != CSDR_OK) return rc;
     codes.resize(ncodes);
     CSDR_HIP_CHECK(hipMemcpyAsync(codes.data(), d_codes.p, ncodes * 2, hipMemcpyDeviceToHost, st));
@@ -665,8 +1127,22 @@ CSDR_API int csdr_hsdr_encode(const float* tiles, size_t n_tiles, int tile_dim, 
         return set_error(CSDR_E_INVALID, "hsdr_encode: null pointer");
     const int rc = check_mp_shape((long long)n_tiles, tile_dim, n_atoms, n_stages, k_per_stage);
     if (rc != CSDR_OK) return rc;
-    return launch_mp(tiles, (long long)n_tiles, tile_dim, D, n_atoms, n_stages, k_per_stage,
-                     stage_scales, codes, static_cast<hipStream_t>(hip_stream));
+    // The Gram path's workspace is stream-ordered memory; a stream under capture (or one whose
+    // state cannot be asked for) and an allocation that fails keep mp_kernel, which needs none.
+    hipStream_t st = static_cast<hipStream_t>(hip_stream);
+    void* ws = nullptr;
+    if (n_tiles && gram_pays((long long)n_tiles, tile_dim, n_atoms, n_stages, k_per_stage)) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusActive;
+        if (hipStreamIsCapturing(st, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+            hipMallocAsync(&ws, gram_ws_bytes((long long)n_tiles, n_atoms), st) != hipSuccess) {
+            ws = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+    const int mrc = launch_mp(tiles, (long long)n_tiles, tile_dim, D, n_atoms, n_stages,
+                              k_per_stage, stage_scales, codes, ws, st);
+    if (ws) (void)hipFreeAsync(ws, st);
+    return mrc;
 }
 
 CSDR_API int csdr_hsdr_init_dictionary(const float* tiles, uint32_t n_tiles, uint32_t tile_dim,

@@ -85,6 +85,29 @@ def test_encode_tiles_per_workgroup_match_oracle(gpu, monkeypatch, tt, n, C, K, 
     assert np.array_equal(got, want), f"TT={tt}"
 
 
+# The Gram-matrix form of matching pursuit against the oracle where its bound has to give way:
+# atoms held twice (exact ties), zero tiles, tiles far outside the bounded range, zero atoms,
+# K off the wave's multiples and each scores-per-lane size, unaligned tile lengths.
+@pytest.mark.parametrize("n,C,K,S,k", [(200, 64, 65, 3, 4), (130, 39, 256, 2, 5),
+                                       (150, 100, 300, 2, 4), (90, 200, 520, 2, 3),
+                                       (70, 33, 1030, 1, 5), (65, 8, 8, 2, 8)])
+def test_encode_ties_and_odd_tiles_match_oracle(gpu, monkeypatch, n, C, K, S, k):
+    monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
+    rng = np.random.default_rng(n + C + K)
+    t = (rng.standard_normal((n, C)) * 0.02).astype(np.float32)
+    t[3] = 0
+    t[5] *= np.float32(1e-20)
+    t[6] *= np.float32(1e15)
+    t[8] = t[9]
+    D = t[rng.integers(16, n, K)].copy()   # duplicates, and atoms that are tiles
+    D /= np.linalg.norm(D, axis=1, keepdims=True)
+    D *= 0.02 * np.sqrt(C / (S * k))
+    D[K // 2] = 0
+    D = D.astype(np.float32)
+    g = (0.5 ** np.arange(S)).astype(np.float32)
+    assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), oracle.hsdr_mp(t, D, g, S, k))
+
+
 def test_encode_large_tile_falls_back_to_one_per_workgroup(gpu, monkeypatch):
     # 2 x (C + K) x 4 bytes > 64 KiB: the natural choice is one tile per workgroup
     monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
