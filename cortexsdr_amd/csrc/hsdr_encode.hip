@@ -749,90 +749,228 @@ int launch_mp(const float* tiles, long long n, int C, const float* D, int K, int
 // ---------------------------------------------------------------- K-SVD atom update
 
 // atomUpdateStep (HierarchicalSDRStrategy.cpp:281-490) on the device, per refinement pass:
-//  residual_kernel: residual = tile - sum over slots of gamma_l * sign * D[idx], one thread
-//    per element, slots in order, each term fused (the reference's r[c] += scale * atom[c],
-//    :300-311), then tile - recon (:316-320);
-//  atom_update_kernel: one workgroup per atom with users; correction[c] = sum over the atom's
-//    users, in (tile, slot) order, of sign * gamma * residual (double, fused: :428-437), the
-//    new value atom + correction * (0.5 / sum gamma^2) rounded to float (:448-458), a
-//    non-finite value flags the atom for the host's re-seed (:461), the squared norm summed
-//    in element order as the reference's loop does (:456), and atoms longer than the cap
-//    scaled back to the target norm (:482-487). Atoms without users are re-seeded by the
-//    host (:411-425).
-struct ResArgs {
+//  users_count / scan / fill: every atom's users in (tile, slot) order (:325-339) with their
+//    sign * gamma, and 0.5 / the sum of gamma^2 over them in that order (fused, :428-437; 0
+//    when the sum is <= 1e-12). Counts by LDS histograms, one workgroup scans them, and one
+//    workgroup per atom then walks all codes: thread t takes the t-th run of them, counts its
+//    users, and writes them behind those of the threads before it. On the host this was a
+//    copy of the codes, a synchronisation and 0.5 ms per pass;
+//  residual_kernel: residual = tile - sum over slots of gamma_l * sign * D[idx], slots in
+//    order, each term fused (the reference's r[c] += scale * atom[c], :300-311), then tile -
+//    recon (:316-320). A workgroup per tile: its codes are uniform (scalar loads) and a thread
+//    keeps 4 elements, with the next slots' atom rows in flight (84 -> RES_US us at 4864 x 896,
+//    24 slots: a thread per element with a 64-bit division each);
+//  atom_sum_kernel: correction[c] = sum over the atom's users, in order, of sign * gamma *
+//    residual (double, fused: :428-437), the new value atom + correction * (0.5 / sum gamma^2)
+//    rounded to float (:448-458). One thread per element; the users' rows are L2 reads whose
+//    latency bounds it, so a workgroup takes 256 elements of one atom (K x C / 256 of them)
+//    and eight rows are in flight;
+//  atom_finish_kernel: per atom, a non-finite value flags it for the host's re-seed (:461), the
+//    squared norm is summed in element order as the reference's loop does (:456), and atoms
+//    longer than the cap are scaled back to the target norm (:482-487). Atoms without users
+//    are re-seeded by the host (:411-425). Sum and finish: 273 -> UPD_US us at K = 512.
+struct FitArgs {
     const float* tiles;
-    const float* D;
     const uint16_t* codes;
-    float* res;
-    long long n;
-    int C, S, k;
+    float* D;
+    float* nv;      // K x C new values
+    float* res;     // n x C
+    int* off;       // K + 1
+    uint32_t* utile;
+    double* ucoef;
+    double* inv_w;  // K
+    uint8_t* flag;  // K
+    long long n, ncodes;
+    int C, K, S, k;
+    double cap, target;
     float gamma[kMaxStages];
 };
 
-__global__ __launch_bounds__(kEThreads) void residual_kernel(ResArgs a) {
-    const long long total = a.n * a.C;
+__global__ __launch_bounds__(kEThreads) void users_count_kernel(FitArgs a) {
+    extern __shared__ int hist_s[];
+    for (int j = threadIdx.x; j < a.K; j += kEThreads) hist_s[j] = 0;
+    __syncthreads();
+    for (long long i = (long long)blockIdx.x * kEThreads + threadIdx.x; i < a.ncodes;
+         i += (long long)gridDim.x * kEThreads)
+        atomicAdd(&hist_s[a.codes[i] & 0x7FFF], 1);
+    __syncthreads();
+    for (int j = threadIdx.x; j < a.K; j += kEThreads)
+        if (hist_s[j]) atomicAdd(&a.off[j + 1], hist_s[j]);
+}
+
+// Exclusive prefix sum over `v` of a 256-thread workgroup; the total in *total.
+__device__ __forceinline__ int block_scan(int v, int* total) {
+    __shared__ int wsum[kEThreads / 64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    int x = v;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const int y = __shfl_up(x, off, 64);
+        if (lane >= off) x += y;
+    }
+    if (lane == 63) wsum[wave] = x;
+    __syncthreads();
+    int before = 0, sum = 0;
+#pragma unroll
+    for (int w = 0; w < kEThreads / 64; ++w) {
+        if (w < wave) before += wsum[w];
+        sum += wsum[w];
+    }
+    __syncthreads();
+    *total = sum;
+    return before + x - v;
+}
+
+__global__ __launch_bounds__(kEThreads) void users_zero_kernel(FitArgs a) {
+    for (int j = blockIdx.x * kEThreads + threadIdx.x; j <= a.K; j += gridDim.x * kEThreads)
+        a.off[j] = 0;
+}
+
+__global__ __launch_bounds__(kEThreads) void users_scan_kernel(FitArgs a) {
+    int base = 0;
+    for (int j0 = 0; j0 < a.K; j0 += kEThreads) {
+        const int j = j0 + threadIdx.x;
+        const int c = j < a.K ? a.off[j + 1] : 0;
+        int total;
+        const int e = block_scan(c, &total);
+        if (j < a.K) a.off[j + 1] = base + e + c;
+        base += total;
+    }
+}
+
+__global__ __launch_bounds__(kEThreads) void users_fill_kernel(FitArgs a) {
+    __shared__ double gm_s[kEThreads];
+    const int j = blockIdx.x, tid = threadIdx.x;
+    const int u0 = a.off[j], u1 = a.off[j + 1];
     const int slots = a.S * a.k;
-    for (long long e = (long long)blockIdx.x * kEThreads + threadIdx.x; e < total;
-         e += (long long)gridDim.x * kEThreads) {
-        const long long i = e / a.C;
-        const int c = (int)(e - i * a.C);
-        const uint16_t* cd = a.codes + i * slots;
-        float rec = 0.0f;
-        for (int sl = 0; sl < slots; ++sl) {
-            const uint16_t v = cd[sl];
-            const float scale = a.gamma[sl / a.k] * ((v & 0x8000) ? -1.0f : 1.0f);
-            rec = fmaf(scale, a.D[(size_t)(v & 0x7FFF) * a.C + c], rec);
+    const uint16_t want = (uint16_t)j;
+    // runs of a multiple of 8 codes, read 16 bytes at a time (codes is 16-byte aligned)
+    const long long run = (a.ncodes + (long long)kEThreads * 8 - 1) / (kEThreads * 8) * 8;
+    const long long i0 = min(tid * run, a.ncodes), i1 = min(i0 + run, a.ncodes);
+    auto walk = [&](auto&& use) {
+        long long i = i0;
+        for (; i + 8 <= i1; i += 8) {
+            const uint4 w = *reinterpret_cast<const uint4*>(a.codes + i);
+            const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                if ((ws[q] & 0x7FFF) == want) use(i + 2 * q, (uint16_t)ws[q]);
+                if ((ws[q] >> 16 & 0x7FFF) == want) use(i + 2 * q + 1, (uint16_t)(ws[q] >> 16));
+            }
         }
-        a.res[e] = a.tiles[e] - rec;
+        for (; i < i1; ++i)
+            if ((a.codes[i] & 0x7FFF) == want) use(i, a.codes[i]);
+    };
+    int mine = 0;
+    if (u1 > u0) walk([&](long long, uint16_t) { ++mine; });
+    int total;
+    int p = u0 + block_scan(mine, &total);
+    if (mine)
+        walk([&](long long i, uint16_t v) {
+            const long long tile = i / slots;
+            const double gm = (double)a.gamma[(int)(i - tile * slots) / a.k];
+            a.utile[p] = (uint32_t)tile;
+            a.ucoef[p] = (v & 0x8000) ? -gm : gm;
+            ++p;
+        });
+    __syncthreads();
+    double w = 0.0;  // thread 0
+    for (int b = u0; b < u1; b += kEThreads) {
+        gm_s[tid] = b + tid < u1 ? a.ucoef[b + tid] : 0.0;
+        __syncthreads();
+        if (tid == 0)
+            for (int q = 0; q < min(kEThreads, u1 - b); ++q) w = fma(gm_s[q], gm_s[q], w);
+        __syncthreads();
+    }
+    if (tid == 0) a.inv_w[j] = w <= 1e-12 ? 0.0 : 0.5 / w;
+}
+
+__global__ __launch_bounds__(kEThreads) void residual_kernel(FitArgs a) {
+    const int slots = a.S * a.k;
+    const uint16_t* cd = a.codes + (size_t)blockIdx.x * slots;
+    const float* x = a.tiles + (size_t)blockIdx.x * a.C;
+    float* out = a.res + (size_t)blockIdx.x * a.C;
+    for (int c0 = threadIdx.x; c0 < a.C; c0 += 4 * kEThreads) {
+        int c[4];
+        float rec[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            c[e] = min(c0 + e * kEThreads, a.C - 1);
+            rec[e] = 0.f;
+        }
+        int sl = 0;
+        for (int l = 0; l < a.S; ++l) {
+            const float g = a.gamma[l];
+#pragma unroll 8
+            for (int q = 0; q < a.k; ++q, ++sl) {
+                const uint16_t v = cd[sl];
+                const float scale = g * ((v & 0x8000) ? -1.0f : 1.0f);
+                const float* d = a.D + (size_t)(v & 0x7FFF) * a.C;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rec[e] = fmaf(scale, d[c[e]], rec[e]);
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (c0 + e * kEThreads < a.C) out[c0 + e * kEThreads] = x[c[e]] - rec[e];
     }
 }
 
 constexpr uint8_t kAtomKept = 0, kAtomNonFinite = 1, kAtomDead = 2;
 
-__global__ __launch_bounds__(kEThreads) void atom_update_kernel(
-    const float* __restrict__ res, int C, float* __restrict__ D, const int* __restrict__ off,
-    const uint32_t* __restrict__ utile, const double* __restrict__ ucoef,
-    const double* __restrict__ inv_w, double cap, double target, uint8_t* __restrict__ flag) {
+__global__ __launch_bounds__(kEThreads) void atom_sum_kernel(FitArgs a) {
+    constexpr int kU = 8;  // users' rows in flight
+    const int j = blockIdx.x, c = blockIdx.y * kEThreads + threadIdx.x;
+    const int u0 = a.off[j], u1 = a.off[j + 1];
+    const double iw = a.inv_w[j];
+    if (u0 == u1 || iw == 0.0 || c >= a.C) return;
+    double corr = 0.0;
+    int u = u0;
+    for (; u + kU <= u1; u += kU) {
+        float v[kU];
+#pragma unroll
+        for (int q = 0; q < kU; ++q) v[q] = a.res[(size_t)a.utile[u + q] * a.C + c];
+#pragma unroll
+        for (int q = 0; q < kU; ++q) corr = fma(a.ucoef[u + q], (double)v[q], corr);
+    }
+    for (; u < u1; ++u) corr = fma(a.ucoef[u], (double)a.res[(size_t)a.utile[u] * a.C + c], corr);
+    // the new value through double; one that float cannot hold comes out infinite
+    a.nv[(size_t)j * a.C + c] = (float)fma(corr, iw, (double)a.D[(size_t)j * a.C + c]);
+}
+
+__global__ __launch_bounds__(kEThreads) void atom_finish_kernel(FitArgs a) {
     extern __shared__ float nv[];  // C: the atom's new values
     __shared__ double nsq_s;
-    const int j = blockIdx.x, tid = threadIdx.x;
-    const int u0 = off[j], u1 = off[j + 1];
-    if (u0 == u1) {
-        if (tid == 0) flag[j] = kAtomDead;
+    const int j = blockIdx.x, tid = threadIdx.x, C = a.C;
+    const bool dead = a.off[j] == a.off[j + 1];
+    if (dead || a.inv_w[j] == 0.0) {  // no users, or sum of gamma^2 <= 1e-12: the atom stays
+        if (tid == 0) a.flag[j] = dead ? kAtomDead : kAtomKept;
         return;
     }
-    const double iw = inv_w[j];
-    if (iw == 0.0) {  // sum of gamma^2 <= 1e-12: the atom stays
-        if (tid == 0) flag[j] = kAtomKept;
-        return;
-    }
-    float* atom = D + (size_t)j * C;
+    float* atom = a.D + (size_t)j * C;
     int bad = 0;
     for (int c = tid; c < C; c += kEThreads) {
-        double corr = 0.0;
-        for (int u = u0; u < u1; ++u)
-            corr = fma(ucoef[u], (double)res[(size_t)utile[u] * C + c], corr);
-        const double v = fma(corr, iw, (double)atom[c]);
-        const float vf = (float)v;
-        if (!isfinite(v) || !isfinite(vf)) bad = 1;
+        const float vf = a.nv[(size_t)j * C + c];
+        if (!isfinite(vf)) bad = 1;
         nv[c] = vf;
     }
     if (__syncthreads_or(bad)) {
-        if (tid == 0) flag[j] = kAtomNonFinite;
+        if (tid == 0) a.flag[j] = kAtomNonFinite;
         return;
     }
     if (tid == 0) {
         double sq = 0.0;
+#pragma unroll 8
         for (int c = 0; c < C; ++c) sq = fma((double)nv[c], (double)nv[c], sq);
         nsq_s = sq;
-        flag[j] = isfinite(sq) ? kAtomKept : kAtomNonFinite;
+        a.flag[j] = isfinite(sq) ? kAtomKept : kAtomNonFinite;
     }
     __syncthreads();
     const double nsq = nsq_s;
     if (!isfinite(nsq)) return;
     const double nn = sqrt(nsq);
-    if (nn > cap) {
-        const double sc = target / nn;
+    if (nn > a.cap) {
+        const double sc = a.target / nn;
         for (int c = tid; c < C; c += kEThreads) atom[c] = (float)((double)nv[c] * sc);
     } else {
         for (int c = tid; c < C; c += kEThreads) atom[c] = nv[c];
@@ -891,96 +1029,76 @@ struct DevBuf {
     uint16_t* u16() const { return static_cast<uint16_t*>(p); }
 };
 
-// One atomUpdateStep per pass (HierarchicalSDRStrategy.cpp:281-490): the users of every atom
-// gathered on the host from the current codes in (tile, slot) order (:325-339) with their
-// sign * gamma and the sum of gamma^2 (fused, :428-437), the residuals and the updates on the
-// device, the re-seeds on the host from the fit's generator (base seed :403).
+// One atomUpdateStep per pass (HierarchicalSDRStrategy.cpp:281-490): users, residuals and
+// updates on the device, the re-seeds on the host from the fit's generator (base seed :403).
 struct Refine {
-    DevBuf res, off, utile, ucoef, invw, flag;
-    double target = 0.0, cap = 0.0;
+    DevBuf res, nv, off, utile, ucoef, invw, flag;
+    FitArgs fa{};
 
-    int init(const Geometry& g, const std::vector<float>& tiles, hipStream_t) {
+    int init(const Geometry& g, const std::vector<float>& tiles, const std::vector<float>& gamma,
+             const float* d_tiles, float* d_D, const uint16_t* d_codes) {
         const size_t slots = (size_t)g.S * g.k, ncodes = (size_t)g.n_tiles * slots;
-        target = std::max(1e-6, csdr::hsdr_mean_tile_norm(tiles.data(), g.n_tiles, g.tile_dim) /
-                                    std::sqrt((double)slots));  // :390-392
-        cap = 1.5 * target;
+        const size_t kc = (size_t)g.K * g.tile_dim;
         CSDR_HIP_CHECK(hipMalloc(&res.p, tiles.size() * 4));
+        CSDR_HIP_CHECK(hipMalloc(&nv.p, kc * 4));
         CSDR_HIP_CHECK(hipMalloc(&off.p, ((size_t)g.K + 1) * 4));
         CSDR_HIP_CHECK(hipMalloc(&utile.p, std::max<size_t>(ncodes, 1) * 4));
         CSDR_HIP_CHECK(hipMalloc(&ucoef.p, std::max<size_t>(ncodes, 1) * 8));
         CSDR_HIP_CHECK(hipMalloc(&invw.p, (size_t)g.K * 8));
         CSDR_HIP_CHECK(hipMalloc(&flag.p, (size_t)g.K));
-        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&atom_update_kernel),
+        fa.tiles = d_tiles;
+        fa.codes = d_codes;
+        fa.D = d_D;
+        fa.nv = nv.f();
+        fa.res = res.f();
+        fa.off = static_cast<int*>(off.p);
+        fa.utile = static_cast<uint32_t*>(utile.p);
+        fa.ucoef = static_cast<double*>(ucoef.p);
+        fa.inv_w = static_cast<double*>(invw.p);
+        fa.flag = static_cast<uint8_t*>(flag.p);
+        fa.n = g.n_tiles;
+        fa.ncodes = (long long)ncodes;
+        fa.C = (int)g.tile_dim;
+        fa.K = g.K;
+        fa.S = g.S;
+        fa.k = g.k;
+        fa.target = std::max(1e-6, csdr::hsdr_mean_tile_norm(tiles.data(), g.n_tiles, g.tile_dim) /
+                                       std::sqrt((double)slots));  // :390-392
+        fa.cap = 1.5 * fa.target;
+        for (uint32_t l = 0; l < g.S; ++l) fa.gamma[l] = gamma[l];
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&atom_finish_kernel),
                                   hipFuncAttributeMaxDynamicSharedMemorySize,
                                   (int)(g.tile_dim * 4));
+        (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&users_count_kernel),
+                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)g.K * 4);
         return CSDR_OK;
     }
 
-    int pass(const Geometry& g, const std::vector<float>& tiles, const std::vector<float>& gamma,
-             const float* d_tiles, float* d_D, const uint16_t* d_codes, std::mt19937& rng,
-             hipStream_t st) {
-        const size_t slots = (size_t)g.S * g.k, ncodes = (size_t)g.n_tiles * slots;
-        const uint32_t C = g.tile_dim;
-        std::vector<uint16_t> codes(ncodes);
-        CSDR_HIP_CHECK(
-            hipMemcpyAsync(codes.data(), d_codes, ncodes * 2, hipMemcpyDeviceToHost, st));
-        CSDR_HIP_CHECK(hipStreamSynchronize(st));
-        std::vector<int> offs((size_t)g.K + 1, 0);
-        for (uint16_t v : codes) {
-            if ((v & 0x7FFF) >= g.K) return set_error(CSDR_E_INVALID, "hsdr_compress: bad code");
-            ++offs[(v & 0x7FFF) + 1];
-        }
-        for (uint32_t j = 0; j < g.K; ++j) offs[j + 1] += offs[j];
-        std::vector<int> pos(offs.begin(), offs.end() - 1);
-        std::vector<uint32_t> ut(ncodes);
-        std::vector<double> uc(ncodes), wsum(g.K, 0.0), iw(g.K, 0.0);
-        for (size_t i = 0; i < g.n_tiles; ++i)
-            for (size_t sl = 0; sl < slots; ++sl) {
-                const uint16_t v = codes[i * slots + sl];
-                const uint32_t j = v & 0x7FFF;
-                const double gm = (double)gamma[sl / g.k];
-                const int p = pos[j]++;
-                ut[p] = (uint32_t)i;
-                uc[p] = ((v & 0x8000) ? -1.0 : 1.0) * gm;
-                wsum[j] = std::fma(gm, gm, wsum[j]);
-            }
-        for (uint32_t j = 0; j < g.K; ++j) iw[j] = wsum[j] <= 1e-12 ? 0.0 : 0.5 / wsum[j];
-        CSDR_HIP_CHECK(
-            hipMemcpyAsync(off.p, offs.data(), offs.size() * 4, hipMemcpyHostToDevice, st));
-        CSDR_HIP_CHECK(hipMemcpyAsync(utile.p, ut.data(), ncodes * 4, hipMemcpyHostToDevice, st));
-        CSDR_HIP_CHECK(hipMemcpyAsync(ucoef.p, uc.data(), ncodes * 8, hipMemcpyHostToDevice, st));
-        CSDR_HIP_CHECK(hipMemcpyAsync(invw.p, iw.data(), iw.size() * 8, hipMemcpyHostToDevice, st));
+    int pass(const std::vector<float>& tiles, std::mt19937& rng, hipStream_t st) {
+        const uint32_t C = (uint32_t)fa.C, K = (uint32_t)fa.K;
         const uint64_t base_seed = static_cast<uint64_t>(rng()) ^ 0xA0B1C2D3u;
-
-        ResArgs ra{};
-        ra.tiles = d_tiles;
-        ra.D = d_D;
-        ra.codes = d_codes;
-        ra.res = res.f();
-        ra.n = g.n_tiles;
-        ra.C = (int)C;
-        ra.S = g.S;
-        ra.k = g.k;
-        for (uint32_t l = 0; l < g.S; ++l) ra.gamma[l] = gamma[l];
-        const long long total = (long long)g.n_tiles * C;
-        const int rgrid = (int)std::min<long long>((total + kEThreads - 1) / kEThreads, 16384);
-        residual_kernel<<<rgrid, kEThreads, 0, st>>>(ra);
+        users_zero_kernel<<<(K + kEThreads) / kEThreads, kEThreads, 0, st>>>(fa);
+        const unsigned cgrid =
+            (unsigned)std::min<long long>((fa.ncodes + 4 * kEThreads - 1) / (4 * kEThreads), 256);
+        users_count_kernel<<<cgrid, kEThreads, K * 4, st>>>(fa);
+        users_scan_kernel<<<1, kEThreads, 0, st>>>(fa);
+        users_fill_kernel<<<K, kEThreads, 0, st>>>(fa);
+        CSDR_LAUNCH_CHECK("hsdr_compress users");
+        residual_kernel<<<(unsigned)fa.n, kEThreads, 0, st>>>(fa);
         CSDR_LAUNCH_CHECK("hsdr_compress residual");
-        atom_update_kernel<<<g.K, kEThreads, (size_t)C * 4, st>>>(
-            res.f(), (int)C, d_D, static_cast<const int*>(off.p),
-            static_cast<const uint32_t*>(utile.p), static_cast<const double*>(ucoef.p),
-            static_cast<const double*>(invw.p), cap, target, static_cast<uint8_t*>(flag.p));
+        atom_sum_kernel<<<dim3(K, (C + kEThreads - 1) / kEThreads), kEThreads, 0, st>>>(fa);
+        atom_finish_kernel<<<K, kEThreads, (size_t)C * 4, st>>>(fa);
         CSDR_LAUNCH_CHECK("hsdr_compress atom update");
-        std::vector<uint8_t> fl(g.K);
-        CSDR_HIP_CHECK(hipMemcpyAsync(fl.data(), flag.p, g.K, hipMemcpyDeviceToHost, st));
+        std::vector<uint8_t> fl(K);
+        CSDR_HIP_CHECK(hipMemcpyAsync(fl.data(), flag.p, K, hipMemcpyDeviceToHost, st));
         CSDR_HIP_CHECK(hipStreamSynchronize(st));
         std::vector<float> atom(C);
-        for (uint32_t j = 0; j < g.K; ++j) {
+        for (uint32_t j = 0; j < K; ++j) {
             if (fl[j] == kAtomKept) continue;
-            csdr::hsdr_reseed_atom(tiles.data(), g.n_tiles, C, base_seed, j,
-                                   fl[j] == kAtomDead ? 0x9E3779B1u : 0xB7E15163u, target,
+            csdr::hsdr_reseed_atom(tiles.data(), (uint32_t)fa.n, C, base_seed, j,
+                                   fl[j] == kAtomDead ? 0x9E3779B1u : 0xB7E15163u, fa.target,
                                    atom.data());
-            CSDR_HIP_CHECK(hipMemcpy(d_D + (size_t)j * C, atom.data(), (size_t)C * 4,
+            CSDR_HIP_CHECK(hipMemcpy(fa.D + (size_t)j * C, atom.data(), (size_t)C * 4,
                                      hipMemcpyHostToDevice));
         }
         return CSDR_OK;
@@ -1031,10 +1149,10 @@ int fit_tiles(const std::vector<float>& tiles, uint32_t n_tiles, uint32_t tile_d
     if (rc != CSDR_OK) return rc;
     if (ksvd_iters) {
         Refine rf;
-        rc = rf.init(g, tiles, st);
+        rc = rf.init(g, tiles, gamma, d_tiles.f(), d_D.f(), d_codes.u16());
         if (rc != CSDR_OK) return rc;
         for (int it = 0; it < ksvd_iters; ++it) {  // atom update, then encode again (:570-573)
-            rc = rf.pass(g, tiles, gamma, d_tiles.f(), d_D.f(), d_codes.u16(), rng, st);
+            rc = rf.pass(tiles, rng, st);
             if (rc != CSDR_OK) return rc;
             rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
                            d_codes.u16(), d_gram.p, st);
