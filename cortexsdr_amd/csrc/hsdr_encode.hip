@@ -38,11 +38,10 @@
 #include "common.hpp"
 
 namespace csdr {
-// fitHierarchicalKSVD's dictionary initialisation, in the reference build's arithmetic, the
-// mean tile norm and atomUpdateStep's re-seed of an atom (hsdr_init.cpp).
-void hsdr_init_dictionary(const float* tiles, uint32_t n, uint32_t C, uint16_t K, uint32_t slots,
-                          float* D, std::mt19937* rng);
-double hsdr_mean_tile_norm(const float* tiles, uint32_t n, uint32_t C);
+// fitHierarchicalKSVD's dictionary initialisation, in the reference build's arithmetic (returns
+// the mean tile norm), and atomUpdateStep's re-seed of an atom (hsdr_init.cpp).
+double hsdr_init_dictionary(const float* tiles, uint32_t n, uint32_t C, uint16_t K,
+                            uint32_t slots, float* D, std::mt19937* rng);
 void hsdr_reseed_atom(const float* tiles, uint32_t n, uint32_t C, uint64_t base_seed, uint32_t j,
                       uint32_t mul, double target_norm, float* atom);
 }  // namespace csdr
@@ -758,7 +757,7 @@ int launch_mp(const float* tiles, long long n, int C, const float* D, int K, int
 //  residual_kernel: residual = tile - sum over slots of gamma_l * sign * D[idx], slots in
 //    order, each term fused (the reference's r[c] += scale * atom[c], :300-311), then tile -
 //    recon (:316-320). A workgroup per tile: its codes are uniform (scalar loads) and a thread
-//    keeps 4 elements, with the next slots' atom rows in flight (84 -> RES_US us at 4864 x 896,
+//    keeps 4 elements, with the next slots' atom rows in flight (84 -> 24 us at 4864 x 896,
 //    24 slots: a thread per element with a 64-bit division each);
 //  atom_sum_kernel: correction[c] = sum over the atom's users, in order, of sign * gamma *
 //    residual (double, fused: :428-437), the new value atom + correction * (0.5 / sum gamma^2)
@@ -768,7 +767,7 @@ int launch_mp(const float* tiles, long long n, int C, const float* D, int K, int
 //  atom_finish_kernel: per atom, a non-finite value flags it for the host's re-seed (:461), the
 //    squared norm is summed in element order as the reference's loop does (:456), and atoms
 //    longer than the cap are scaled back to the target norm (:482-487). Atoms without users
-//    are re-seeded by the host (:411-425). Sum and finish: 273 -> UPD_US us at K = 512.
+//    are re-seeded by the host (:411-425). Sum and finish: 273 -> 34 + 15 us at K = 512.
 struct FitArgs {
     const float* tiles;
     const uint16_t* codes;
@@ -1035,11 +1034,11 @@ struct Refine {
     DevBuf res, nv, off, utile, ucoef, invw, flag;
     FitArgs fa{};
 
-    int init(const Geometry& g, const std::vector<float>& tiles, const std::vector<float>& gamma,
+    int init(const Geometry& g, double mean_norm, const std::vector<float>& gamma,
              const float* d_tiles, float* d_D, const uint16_t* d_codes) {
         const size_t slots = (size_t)g.S * g.k, ncodes = (size_t)g.n_tiles * slots;
         const size_t kc = (size_t)g.K * g.tile_dim;
-        CSDR_HIP_CHECK(hipMalloc(&res.p, tiles.size() * 4));
+        CSDR_HIP_CHECK(hipMalloc(&res.p, (size_t)g.n_tiles * g.tile_dim * 4));
         CSDR_HIP_CHECK(hipMalloc(&nv.p, kc * 4));
         CSDR_HIP_CHECK(hipMalloc(&off.p, ((size_t)g.K + 1) * 4));
         CSDR_HIP_CHECK(hipMalloc(&utile.p, std::max<size_t>(ncodes, 1) * 4));
@@ -1062,8 +1061,7 @@ struct Refine {
         fa.K = g.K;
         fa.S = g.S;
         fa.k = g.k;
-        fa.target = std::max(1e-6, csdr::hsdr_mean_tile_norm(tiles.data(), g.n_tiles, g.tile_dim) /
-                                       std::sqrt((double)slots));  // :390-392
+        fa.target = std::max(1e-6, mean_norm / std::sqrt((double)slots));  // :390-392
         fa.cap = 1.5 * fa.target;
         for (uint32_t l = 0; l < g.S; ++l) fa.gamma[l] = gamma[l];
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&atom_finish_kernel),
@@ -1074,7 +1072,7 @@ struct Refine {
         return CSDR_OK;
     }
 
-    int pass(const std::vector<float>& tiles, std::mt19937& rng, hipStream_t st) {
+    int pass(const float* tiles, std::mt19937& rng, hipStream_t st) {
         const uint32_t C = (uint32_t)fa.C, K = (uint32_t)fa.K;
         const uint64_t base_seed = static_cast<uint64_t>(rng()) ^ 0xA0B1C2D3u;
         users_zero_kernel<<<(K + kEThreads) / kEThreads, kEThreads, 0, st>>>(fa);
@@ -1095,7 +1093,7 @@ struct Refine {
         std::vector<float> atom(C);
         for (uint32_t j = 0; j < K; ++j) {
             if (fl[j] == kAtomKept) continue;
-            csdr::hsdr_reseed_atom(tiles.data(), (uint32_t)fa.n, C, base_seed, j,
+            csdr::hsdr_reseed_atom(tiles, (uint32_t)fa.n, C, base_seed, j,
                                    fl[j] == kAtomDead ? 0x9E3779B1u : 0xB7E15163u, fa.target,
                                    atom.data());
             CSDR_HIP_CHECK(hipMemcpy(fa.D + (size_t)j * C, atom.data(), (size_t)C * 4,
@@ -1116,7 +1114,7 @@ void put(std::vector<uint8_t>& out, const T& v) {
 // matching pursuit on the GPU, then ksvd_iters atom-update passes each followed by matching
 // pursuit again (:570-573); D (K x tile_dim, non-finite values zeroed as :592-601) and, when
 // codes is not null, the final codes.
-int fit_tiles(const std::vector<float>& tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t K,
+int fit_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t K,
               uint8_t S, uint8_t k, uint8_t ksvd_iters, const std::vector<float>& gamma,
               std::vector<float>& D, std::vector<uint16_t>* codes_out, hipStream_t st) {
     Geometry g{};
@@ -1132,16 +1130,16 @@ int fit_tiles(const std::vector<float>& tiles, uint32_t n_tiles, uint32_t tile_d
     if (rc != CSDR_OK) return rc;
     D.assign((size_t)K * tile_dim, 0.0f);
     std::mt19937 rng(0xC0DE);  // the fit's generator (:513), through init and every pass
-    csdr::hsdr_init_dictionary(tiles.data(), n_tiles, tile_dim, K, (uint32_t)S * k, D.data(),
-                               &rng);
+    const double mean_norm = csdr::hsdr_init_dictionary(tiles, n_tiles, tile_dim, K,
+                                                        (uint32_t)S * k, D.data(), &rng);
     const size_t ncodes = (size_t)n_tiles * S * k;
     DevBuf d_tiles, d_D, d_codes, d_gram;
     if (gram_pays(n_tiles, (int)tile_dim, K, S, k))
         CSDR_HIP_CHECK(hipMalloc(&d_gram.p, gram_ws_bytes(n_tiles, K)));
-    CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, std::max<size_t>(tiles.size(), 1) * 4));
+    CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, (size_t)n_tiles * tile_dim * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_D.p, D.size() * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
-    CSDR_HIP_CHECK(hipMemcpyAsync(d_tiles.p, tiles.data(), tiles.size() * 4,
+    CSDR_HIP_CHECK(hipMemcpyAsync(d_tiles.p, tiles, (size_t)n_tiles * tile_dim * 4,
                                   hipMemcpyHostToDevice, st));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_D.p, D.data(), D.size() * 4, hipMemcpyHostToDevice, st));
     rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
@@ -1149,7 +1147,7 @@ int fit_tiles(const std::vector<float>& tiles, uint32_t n_tiles, uint32_t tile_d
     if (rc != CSDR_OK) return rc;
     if (ksvd_iters) {
         Refine rf;
-        rc = rf.init(g, tiles, gamma, d_tiles.f(), d_D.f(), d_codes.u16());
+        rc = rf.init(g, mean_norm, gamma, d_tiles.f(), d_D.f(), d_codes.u16());
         if (rc != CSDR_OK) return rc;
         for (int it = 0; it < ksvd_iters; ++it) {  // atom update, then encode again (:570-573)
             rc = rf.pass(tiles, rng, st);
@@ -1298,9 +1296,11 @@ CSDR_API int csdr_hsdr_compress(const float* w, uint32_t rows, uint32_t cols, ui
         return set_error(CSDR_E_UNSUPPORTED,
                          "hsdr_compress: K-SVD refinement takes tiles of at most 32768 values");
     hipStream_t st = static_cast<hipStream_t>(hip_stream);
-    // tiles in row-major tile order (extractTiles :94-116) of the aligned block
-    std::vector<float> tiles = extract_tiles(w, g.R_full, g.C, g.tr, g.tc);
-    tiles.resize((size_t)g.n_tiles * g.tile_dim);
+    // tiles in row-major tile order (extractTiles :94-116) of the aligned block; whole-row
+    // tiles lie in that order already
+    std::vector<float> copied;
+    if (!(g.tr == 1 && g.tc == g.C)) copied = extract_tiles(w, g.R_full, g.C, g.tr, g.tc);
+    const float* tiles = copied.empty() ? w : copied.data();
     std::vector<float> gamma(g.S), D;
     for (uint32_t l = 0; l < g.S; ++l) gamma[l] = std::pow(stage_decay, (float)l);
     std::vector<uint16_t> codes;
@@ -1308,9 +1308,12 @@ CSDR_API int csdr_hsdr_compress(const float* w, uint32_t rows, uint32_t cols, ui
     if (rc != CSDR_OK) return rc;
 
     // serialisation (:1197-1237): header, stage scales, D, packed codes, edge strips
-    std::vector<uint8_t> s;
-    s.reserve(stream_bytes(g));
-    s.insert(s.end(), {'H', 'S', 'D', 'R'});
+    uint8_t* o = out;
+    const auto bytes = [&](const void* p, size_t n) {
+        if (n) std::memcpy(o, p, n);
+        o += n;
+    };
+    std::vector<uint8_t> s{'H', 'S', 'D', 'R'};
     put<uint32_t>(s, 2);
     put<uint32_t>(s, g.R);
     put<uint32_t>(s, g.C);
@@ -1322,14 +1325,13 @@ CSDR_API int csdr_hsdr_compress(const float* w, uint32_t rows, uint32_t cols, ui
     put<uint8_t>(s, g.k);
     put<float>(s, stage_decay);
     put<uint32_t>(s, g.edge_floats * 4);
-    for (float x : gamma) put<float>(s, x);
-    for (float x : D) put<float>(s, x);
-    for (uint16_t c : codes) put<uint16_t>(s, c);
+    bytes(s.data(), s.size());
+    bytes(gamma.data(), gamma.size() * 4);
+    bytes(D.data(), D.size() * 4);
+    bytes(codes.data(), codes.size() * 2);
     for (uint32_t r = 0; r < g.R_full; ++r)
-        for (uint32_t c = g.C_full; c < g.C; ++c) put<float>(s, w[(size_t)r * g.C + c]);
-    for (uint32_t r = g.R_full; r < g.R; ++r)
-        for (uint32_t c = 0; c < g.C; ++c) put<float>(s, w[(size_t)r * g.C + c]);
-    std::memcpy(out, s.data(), s.size());
+        bytes(w + (size_t)r * g.C + g.C_full, (size_t)(g.C - g.C_full) * 4);
+    bytes(w + (size_t)g.R_full * g.C, (size_t)(g.R - g.R_full) * g.C * 4);
     return CSDR_OK;
 }
 
@@ -1448,7 +1450,7 @@ CSDR_API int csdr_hsda_build(int n, const char* const* names, const float* const
             }
             Dict d;
             d.key = key;
-            int rc = fit_tiles(pool, fill, tile_dim, key.n_atoms, key.n_stages, key.k, ksvd_iters,
+            int rc = fit_tiles(pool.data(), fill, tile_dim, key.n_atoms, key.n_stages, key.k, ksvd_iters,
                                gamma, d.atoms, nullptr, st);
             if (rc != CSDR_OK) return rc;
             const size_t di = dicts.size();
