@@ -31,12 +31,14 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cmath>
+#include <initializer_list>
 #include <new>
 #include <string>
 #include <vector>
 
 #include "common.hpp"
 #include "hsdb_impl.hpp"
+#include "split_gemm.hpp"
 
 namespace {
 
@@ -168,6 +170,7 @@ struct csdr_decoder {
     int pf_rows = 0;
     float *pf_x = nullptr, *pf_h = nullptr, *pf_q = nullptr, *pf_k = nullptr, *pf_v = nullptr;
     float *pf_a = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_w = nullptr;
+    float* pf_s = nullptr;          // the split form's token planes, row scales and partial sums
     int* pf_tok = nullptr;
     // on-demand layer streaming (blocks of host-resident segments)
     bool prefetch = true;           // copy block j + 2 while block j + 1 runs (else j + 1 after j)
@@ -405,13 +408,39 @@ __global__ void pass_tokens_kernel(const int* __restrict__ ring, int cap, int B,
 
 void free_prefill(csdr_decoder* d) {
     for (float* p : {d->pf_x, d->pf_h, d->pf_q, d->pf_k, d->pf_v, d->pf_a, d->pf_g, d->pf_u,
-                     d->pf_w})
+                     d->pf_w, d->pf_s})
         if (p) (void)hipFree(p);
     if (d->pf_tok) (void)hipFree(d->pf_tok);
     d->pf_x = d->pf_h = d->pf_q = d->pf_k = d->pf_v = d->pf_a = d->pf_g = d->pf_u = d->pf_w =
-        nullptr;
+        d->pf_s = nullptr;
     d->pf_tok = nullptr;
     d->pf_rows = 0;
+}
+
+constexpr int kMinSplitRows = 8;  // fewer: a row of W per wave (csdr_dense_linear_ex)
+
+// The prefill's split form (split_gemm.hpp) needs every block's matrices in its layout.
+bool prefill_split(const csdr_decoder* d) {
+    for (const Layer& L : d->layers)
+        for (const csdr_hsdb* w : {L.q, L.k, L.v, L.o, L.gate, L.up, L.down})
+            if (!csdr::split_eligible(w)) return false;
+    return true;
+}
+
+// Floats of the split form's buffers: planes of the largest weight group with a scale per row,
+// and for `rows` token rows planes of the widest input, a scale each and the partial sums.
+size_t split_w_floats(const csdr_decoder_config& c) {
+    const size_t H = c.hidden, F = c.ffn, kvw = (size_t)c.n_kv_heads * c.head_dim;
+    const size_t hl = csdr::split_ld(c.hidden), fl = csdr::split_ld(c.ffn);
+    return std::max({(H + 2 * kvw) * (hl + 1), 2 * F * (hl + 1), H * (fl + 1)}) + 16;
+}
+size_t split_part_rows(const csdr_decoder_config& c, int rows) {
+    return (size_t)rows * std::max(csdr::split_count(c.hidden, c.hidden, rows),
+                                   csdr::split_count(c.hidden, c.ffn, rows));
+}
+size_t split_x_floats(const csdr_decoder_config& c, int rows) {
+    const size_t widest = std::max(csdr::split_ld(c.hidden), csdr::split_ld(c.ffn));
+    return (size_t)rows * (widest + 1) + 16 + split_part_rows(c, rows) * c.hidden;
 }
 
 // Buffers of a prefill pass over `rows` token rows (kept for later passes of up to as many).
@@ -421,11 +450,14 @@ int ensure_prefill(csdr_decoder* d, int rows) {
     const csdr_decoder_config& c = d->cfg;
     const size_t n = (size_t)rows, H = c.hidden, F = c.ffn;
     const size_t kvw = (size_t)c.n_kv_heads * c.head_dim;
-    const size_t wmax = std::max({H * H, kvw * H, F * H});
+    const bool split = prefill_split(d);
+    const size_t wmax =
+        std::max({H * H, kvw * H, F * H, split ? split_w_floats(c) : (size_t)0});
     const std::pair<float**, size_t> bufs[] = {
         {&d->pf_x, n * H},   {&d->pf_h, n * H},   {&d->pf_q, n * H},
         {&d->pf_k, n * kvw}, {&d->pf_v, n * kvw}, {&d->pf_a, n * std::max(H, F)},
-        {&d->pf_g, n * F},   {&d->pf_u, n * F},   {&d->pf_w, wmax}};
+        {&d->pf_g, n * F},   {&d->pf_u, n * F},   {&d->pf_w, wmax},
+        {&d->pf_s, split ? split_x_floats(c, rows) : 4}};
     for (const auto& b : bufs) {
         void* p = nullptr;
         if (hipMalloc(&p, b.second * 4) != hipSuccess) {
@@ -455,6 +487,87 @@ int pass_linear(csdr_decoder* d, const csdr_hsdb* w, const float* x, int M, floa
     return csdr_dense_linear_ex(d->pf_w, (int)info.rows, (int)info.cols, x, M, y, bias, flags, st);
 }
 
+// The split form of a pass: each group of weights that reads one input is decoded into fp16
+// planes and multiplied in one product (split_gemm.hip). The o and down products' parts are
+// added to x, in order, by the next norm.
+int prefill_layers_split(csdr_decoder* d, int p0, int T, hipStream_t st) {
+    const csdr_decoder_config& c = d->cfg;
+    const int B = d->B, M = B * T, H = c.hidden, F = c.ffn, kvw = c.n_kv_heads * c.head_dim;
+    const int widest = std::max(csdr::split_ld(H), csdr::split_ld(F));
+    // fp16 planes and row scales inside a float buffer (16-byte aligned: ld is a multiple of 64)
+    const auto planes = [](float*& p, size_t rows, int ld) {
+        csdr::SplitPlanes s;
+        s.hi = reinterpret_cast<_Float16*>(p);
+        s.lo = s.hi + rows * ld;
+        p += rows * ld;
+        s.ld = ld;
+        return s;
+    };
+    float* sp = d->pf_s;
+    csdr::SplitPlanes x = planes(sp, M, widest);
+    x.inv = sp;
+    float* parts = sp + (M + 3) / 4 * 4;
+    const auto linear = [&](std::initializer_list<const csdr_hsdb*> ws,
+                            std::initializer_list<float*> ys, const float* const* bias,
+                            int splits) -> int {
+        const int n = (int)ws.size();
+        csdr::SplitPlanes wp[csdr::kSplitMats];
+        int R[csdr::kSplitMats];
+        float* p = d->pf_w;
+        for (int i = 0; i < n; ++i) {
+            R[i] = (int)ws.begin()[i]->R;
+            wp[i] = planes(p, R[i], x.ld);
+        }
+        for (int i = 0; i < n; ++i) {
+            wp[i].inv = p;
+            p += R[i];
+        }
+        RC(csdr::split_decode(n, ws.begin(), wp, st));
+        return csdr::split_gemm(n, wp, R, x, M, ys.begin(), bias, splits, st);
+    };
+    // parts of the o and down products (a pass of fewer rows than the buffers were sized for may
+    // want more parts than they hold)
+    const size_t room = split_part_rows(c, d->pf_rows) / M;
+    const int so = (int)std::min<size_t>(csdr::split_count(H, H, M), room);
+    const int sd = (int)std::min<size_t>(csdr::split_count(H, F, M), room);
+    int pending = 0;  // parts to be added to x
+    for (int l = 0; l < c.n_layers; ++l) {
+        const Layer& L = d->layers[l];
+        RC(layer_begin(d, l, st));
+        x.ld = csdr::split_ld(H);
+        x.lo = x.hi + (size_t)M * x.ld;
+        RC(csdr::split_rows(csdr::SplitOp::rms_norm, d->pf_x, L.attn_norm, parts, pending, M, H,
+                            c.rms_eps, x, st));
+        const float* bias[3] = {L.bq, L.bk, L.bv};
+        // the pass leaves only K and V behind: the last block ends with them
+        const bool last = l + 1 == c.n_layers;
+        if (last)
+            RC(linear({L.k, L.v}, {d->pf_k, d->pf_v}, bias + 1, 1));
+        else
+            RC(linear({L.q, L.k, L.v}, {d->pf_q, d->pf_k, d->pf_v}, bias, 1));
+        RC(csdr_rope_kv_rows(d->pf_q, d->pf_k, d->pf_v, B, T, p0, c.n_heads, c.n_kv_heads,
+                             c.head_dim, c.rope_theta, L.kc, L.vc, c.kv_dtype, c.max_ctx, st));
+        if (!last) {
+            RC(csdr_attn_prefill(d->pf_q, L.kc, L.vc, c.kv_dtype, B, T, p0, c.max_ctx, c.n_heads,
+                                 c.n_kv_heads, c.head_dim, 0.0f, d->pf_a, st));
+            RC(csdr::split_rows(csdr::SplitOp::plain, d->pf_a, nullptr, nullptr, 0, M, H, 0.f, x,
+                                st));
+            RC(linear({L.o}, {parts}, nullptr, so));
+            RC(csdr::split_rows(csdr::SplitOp::rms_norm, d->pf_x, L.ffn_norm, parts, so, M, H,
+                                c.rms_eps, x, st));
+            RC(linear({L.gate, L.up}, {d->pf_g, d->pf_u}, nullptr, 1));
+            x.ld = csdr::split_ld(F);
+            x.lo = x.hi + (size_t)M * x.ld;
+            RC(csdr::split_rows(csdr::SplitOp::silu_mul, d->pf_g, d->pf_u, nullptr, 0, M, F, 0.f,
+                                x, st));
+            RC(linear({L.down}, {parts}, nullptr, sd));
+            pending = sd;
+        }
+        RC(layer_end(d, l, st));
+    }
+    return CSDR_OK;
+}
+
 // The decoder body (no head) over positions [p0, p0 + T) of every sequence as one pass of
 // M = B x T token rows: K/V of those positions land in the caches as the decode step would
 // write them.
@@ -466,6 +579,10 @@ int prefill_pass(csdr_decoder* d, int p0, int T, hipStream_t st) {
     CSDR_LAUNCH_CHECK("decoder pass tokens");
     RC(csdr_hsdb_decode_rows(d->emb, d->pf_tok, M, d->pf_x, st));
     RC(stream_begin(d, st));
+    if (M >= kMinSplitRows && prefill_split(d)) {
+        RC(prefill_layers_split(d, p0, T, st));
+        return stream_end(d, st);
+    }
     for (int l = 0; l < c.n_layers; ++l) {
         const Layer& L = d->layers[l];
         RC(layer_begin(d, l, st));

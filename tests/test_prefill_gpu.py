@@ -203,6 +203,32 @@ def test_decoder_prefill_passes_match_token_at_a_time(gpu, B):
             assert rel_l2(np.atleast_2d(sc[i])[b], ref[i]) < 1e-3, (b, i)
 
 
+# The split-plane product of the passes at its edges: 8 token rows (its smallest), rows off the
+# tiles, edge strips in the contraction (ffn % 64 != 0), 4, 6, 8 and 16 slots, one to five
+# tiles per thread of the decode, parts of the contraction, one block only (no product but k
+# and v). Against the token-at-a-time prefill, which sums in fp32 too: two forms of a few
+# blocks' fp32 sums differ by some 1e-6 a product, so 1e-4 as above.
+@pytest.mark.parametrize("layers,heads,ffn,nnz,n_prompt", [
+    (2, 3, 200, 4, 9), (2, 2, 1100, 6, 71), (2, 1, 2200, 8, 140), (1, 2, 64, 8, 33),
+    (3, 14, 136, 16, 66),
+])
+def test_prefill_product_edges(gpu, layers, heads, ffn, nnz, n_prompt):
+    from cortexsdr_amd.decoder import Decoder, DecoderSpec, synthetic_weights
+
+    spec = DecoderSpec(layers, 64 * heads, heads, 1, 64, ffn, 333, n_prompt + 8)
+    w = synthetic_weights(spec, n_atoms=96, nnz=nnz, seed=ffn, sigma=0.1, norm_jitter=0.1,
+                          bias_sigma=0.1)
+    prompt = ((np.arange(n_prompt) * 7919 + 11) % spec.vocab).astype(np.int32)
+    runs = []
+    for chunk in (0, 512, max(8, n_prompt // 2 - 1)):
+        dec = Decoder(w, prefill_chunk=chunk)
+        try:
+            runs.append(_run(dec, prompt, 3))
+        finally:
+            dec.close()
+    _compare(runs, 3, 1e-4)
+
+
 def test_cfg4_full_model_long_prompt(gpu):
     """configs[3] at full size with a 160-token prompt: one multi-token pass (and passes of 64)
     against the token-at-a-time prefill."""
