@@ -45,6 +45,7 @@ using csdr::set_error;
 
 constexpr int kThreads = 256;
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Word 3 of a raw (stride 0) buffer resource on CDNA: 32-bit data format, no swizzle; with it a
 // lane whose offset is at or past num_records reads zeros and makes no memory access.
 constexpr int kRawBufferDword3 = 0x00020000;
@@ -85,18 +86,20 @@ struct MatDesc {
     int R, K, NB, NBc, nchunks, slots, blen, Ce, C_full;
     int PB;                   // dx: block columns per workgroup (block length 64)
     int dx_base, dx_count;    // dx workgroup ids [base, base + count)
+    int dg_base, dg_count;    // the same in dxg_kernel's launch (blocks other than 64 long)
     int g_base, g_count;      // gather workgroup ids, base a multiple of 8
     int splits;               // gather workgroups per chunk
     int rows_per_wg;          // rows of a chunk handled by one gather workgroup
     int rsplit[4], rrpw[4];   // M == 1 gather: ranges and rows per range of the remainder chunks
-    int Rt;                   // M > 1 gather: rows per workgroup
+    int Rt;                   // generic gather: rows per workgroup
     float sgam[kMaxSlotsArg]; // gamma of each slot (slots <= kMaxSlotsArg; scalar loads)
     int gunif;                // every slot has gamma sgam[0]
 };
 
 struct Params {
     MatDesc m[kMaxGroup];
-    int G, M, MVz, x_f16;
+    int G, M, x_f16;
+    int z0;  // generic gather: the launch's first group of MC columns
     int tm;  // token-major X (M x C) and Y (M x R) instead of feature-major (C x M, R x M)
     int accumulate;  // 1: Y += W.X (+ bias); 0: Y = W.X (+ bias)
     // input transform applied while staging x (csdr_hsdb_matmul_group_xop)
@@ -509,6 +512,22 @@ __device__ void stage_x_m1(const Params& p, const MatDesc& d, int b0, int nb, fl
     __syncthreads();
 }
 
+// Y initialisation for the gathers' accumulation: 0 or bias, or left as it is (+ bias), by
+// workgroup u of the n that the matrix has in the dx launch (NT threads each).
+template <int NT>
+__device__ __forceinline__ void init_y(const Params& p, const MatDesc& d, int u, int n) {
+    const size_t ytot = (size_t)d.R * p.M;
+    const size_t yper = (ytot + n - 1) / n;
+    const size_t ye = min(ytot, (size_t)(u + 1) * yper);
+    // (kept with no bias: nothing to do, and no read of y to wait for)
+    if (!p.accumulate || d.bias) {
+        for (size_t i = (size_t)u * yper + threadIdx.x; i < ye; i += NT) {
+            const float bv = d.bias ? d.bias[p.tm ? i % d.R : i / p.M] : 0.0f;
+            d.y[i] = p.accumulate ? d.y[i] + bv : bv;
+        }
+    }
+}
+
 // XOP: p.xop at compile time (the M == 1 staging's registers depend on it)
 template <int XOP>
 __global__ __launch_bounds__(kThreads) void dx_kernel(Params p) {
@@ -520,20 +539,8 @@ __global__ __launch_bounds__(kThreads) void dx_kernel(Params p) {
     const int u = wg - d.dx_base;
     const int tid = threadIdx.x;
     const int M = p.M;
+    init_y<kThreads>(p, d, u, d.dx_count);
     {
-        // Y initialisation for the gathers' accumulation: 0 or bias, or left as it is (+ bias)
-        const size_t ytot = (size_t)d.R * M;
-        const size_t yper = (ytot + d.dx_count - 1) / d.dx_count;
-        const size_t ye = min(ytot, (size_t)(u + 1) * yper);
-        // (kept with no bias: nothing to do, and no read of y to wait for)
-        if (!p.accumulate || d.bias) {
-            for (size_t i = (size_t)u * yper + tid; i < ye; i += kThreads) {
-                const float bv = d.bias ? d.bias[p.tm ? i % d.R : i / M] : 0.0f;
-                d.y[i] = p.accumulate ? d.y[i] + bv : bv;
-            }
-        }
-    }
-    if (d.blen == 64) {
         // 16 lanes per atom: lane l holds D[a][4l .. 4l+3] (one coalesced 16-byte load; a
         // wave reads 4 whole rows). The x range of this workgroup is staged in LDS in one
         // coalesced pass; per (block, column) each lane does 4 FMAs against its 4 x values
@@ -593,75 +600,118 @@ __global__ __launch_bounds__(kThreads) void dx_kernel(Params p) {
                 if (live && l16 == 0) Pout[bb * pstride + m] = sum;
             }
         }
-    } else {
-        // any block length (the reference's own 1-row geometry has blocks of C features): one
-        // wave per (b, a, group of 8 columns), lane-strided dot. Rounds of kR features per
-        // lane with every load of a round issued before its first use, at clamped indices and
-        // with the element type's branch around the round (a load per feature under that
-        // branch ran one round trip per feature); lanes past the block keep their sums.
-        constexpr int kR = 8;
-        const int lane = tid & 63;
-        const int mg = (M + 7) / 8;
-        const long long item = (long long)u * (kThreads / 64) + (tid >> 6);
-        if (item < (long long)d.NB * d.K * mg) {
-            const int gi = (int)(item % mg);
-            const long long ba = item / mg;
-            const int b = (int)(ba / d.K), a = (int)(ba % d.K);
-            const int m0 = gi * 8, nm = min(8, M - m0);
-            float acc[8];
+    }
+}
+
+// ---- kernel 1, blocks other than 64 long (the reference's own 1-row geometry has blocks of C
+// features): P[b][a][m] for 16 atoms and 16 columns per workgroup on the fp32 matrix cores.
+// The contraction is cut into 64-feature pieces, one per wave at a time, so a block of 1024
+// features is one round trip of loads; the 16 waves' tiles meet in LDS. Lane group l / 16 takes
+// features 4 (l / 16) .. + 3 of each 16 (VEC: rows of whole 16-byte pieces), or feature l / 16 of
+// each 4, so a load instruction covers 64 (16) contiguous bytes of 16 atoms; a lane's 16
+// features in a row instead made it 64 lines, 10.7 us. Bound by the chain of load, 16 products
+// and the sum over waves. (4864 x 896, K = 512, M = 8:
+// 17.8 us as a wave per atom with 64 scalar loads of x per lane, 6.6 here.)
+// At M = 1 a wave per (block, atom) instead, lanes striding the block: 15 of the 16 columns would
+// be idle, and K waves in as many workgroups as CUs load the dictionary faster than K / 16
+// workgroups (a call on 896 x 896, K = 256: 6.7 us against 8.9; 8000 x 2047: 7.5 against 16.0).
+constexpr int kDgThreads = 1024;
+
+template <typename XT>
+__global__ __launch_bounds__(kThreads) void dxw_kernel(Params p) {
+    constexpr int kR = 8;  // features per lane and round, all loads issued at clamped indices
+    int g = 0;
+    while (g + 1 < p.G && (int)blockIdx.x >= p.m[g + 1].dg_base) ++g;
+    const MatDesc& d = p.m[g];
+    const int u = (int)blockIdx.x - d.dg_base;
+    const int lane = threadIdx.x & 63;
+    init_y<kThreads>(p, d, u, d.dg_count);
+    const long long item = (long long)u * (kThreads / 64) + (threadIdx.x >> 6);  // b * K + a
+    if (item >= (long long)d.NB * d.K) return;
+    const int b = (int)(item / d.K), a = (int)(item - (long long)b * d.K);
+    const float* drow = d.dict + (size_t)a * d.blen;
+    const XT* x = static_cast<const XT*>(d.x) + (size_t)b * d.blen;
+    float acc = 0.f;
+    for (int t0 = 0; t0 < d.blen; t0 += 64 * kR) {
+        float dv[kR], xv[kR];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
-            const float* drow = d.dict + (size_t)a * d.blen;
-            for (int t0 = 0; t0 < d.blen; t0 += 64 * kR) {
-                float dv[kR];
-                size_t xo[kR];
-#pragma unroll
-                for (int r = 0; r < kR; ++r) {
-                    const int t = min(t0 + r * 64 + lane, d.blen - 1);
-                    dv[r] = drow[t];
-                    xo[r] = xi(p, d, b * d.blen + t, m0);
-                }
-                if (nm == 1) {
-                    float xv[kR];
-                    if (p.x_f16) {
-#pragma unroll
-                        for (int r = 0; r < kR; ++r) xv[r] = xval<_Float16>(d.x, xo[r]);
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < kR; ++r) xv[r] = xval<float>(d.x, xo[r]);
-                    }
-#pragma unroll
-                    for (int r = 0; r < kR; ++r)
-                        if (t0 + r * 64 + lane < d.blen) acc[0] = fmaf(dv[r], xv[r], acc[0]);
-                } else {
-                    // the columns of feature t: xo + j (feature-major) or + j * C (token-major)
-                    const size_t cs = p.tm ? (size_t)(d.C_full + d.Ce) : 1;
-                    float xv[kR][8];
-                    if (p.x_f16) {
-#pragma unroll
-                        for (int r = 0; r < kR; ++r)
-#pragma unroll
-                            for (int j = 0; j < 8; ++j)
-                                xv[r][j] = xval<_Float16>(d.x, xo[r] + (size_t)min(j, nm - 1) * cs);
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < kR; ++r)
-#pragma unroll
-                            for (int j = 0; j < 8; ++j)
-                                xv[r][j] = xval<float>(d.x, xo[r] + (size_t)min(j, nm - 1) * cs);
-                    }
-#pragma unroll
-                    for (int r = 0; r < kR; ++r)
-                        if (t0 + r * 64 + lane < d.blen)
-#pragma unroll
-                            for (int j = 0; j < 8; ++j) acc[j] = fmaf(dv[r], xv[r][j], acc[j]);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = csdr::wave_sum(acc[j]);
-            if (lane == 0)
-                for (int j = 0; j < nm; ++j) d.P[((size_t)b * d.K + a) * M + m0 + j] = acc[j];
+        for (int r = 0; r < kR; ++r) {
+            const int t = min(t0 + r * 64 + lane, d.blen - 1);
+            dv[r] = drow[t];
+            xv[r] = csdr::to_f32(x[t]);
         }
+#pragma unroll
+        for (int r = 0; r < kR; ++r)
+            if (t0 + r * 64 + lane < d.blen) acc = fmaf(dv[r], xv[r], acc);
+    }
+    acc = csdr::wave_sum(acc);
+    if (lane == 0) d.P[item] = acc;
+}
+
+template <typename XT, bool VEC>
+__global__ __launch_bounds__(kDgThreads) void dxg_kernel(Params p) {
+    __shared__ float red[kDgThreads / 64][256];
+    int g = 0;
+    while (g + 1 < p.G && (int)blockIdx.x >= p.m[g + 1].dg_base) ++g;
+    const MatDesc& d = p.m[g];
+    const int u = (int)blockIdx.x - d.dg_base;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int li = lane & 15, lg = lane >> 4;
+    const int M = p.M;
+    init_y<kDgThreads>(p, d, u, d.dg_count);
+    const int na = (d.K + 15) / 16, nm = (M + 15) / 16;
+    const int at = u % na, mt = u / na % nm, b = u / na / nm;
+    const int a = min(at * 16 + li, d.K - 1), m = min(mt * 16 + li, M - 1);
+    const float* drow = d.dict + (size_t)a * d.blen;
+    const XT* x = static_cast<const XT*>(d.x);
+    const size_t xs = p.tm ? 1 : (size_t)M;  // from a feature to the next
+    const size_t x0 = p.tm ? (size_t)m * (d.C_full + d.Ce) + (size_t)b * d.blen
+                           : (size_t)b * d.blen * M + m;
+    f32x4 acc[4];  // independent chains of 4 products: less latency, less rounding
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int f0 = wave * 64; f0 < d.blen; f0 += kDgThreads) {
+        float dv[16], xv[16];
+        if constexpr (VEC) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const f32x4 v = *reinterpret_cast<const f32x4*>(
+                    drow + min(f0 + 16 * j + 4 * lg, d.blen - 4));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) dv[4 * j + e] = v[e];
+            }
+        }
+        const auto feature = [&](int s) {
+            return VEC ? f0 + 16 * (s >> 2) + 4 * lg + (s & 3) : f0 + 4 * s + lg;
+        };
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const int fc = min(feature(s), d.blen - 1);
+            if constexpr (!VEC) dv[s] = drow[fc];
+            xv[s] = csdr::to_f32(x[x0 + fc * xs]);
+        }
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const bool in = feature(s) < d.blen;
+            acc[s & 3] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? dv[s] : 0.f, in ? xv[s] : 0.f,
+                                                              acc[s & 3], 0, 0, 0);
+        }
+    }
+    const f32x4 sum4 = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) red[wave][(4 * lg + v) * 16 + li] = sum4[v];
+    __syncthreads();
+    if (tid < 256) {
+        float t[kDgThreads / 64];
+#pragma unroll
+        for (int w = 0; w < kDgThreads / 64; ++w) t[w] = red[w][tid];
+#pragma unroll
+        for (int h = kDgThreads / 128; h > 0; h >>= 1)
+#pragma unroll
+            for (int w = 0; w < h; ++w) t[w] += t[w + h];
+        const float sum = t[0];
+        const int ao = at * 16 + (tid >> 4), mo = mt * 16 + (tid & 15);
+        if (ao < d.K && mo < M) d.P[((size_t)b * d.K + ao) * M + mo] = sum;
     }
 }
 
@@ -678,8 +728,7 @@ __global__ __launch_bounds__(kThreads) void dx_kernel(Params p) {
 // combine is staged for the workgroup's blocks in LDS first (stage_x_m1).
 template <int XOP, int NT>
 __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+        typedef unsigned int u4 __attribute__((ext_vector_type(4)));
     constexpr int kAtoms = NT / 4;  // 16 per wave
     int g = 0;
     while (g + 1 < p.G && wg >= p.m[g + 1].dx_base) ++g;
@@ -704,9 +753,9 @@ __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
     const int a = min(ag * kAtoms + wave * 16 + li, d.K - 1);
     const int b = min(bg * 16 + li, d.NB - 1);
     const int f0 = b * 64 + lg * 16;  // this lane's 16 features
-    f4 dv[4];
+    f32x4 dv[4];
     {
-        const f4* src = reinterpret_cast<const f4*>(d.dict + (size_t)a * 64 + lg * 16);
+        const f32x4* src = reinterpret_cast<const f32x4*>(d.dict + (size_t)a * 64 + lg * 16);
 #pragma unroll
         for (int i = 0; i < 4; ++i) dv[i] = src[i];
     }
@@ -717,10 +766,10 @@ __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
         __shared__ __attribute__((aligned(16))) float xs_attn[16 * 64];
         const int b0 = bg * 16;
         stage_x_m1<NT, XOP>(p, d, b0, min(16, d.NB - b0), xs_attn, u == 0);  // (ends in a barrier)
-        const f4* src = reinterpret_cast<const f4*>(xs_attn + (b - b0) * 64 + lg * 16);
+        const f32x4* src = reinterpret_cast<const f32x4*>(xs_attn + (b - b0) * 64 + lg * 16);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const f4 v = src[i];
+            const f32x4 v = src[i];
             xv[4 * i] = v.x;
             xv[4 * i + 1] = v.y;
             xv[4 * i + 2] = v.z;
@@ -737,10 +786,10 @@ __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
             xv[9 + 2 * i] = csdr::h2f(h1[i] >> 16);
         }
     } else {
-        const f4* src = reinterpret_cast<const f4*>(static_cast<const float*>(d.x) + f0);
+        const f32x4* src = reinterpret_cast<const f32x4*>(static_cast<const float*>(d.x) + f0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const f4 v = src[i];
+            const f32x4 v = src[i];
             xv[4 * i] = v.x;
             xv[4 * i + 1] = v.y;
             xv[4 * i + 2] = v.z;
@@ -787,7 +836,7 @@ __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
             d.xe[t] = x;
         }
     }
-    f4 acc = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 16; ++s)
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(dv[s >> 2][s & 3], xv[s], acc, 0, 0, 0);
@@ -797,7 +846,7 @@ __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
         if (ao + 3 < d.K && (d.K & 3) == 0) {
             // streamed past this XCD's L2: the gather reads P from every XCD (headline step
             // 15.64 -> 15.42 us)
-            __builtin_nontemporal_store(acc, reinterpret_cast<f4*>(out));
+            __builtin_nontemporal_store(acc, reinterpret_cast<f32x4*>(out));
         } else {
 #pragma unroll
             for (int v = 0; v < 4; ++v)
@@ -848,8 +897,7 @@ constexpr int kXsStride = 68;
 
 template <int XOP, int MC>
 __global__ __launch_bounds__(kThreads) void dxmm_kernel(Params p) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    static_assert(MC == 2 || MC == 4 || MC == 8 || MC == 16, "MC");
+        static_assert(MC == 2 || MC == 4 || MC == 8 || MC == 16, "MC");
     static_assert(kThreads == 256, "one X element per thread and pass");
     constexpr int BPT = 16 / MC;  // block columns per N tile
     __shared__ __attribute__((aligned(16))) float xs[16 * kXsStride];
@@ -865,9 +913,9 @@ __global__ __launch_bounds__(kThreads) void dxmm_kernel(Params p) {
     const int ag = u % na, ng = u / na;
     const int a0 = ag * 64 + wave * 16;
     // dictionary operand first (the longest round trip), then the X tile
-    f4 dv[4];
+    f32x4 dv[4];
     {
-        const f4* src = reinterpret_cast<const f4*>(d.dict + (size_t)min(a0 + li, d.K - 1) * 64 +
+        const f32x4* src = reinterpret_cast<const f32x4*>(d.dict + (size_t)min(a0 + li, d.K - 1) * 64 +
                                                     lg * 16);
 #pragma unroll
         for (int i = 0; i < 4; ++i) dv[i] = src[i];
@@ -945,11 +993,11 @@ __global__ __launch_bounds__(kThreads) void dxmm_kernel(Params p) {
         }
     }
     __syncthreads();
-    f4 xb[4];
+    f32x4 xb[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-        xb[i] = *reinterpret_cast<const f4*>(xs + li * kXsStride + lg * 16 + 4 * i);
-    f4 acc = {0.f, 0.f, 0.f, 0.f};
+        xb[i] = *reinterpret_cast<const f32x4*>(xs + li * kXsStride + lg * 16 + 4 * i);
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < 16; ++s)
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(dv[s >> 2][s & 3], xb[s >> 2][s & 3], acc, 0, 0, 0);
@@ -978,24 +1026,6 @@ __global__ __launch_bounds__(kThreads) void dxmm_kernel(Params p) {
             if (a < d.K) __builtin_nontemporal_store(acc[v], out + (size_t)a * M);
         }
     }
-}
-
-// Finds this gather workgroup's matrix and (chunk, split); false for padding slots.
-// Workgroups of one chunk are numbered to share an XCD (dispatch is round-robin over the
-// 8 XCDs), so that chunk's P slice is fetched into one L2 only.
-__device__ __forceinline__ bool gather_slot(const Params& p, int& g, int& c, int& sidx) {
-    const int wg = blockIdx.x;
-    g = -1;
-    for (int i = 0; i < p.G; ++i)
-        if (wg >= p.m[i].g_base && wg < p.m[i].g_base + p.m[i].g_count) g = i;
-    if (g < 0) return false;
-    const MatDesc& d = p.m[g];
-    const int u = wg - d.g_base;
-    const int j = u >> 3;
-    const int cl = j / d.splits;
-    sidx = j - cl * d.splits;
-    c = cl * 8 + (u & 7);
-    return c < d.nchunks;
 }
 
 __device__ __forceinline__ float edge_term(const Params& p, const MatDesc& d, int r, int m) {
@@ -1119,10 +1149,10 @@ __device__ __forceinline__ void gatherw_body(const Params& p, int wg) {
     if constexpr (P4) {
         // nontemporal: the slice was just streamed out by the dx launch (headline step 15.35 ->
         // 14.72 us; a gather that re-reads a slice still in its L2 is slower this way)
-        typedef float f4v __attribute__((ext_vector_type(4)));
-        const f4v* sv = reinterpret_cast<const f4v*>(Pg);
+        typedef float f32x4v __attribute__((ext_vector_type(4)));
+        const f32x4v* sv = reinterpret_cast<const f32x4v*>(Pg);
         auto ld = [&](int i) {
-            const f4v v = __builtin_nontemporal_load(sv + i);
+            const f32x4v v = __builtin_nontemporal_load(sv + i);
             return make_float4(v.x, v.y, v.z, v.w);
         };
         pv0 = ld(min(tid, np4 - 1));
@@ -1245,8 +1275,7 @@ template <int SLOTS, int MC, int TD, int LPR, bool P16, typename TileFn>
 __device__ __forceinline__ void gatherv_stream(const MatDesc& d, const float* Ps, float* rowt,
                                                u32x4 (*buf)[SLOTS / 4], TileFn tile, int nk,
                                                int wfirst, int ntiles) {
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    typedef float f2 __attribute__((ext_vector_type(2)));
+        typedef float f2 __attribute__((ext_vector_type(2)));
     constexpr int PPB = SLOTS / 4;
     constexpr int G = MC / 4;
     constexpr int kStep = 64;
@@ -1290,7 +1319,7 @@ __device__ __forceinline__ void gatherv_stream(const MatDesc& d, const float* Ps
             } else {
 #pragma unroll
                 for (int h = 0; h < G; ++h) {
-                    const f4 v = *reinterpret_cast<const f4*>(Ps + (size_t)e * MC + 4 * h);
+                    const f32x4 v = *reinterpret_cast<const f32x4*>(Ps + (size_t)e * MC + 4 * h);
                     acc[4 * h] = fmaf(cf, v.x, acc[4 * h]);
                     acc[4 * h + 1] = fmaf(cf, v.y, acc[4 * h + 1]);
                     acc[4 * h + 2] = fmaf(cf, v.z, acc[4 * h + 2]);
@@ -1314,7 +1343,7 @@ __device__ __forceinline__ void gatherv_stream(const MatDesc& d, const float* Ps
             if constexpr (MC >= 4) {
 #pragma unroll
                 for (int m4 = 0; m4 < MC; m4 += 4)
-                    *reinterpret_cast<f4*>(rt + m4) = f4{acc[m4], acc[m4 + 1], acc[m4 + 2], acc[m4 + 3]};
+                    *reinterpret_cast<f32x4*>(rt + m4) = f32x4{acc[m4], acc[m4 + 1], acc[m4 + 2], acc[m4 + 3]};
             } else {
 #pragma unroll
                 for (int m = 0; m < MC; ++m) rt[m] = acc[m];
@@ -1408,20 +1437,19 @@ void gatherv_kernel(Params p) {
     // the P round trip and the barrier.
     constexpr int NBUF = TD + 1;
     u32x4 buf[NBUF][PPB];
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    if (P16 || (M == MC && (d.K * MC) % 4 == 0)) {
+        if (P16 || (M == MC && (d.K * MC) % 4 == 0)) {
         // P slice: global [block][atom][M] (fp16 P: [block][atom][8] halves) -> LDS, a
         // straight copy of 16-byte pieces (at most 8 per thread: one round trip)
-        const f4* Pg = P16 ? reinterpret_cast<const f4*>(d.P) + (size_t)b0 * d.K
-                           : reinterpret_cast<const f4*>(d.P + (size_t)b0 * d.K * M);
-        f4* Pl = reinterpret_cast<f4*>(Ps);
+        const f32x4* Pg = P16 ? reinterpret_cast<const f32x4*>(d.P) + (size_t)b0 * d.K
+                           : reinterpret_cast<const f32x4*>(d.P + (size_t)b0 * d.K * M);
+        f32x4* Pl = reinterpret_cast<f32x4*>(Ps);
         const int n4 = nbc * d.K * (P16 ? 4 : MC) / 4;
         for (int i0 = 0; i0 < n4; i0 += kGThreads * 8) {
-            f4 v[8];
+            f32x4 v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {  // nontemporal, as the M == 1 gather's P slice
-                typedef float f4v __attribute__((ext_vector_type(4)));
-                v[j] = __builtin_nontemporal_load(reinterpret_cast<const f4v*>(Pg) +
+                typedef float f32x4v __attribute__((ext_vector_type(4)));
+                v[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4v*>(Pg) +
                                                   min(i0 + j * kGThreads + tid, n4 - 1));
             }
             if (i0 == 0) {
@@ -1488,91 +1516,134 @@ void gatherv_kernel(Params p) {
     }
 }
 
-// ---- kernel 2, any M / any slot count: workgroup = (chunk, row tile of Rt rows); the
-// chunk's P slice is staged MV columns at a time, code words are read per pair.
-template <int MV>
-__global__ __launch_bounds__(kThreads) void gatherm_kernel(Params p) {
-    extern __shared__ float smem[];
-    int g, c, sidx;
-    if (!gather_slot(p, g, c, sidx)) return;
+// ---- kernel 2, any M / any slot count: workgroup = (chunk, Rt rows, MC columns). The chunk's P
+// slice of those columns is staged in LDS as [block][atom][MC]; a row is 4 lanes per group of 4
+// columns, lane q of the four taking the row's words q, q + 4, ... (8 in flight), and the four
+// meet by two butterfly steps, each lane adding one column into Y. Bound by its round trips (P
+// slice, words) where the matrix is small, so a workgroup takes one pass of 256 threads' rows
+// until there are more of those than two per CU. (4864 x 896, 24 slots, K = 512, M = 8: 11.4 us
+// with a thread per row and 4 columns at a time, of which 64 of 256 threads had a row, 4.6
+// here; M = 1: 6.7 -> 4.3; 4096 x 11008, 6 slots, M = 8: 117 -> 36.)
+constexpr int kGgGammaLds = 1024;  // slot gains kept in LDS, at most
+constexpr int kGgWords = 8;        // words in flight per lane
+
+inline __host__ __device__ int gatherg_rows(int mc) { return kThreads / (mc == 8 ? 8 : 4); }
+
+template <int MC>
+__global__ __launch_bounds__(kThreads) void gatherg_kernel(Params p) {
+    constexpr int CPT = MC < 4 ? MC : 4;  // columns per lane
+    constexpr int TPR = MC == 8 ? 8 : 4;  // lanes per row
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    int g = 0;
+    while (g + 1 < p.G && (int)blockIdx.x >= p.m[g + 1].g_base) ++g;
     const MatDesc& d = p.m[g];
+    const int u = (int)blockIdx.x - d.g_base;
+    const int c = u / d.splits, sidx = u - c * d.splits;
     const int tid = threadIdx.x;
-    const int M = p.M;
+    const int M = p.M, m0 = (p.z0 + (int)blockIdx.y) * MC;
     uint32_t b0u, nbcu;
     csdr::chunk_span((uint32_t)c, (uint32_t)d.NB, (uint32_t)d.NBc, b0u, nbcu);
     const int b0 = (int)b0u, nbc = (int)nbcu;
-    const int r0 = sidx * d.Rt;
-    const int nr = min(d.Rt, d.R - r0);
-    if (nr <= 0) return;
-    const int npairs = nr * nbc;
-    const uint32_t* cb =
-        d.codes + (size_t)b0 * d.R * d.slots + (size_t)r0 * nbc * d.slots;
-    float* Ps = smem;                              // nbc * K * MV
-    float* part = smem + (size_t)d.NBc * d.K * MV; // Rt * NBc * MV
+    const int r0 = sidx * d.Rt, rend = min(r0 + d.Rt, d.R);
+    float* Ps = smem;                           // nbc * K * MC
+    float* gs = smem + (size_t)d.NBc * d.K * MC;  // slot gains
+    const bool gl = d.slots <= kGgGammaLds;
+    const int sg = tid & 3, mg = TPR == 8 ? (tid >> 2 & 1) : 0;
+    const int W = nbc * d.slots;  // words of a row
+    const uint32_t* cb = d.codes + (size_t)b0 * d.R * d.slots;
+    // a lane's words of a row, kGgWords at a time (past the row's last one, that one); the first
+    // row's are in flight while P is staged
+    const int r = r0 + tid / TPR;
+    uint32_t wv[kGgWords];
+    auto load_words = [&](uint32_t (&w)[kGgWords], int row, int q0) {
+        const uint32_t* src = cb + (size_t)min(row, d.R - 1) * W;
+#pragma unroll
+        for (int j = 0; j < kGgWords; ++j) w[j] = src[min(q0 + 4 * j + sg, W - 1)];
+    };
+    load_words(wv, r, 0);
+    {
+        const float* Pg = d.P + (size_t)b0 * d.K * M + m0;
+        const int np = nbc * d.K * MC;
+        if (M == MC && MC >= 4) {
+            copy_to_lds4(Pg, np, Ps);  // the slice as it lies (16-byte aligned at MC >= 4)
+        } else {
+            // (kStageBatch loads in flight per thread, at clamped indices)
+            for (int i0 = 0; i0 < np; i0 += kThreads * kStageBatch) {
+                float v[kStageBatch];
+#pragma unroll
+                for (int j = 0; j < kStageBatch; ++j) {
+                    const int i = min(i0 + j * kThreads + tid, np - 1);
+                    v[j] = Pg[(size_t)(i / MC) * M + min(i % MC, M - 1 - m0)];
+                }
+#pragma unroll
+                for (int j = 0; j < kStageBatch; ++j) Ps[min(i0 + j * kThreads + tid, np - 1)] = v[j];
+            }
+        }
+        if (gl)
+            for (int i = tid; i < d.slots; i += kThreads) gs[i] = d.slot_gamma[i];
+    }
+    __syncthreads();
     const bool last_chunk = (c == d.nchunks - 1);
-    for (int z = 0; z < p.MVz; ++z) {
-        const int m0 = z * MV;
-        if (z > 0) __syncthreads();
-        const float* Pg = d.P + (size_t)b0 * d.K * M;
-        // (kStageBatch loads in flight per thread, at clamped indices: a load under the
-        // column test waited for the one before it)
-        const int np = nbc * d.K * MV;
-        for (int i0 = 0; i0 < np; i0 += kThreads * kStageBatch) {
-            float v[kStageBatch];
+    // gain (0 past the last word) and P offset of each of the lane's words from q0 on
+    float gm[kGgWords];
+    int po[kGgWords];
+    auto place = [&](int q0) {
 #pragma unroll
-            for (int j = 0; j < kStageBatch; ++j) {
-                const int i = min(i0 + j * kThreads + tid, np - 1);
-                const int e = i / MV, mm = i - e * MV;
-                v[j] = Pg[(size_t)e * M + min(m0 + mm, M - 1)];
-            }
+        for (int j = 0; j < kGgWords; ++j) {
+            const int q = min(q0 + 4 * j + sg, W - 1);
+            const int bb = nbc == 1 ? 0 : q / d.slots, sl = q - bb * d.slots;
+            gm[j] = q0 + 4 * j + sg >= W ? 0.0f : gl ? gs[sl] : d.slot_gamma[sl];
+            po[j] = bb * d.K * MC + 4 * mg;
+        }
+    };
+    float acc[CPT];
+    auto add = [&](const uint32_t (&w)[kGgWords]) {
 #pragma unroll
-            for (int j = 0; j < kStageBatch; ++j) {
-                const int i = i0 + j * kThreads + tid;
-                if (i < np) Ps[i] = (m0 + (i % MV) < M) ? v[j] : 0.0f;
+        for (int j = 0; j < kGgWords; ++j) {
+            const float cf = gm[j] * csdr::h2f(w[j] >> 16);
+            const float* pv = Ps + po[j] + (w[j] & 0x7FFFu) * MC;
+            if constexpr (CPT == 4) {
+                const float4 v = *reinterpret_cast<const float4*>(pv);
+                acc[0] = fmaf(cf, v.x, acc[0]);
+                acc[1] = fmaf(cf, v.y, acc[1]);
+                acc[2] = fmaf(cf, v.z, acc[2]);
+                acc[3] = fmaf(cf, v.w, acc[3]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < CPT; ++e) acc[e] = fmaf(cf, pv[e], acc[e]);
             }
         }
-        __syncthreads();
-        for (int pi = tid; pi < npairs; pi += kThreads) {
-            const int bb = pi % nbc;
-            const float* Pb = Ps + (size_t)bb * d.K * MV;
-            const uint32_t* src = cb + (size_t)pi * d.slots;
-            float acc[MV];
+    };
+    const bool one = W <= 4 * kGgWords;  // a row is one round of words: the next row's in flight
+    if (one) place(0);
+    for (int row = r; row - tid / TPR < rend; row += kThreads / TPR) {
 #pragma unroll
-            for (int mm = 0; mm < MV; ++mm) acc[mm] = 0.0f;
-            // the pair's code words and gains 8 at a time, all loaded before the first is used
-            // and all used (slots past the last repeat it with a zero coefficient): a load per
-            // slot under the loop's exit ran a round trip per slot
-            for (int s0 = 0; s0 < d.slots; s0 += 8) {
-                uint32_t wv[8];
-                float gv[8];
+        for (int e = 0; e < CPT; ++e) acc[e] = 0.0f;
+        if (one) {
+            uint32_t nx[kGgWords];
+            load_words(nx, row + kThreads / TPR, 0);
+            add(wv);
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int sj = min(s0 + j, d.slots - 1);
-                    wv[j] = src[sj];
-                    gv[j] = d.slot_gamma[sj];
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const uint32_t w = wv[j];
-                    const float cf = s0 + j < d.slots ? gv[j] * csdr::h2f(w >> 16) : 0.0f;
-                    const float* pv = Pb + (size_t)(w & 0x7FFFu) * MV;
-#pragma unroll
-                    for (int mm = 0; mm < MV; ++mm) acc[mm] = fmaf(cf, pv[mm], acc[mm]);
-                }
+            for (int j = 0; j < kGgWords; ++j) wv[j] = nx[j];
+        } else {
+            for (int q0 = 0; q0 < W; q0 += 4 * kGgWords) {
+                load_words(wv, row, q0);
+                place(q0);
+                add(wv);
             }
-#pragma unroll
-            for (int mm = 0; mm < MV; ++mm) part[pi * MV + mm] = acc[mm];
         }
-        __syncthreads();
-        for (int t = tid; t < nr * MV; t += kThreads) {
-            const int rr = t / MV, mm = t - rr * MV;
-            const int m = m0 + mm;
-            if (m >= M) continue;
-            float sum = 0.0f;
-            for (int bb = 0; bb < nbc; ++bb) sum += part[(rr * nbc + bb) * MV + mm];
-            const int r = r0 + rr;
-            if (last_chunk && d.Ce > 0) sum += edge_term(p, d, r, m);
-            __hip_atomic_fetch_add(d.y + yi(p, d, r, m), sum, __ATOMIC_RELAXED,
+        float sum = 0.f;
+#pragma unroll
+        for (int e = 0; e < CPT; ++e) {
+            float v = acc[e];
+            v += dpp_move<0xB1>(v);  // lanes 0-1, 2-3
+            v += dpp_move<0x4E>(v);  // all four
+            if (sg == e) sum = v;
+        }
+        const int m = m0 + 4 * mg + sg;
+        if (sg < CPT && row < rend && m < M) {
+            if (last_chunk && d.Ce > 0) sum += edge_term(p, d, row, m);
+            __hip_atomic_fetch_add(d.y + yi(p, d, row, m), sum, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         }
     }
@@ -2193,11 +2264,12 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
     p.G = n;
     p.M = M;
     p.p16 = vec && group_p16(n, segs, M) ? 1 : 0;
-    // generic gather: P staged 4 columns at a time when that fits in LDS, else 1
+    // generic gather: M rounded up to 1, 2, 4 or 8 columns at a time, fewer where the P slice
+    // would not leave two workgroups a CU's LDS
     size_t max_pk = 0;
     for (int i = 0; i < n; ++i) max_pk = std::max(max_pk, (size_t)segs[i]->NBc * segs[i]->K);
-    const int MV = (M == 1 || max_pk * 4 * 4 > 96 * 1024) ? 1 : 4;
-    p.MVz = (M + MV - 1) / MV;
+    int gmc = M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : 8));
+    while (gmc > 1 && max_pk * 4 * gmc > 72 * 1024) gmc /= 2;
     p.x_f16 = (x_dtype == CSDR_F16);
     p.tm = tm ? 1 : 0;
     p.accumulate = (flags & CSDR_HSDB_ACCUMULATE) ? 1 : 0;
@@ -2213,7 +2285,7 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
     // pieces) and the same count across the group; anything else takes the generic gather
     int slots = -1;
     bool fast = (M == 1);
-    int ndx = 0;
+    int ndx = 0, ndg = 0;
     size_t lds_dx = 0, lds_g = 0;
     // 2 <= M <= 16 with 64-long blocks everywhere: the thread-per-atom dx kernel
     bool dxm = M >= 2 && M <= kMaxXopM;
@@ -2282,11 +2354,17 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
                 extra = ((size_t)d.PB * 64 / std::max(1, xa.hd) + 2) * (xa.nsplit + 1) * 4;
             lds_dx = std::max(lds_dx, (size_t)d.PB * 64 * M * 4 + extra);
         } else {
-            const long long items = (long long)d.NB * d.K * ((M + 7) / 8);
-            d.dx_count = (int)((items + kThreads / 64 - 1) / (kThreads / 64));
+            d.dx_count = 0;  // dxg_kernel's
+            const long long wgs = M == 1 ? ((long long)d.NB * d.K + 3) / (kThreads / 64)
+                                         : (long long)d.NB * ((d.K + 15) / 16) * ((M + 15) / 16);
+            if (wgs + ndg > 0x7fffffffLL)
+                return set_error(CSDR_E_UNSUPPORTED, "hsdb_matmul: too many blocks");
+            d.dg_count = (int)wgs;
         }
         d.dx_base = ndx;
         ndx += d.dx_count;
+        d.dg_base = ndg;
+        ndg += d.dg_count;
     }
     int dev = 0, ncu = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -2329,14 +2407,19 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
             base += d.g_count;
         }
     } else {
+        const int rows = gatherg_rows(gmc);
+        long long units = 0;
+        for (int i = 0; i < n; ++i)
+            units += (long long)p.m[i].nchunks * ((p.m[i].R + rows - 1) / rows);
+        const int passes = (int)std::max(1LL, std::min(16LL, units / (2 * ncu)));
         for (int i = 0; i < n; ++i) {
             MatDesc& d = p.m[i];
-            d.Rt = MV == 1 ? 256 : 64;
-            while (d.Rt > 16 && (size_t)d.Rt * d.NBc > 2048) d.Rt /= 2;
+            d.Rt = rows * passes;
             d.splits = (d.R + d.Rt - 1) / d.Rt;
-            lds_g = std::max(lds_g, ((size_t)d.NBc * d.K * MV + (size_t)d.Rt * d.NBc * MV) * 4);
+            lds_g = std::max(lds_g, (size_t)d.NBc * d.K * gmc * 4 +
+                                        (size_t)std::min(d.slots, kGgGammaLds) * 4);
             d.g_base = base;
-            d.g_count = (d.nchunks + 7) / 8 * 8 * d.splits;
+            d.g_count = d.nchunks * d.splits;
             base += d.g_count;
         }
     }
@@ -2373,7 +2456,7 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
             default: return set_error(CSDR_E_INVALID, "hsdb_matmul: x op not available at M > 1");
         }
         CSDR_LAUNCH_CHECK("hsdb dx");
-    } else if (phases & kPhaseDx) {
+    } else if ((phases & kPhaseDx) && ndx) {
         switch (p.xop) {
             case CSDR_XOP_RMSNORM:
                 dx_kernel<CSDR_XOP_RMSNORM><<<ndx, kThreads, lds_dx, st>>>(p);
@@ -2390,6 +2473,15 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
         }
         CSDR_LAUNCH_CHECK("hsdb dx");
     }
+    if ((phases & kPhaseDx) && ndg) {
+        bool vec4 = true;  // atom rows of whole 16-byte pieces
+        for (int i = 0; i < n; ++i) vec4 = vec4 && p.m[i].blen % 4 == 0;
+        auto go = [&](auto kern) { kern<<<ndg, M == 1 ? kThreads : kDgThreads, 0, st>>>(p); };
+        if (M == 1) p.x_f16 ? go(&dxw_kernel<_Float16>) : go(&dxw_kernel<float>);
+        else if (p.x_f16) vec4 ? go(&dxg_kernel<_Float16, true>) : go(&dxg_kernel<_Float16, false>);
+        else vec4 ? go(&dxg_kernel<float, true>) : go(&dxg_kernel<float, false>);
+        CSDR_LAUNCH_CHECK("hsdb dx");
+    }
     if (phases & kPhaseGather) {
         if (fast)
             launch_gatherw(p, slots, base, lds_g, st);
@@ -2397,10 +2489,21 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
             p.gtotal = base;
             launch_gatherv(p, slots, (base + 7) / 8 * 8, lds_g, st);
         }
-        else if (MV == 1)
-            gatherm_kernel<1><<<base, kThreads, lds_g, st>>>(p);
-        else
-            gatherm_kernel<4><<<base, kThreads, lds_g, st>>>(p);
+        else {
+            auto go = [&](auto kern) {
+                if (lds_g > 64 * 1024)
+                    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                              hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              (int)lds_g);
+                const int nz = (M + gmc - 1) / gmc;
+                for (p.z0 = 0; p.z0 < nz; p.z0 += 65535)
+                    kern<<<dim3(base, std::min(nz - p.z0, 65535)), kThreads, lds_g, st>>>(p);
+            };
+            if (gmc == 1) go(&gatherg_kernel<1>);
+            else if (gmc == 2) go(&gatherg_kernel<2>);
+            else if (gmc == 4) go(&gatherg_kernel<4>);
+            else go(&gatherg_kernel<8>);
+        }
         CSDR_LAUNCH_CHECK("hsdb gather");
     }
     return CSDR_OK;

@@ -150,3 +150,35 @@ def test_matrix_core_path_token_major(gpu, M):
     (y_tm,) = run_group(gpu, [stream], x, np.float16, M, TOKEN_MAJOR)
     assert rel_l2(y_fm, ref) <= 1e-3 and rel_l2(y_tm, ref) <= 1e-3
     assert rel_l2(y_tm, y_fm) <= 1e-6
+
+
+# The any-block-length dx kernels and the any-slot gather: one tile per row (blocks of C features,
+# off the 64-feature pieces and the 16-byte rows), blocks of 48 with a remainder, slot counts off
+# 4 / 8 / 16 and past one round of words, groups of 64-long and other blocks, each column group
+# (1, 2, 4, 8, more), both element types and layouts, bias and accumulation. fp32 sums of
+# differing order: 1e-5 as above.
+@pytest.mark.parametrize("B,slots", [(896, 24), (130, 5), (48, 6), (64, 3), (1000, 40)])
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 19])
+@pytest.mark.parametrize("flags,dtype", [(0, np.float32), (TOKEN_MAJOR, np.float16)])
+def test_any_block_length_and_slots(gpu, B, slots, M, flags, dtype):
+    from cortexsdr_amd import formats
+
+    rng = np.random.default_rng(B * 100 + slots)
+    K, Cc = 75, (B * 3 + 7 if B < 100 else B + (5 if B == 130 else 0))
+    streams, Rs = [], [101, 40]
+    for R, b, s in zip(Rs, (B, 64), (slots, slots if B != 48 else 9)):
+        nb = Cc // b
+        D = synth.dictionary(K, b, b)
+        idx = rng.integers(0, K, (R * nb, s))
+        coef = rng.normal(0, 0.5, (R * nb, s))
+        edge = rng.normal(0, 0.1, (R, Cc - nb * b)).astype(np.float32) if Cc % b else None
+        streams.append(formats.pack_hsdb(R, Cc, D, idx, coef, gamma=(1.0,), edge=edge))
+    x = synth.activations(Cc, M, seed=7, dtype=dtype)
+    bias = [rng.normal(size=R).astype(np.float32) for R in Rs]
+    y0 = [rng.normal(size=(R, M)).astype(np.float32) for R in Rs]
+    want = [oracle.hsdb_matmul(s, x.astype(np.float32)) for s in streams]
+    ys = run_group(gpu, streams[:1], x, dtype, M, flags)
+    assert rel_l2(ys[0], want[0]) <= 1e-5
+    ys = run_group(gpu, streams, x, dtype, M, flags | ACCUMULATE, bias=bias, y0=y0)
+    for y, w, b, a in zip(ys, want, bias, y0):
+        assert rel_l2(y, a + w + b[:, None]) <= (1e-3 if B == 64 and M > 8 else 1e-5)
