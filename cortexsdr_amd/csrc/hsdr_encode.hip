@@ -38,10 +38,13 @@
 #include "common.hpp"
 
 namespace csdr {
-// fitHierarchicalKSVD's dictionary initialisation, in the reference build's arithmetic (returns
-// the mean tile norm), and atomUpdateStep's re-seed of an atom (hsdr_init.cpp).
-double hsdr_init_dictionary(const float* tiles, uint32_t n, uint32_t C, uint16_t K,
-                            uint32_t slots, float* D, std::mt19937* rng);
+// fitHierarchicalKSVD's dictionary initialisation, in the reference build's arithmetic: the
+// tiles picked, the factors of the atoms made from them (returns the common one), the whole of
+// it on the host; and atomUpdateStep's re-seed of an atom (hsdr_init.cpp).
+void hsdr_init_picks(uint32_t n, uint16_t K, std::mt19937& rng, uint32_t* src);
+float hsdr_init_scales(const float* sq, uint16_t K, uint32_t slots, double mean_norm, float* unit);
+void hsdr_init_dictionary(const float* tiles, uint32_t n, uint32_t C, uint16_t K, uint32_t slots,
+                          float* D);
 void hsdr_reseed_atom(const float* tiles, uint32_t n, uint32_t C, uint64_t base_seed, uint32_t j,
                       uint32_t mul, double target_norm, float* atom);
 }  // namespace csdr
@@ -976,6 +979,84 @@ __global__ __launch_bounds__(kEThreads) void atom_finish_kernel(FitArgs a) {
     }
 }
 
+// ---------------------------------------------------------------- the initial dictionary
+
+// hsdr_init.cpp's sums on the device, operation for operation (no contraction: its products and
+// sums are rounded where that file rounds them; fma is one rounding on both). On the host
+// the tile norms were a library call per element, 9 ms for 4864 x 896.
+//  tile_norms_kernel: squared_norm_d of every tile, a lane per one of its four partial sums;
+//  atom_norms_kernel: squared_norm of the picked tiles, a lane per one of its eight;
+//  init_atoms_kernel: (tile * unit) * scale.
+__global__ __launch_bounds__(kEThreads) void tile_norms_kernel(const float* __restrict__ tiles,
+                                                               uint32_t n, uint32_t C,
+                                                               double* __restrict__ out) {
+#pragma clang fp contract(off)
+    const uint32_t i = blockIdx.x * (kEThreads / 4) + threadIdx.x / 4;
+    const int j = threadIdx.x & 3;
+    const float* t = tiles + (size_t)min(i, n - 1) * C;
+    double a = 0.0;
+    uint32_t c = 0;
+#pragma unroll 4
+    for (; c + 8 <= C; c += 8) {
+        const double lo = t[c + j], hi = t[c + 4 + j];
+        const double h2 = hi * hi;
+        a = a + fma(lo, lo, h2);
+    }
+    const double a2 = a + __shfl_xor(a, 2, 4);        // lanes 0 + 2 and 1 + 3
+    double total = a2 + __shfl_xor(a2, 1, 4);
+    if (C - c >= 4) {
+        const double t0 = t[c], t1 = t[c + 1], t2 = t[c + 2], t3 = t[c + 3];
+        const double p2 = t2 * t2, p3 = t3 * t3;
+        const double e0 = fma(t0, t0, p2), e1 = fma(t1, t1, p3);
+        const double e = e0 + e1;
+        total = total + e;
+        c += 4;
+    }
+    for (; c < C; ++c) total = fma((double)t[c], (double)t[c], total);
+    if (i < n && j == 0) out[i] = total;
+}
+
+__global__ __launch_bounds__(kEThreads) void atom_norms_kernel(const float* __restrict__ tiles,
+                                                               const uint32_t* __restrict__ src,
+                                                               uint32_t K, uint32_t C,
+                                                               float* __restrict__ out) {
+#pragma clang fp contract(off)
+    const uint32_t a = blockIdx.x * (kEThreads / 8) + threadIdx.x / 8;
+    const int l = threadIdx.x & 7;
+    const float* d = tiles + (size_t)src[min(a, K - 1)] * C;
+    float v = 0.f;
+    uint32_t c = 0;
+#pragma unroll 4
+    for (; c + 8 <= C; c += 8) v = fmaf(d[c + l], d[c + l], v);
+    const float h = v + __shfl_xor(v, 4, 8);   // h[i] = v[i + 4] + v[i]
+    const float s = h + __shfl_xor(h, 2, 8);   // h[2] + h[0], h[3] + h[1]
+    float sq = s + __shfl_xor(s, 1, 8);
+    if (c + 4 <= C) {
+        float p[4];
+        for (int i = 0; i < 4; ++i) p[i] = d[c + i] * d[c + i];
+        const float b0 = p[2] + p[0], b1 = p[3] + p[1];
+        const float b = b1 + b0;
+        sq = sq + b;
+        c += 4;
+    }
+    for (; c < C; ++c) sq = fmaf(d[c], d[c], sq);
+    if (a < K && l == 0) out[a] = sq;
+}
+
+__global__ __launch_bounds__(kEThreads) void init_atoms_kernel(const float* __restrict__ tiles,
+                                                               const uint32_t* __restrict__ src,
+                                                               const float* __restrict__ unit,
+                                                               float scale, uint32_t C,
+                                                               float* __restrict__ D) {
+    const uint32_t j = blockIdx.x;
+    const float* t = tiles + (size_t)src[j] * C;
+    const float u = unit[j];
+    for (uint32_t c = threadIdx.x; c < C; c += kEThreads) {
+        const float d = t[c] * u;
+        D[(size_t)j * C + c] = d * scale;
+    }
+}
+
 // ---------------------------------------------------------------- compress (host side)
 
 struct Geometry {
@@ -1109,14 +1190,49 @@ void put(std::vector<uint8_t>& out, const T& v) {
     out.insert(out.end(), p, p + sizeof(T));
 }
 
-// fitHierarchicalKSVD (HierarchicalSDRStrategy.cpp:494-607) over host tiles (n x tile_dim):
-// the dictionary initialisation on the host from the fit's generator (mt19937(0xC0DE), :513),
-// matching pursuit on the GPU, then ksvd_iters atom-update passes each followed by matching
-// pursuit again (:570-573); D (K x tile_dim, non-finite values zeroed as :592-601) and, when
-// codes is not null, the final codes.
+// The initial dictionary of device tiles into d_D; returns the tiles' mean norm in *mean_norm
+// (the square roots summed in tile order, as hsdr_init.cpp does).
+int init_dictionary_device(const float* d_tiles, uint32_t n, uint32_t C, uint16_t K,
+                           uint32_t slots, std::mt19937& rng, float* d_D, double* mean_norm,
+                           hipStream_t st) {
+    DevBuf ws;  // n squared norms, then K picks, K squared norms, K factors
+    CSDR_HIP_CHECK(hipMalloc(&ws.p, (size_t)n * 8 + (size_t)K * 12));
+    double* d_norm = static_cast<double*>(ws.p);
+    uint32_t* d_src = reinterpret_cast<uint32_t*>(d_norm + n);
+    float* d_sq = reinterpret_cast<float*>(d_src + K);
+    float* d_unit = d_sq + K;
+    std::vector<uint32_t> src(K);
+    csdr::hsdr_init_picks(n, K, rng, src.data());
+    CSDR_HIP_CHECK(hipMemcpyAsync(d_src, src.data(), (size_t)K * 4, hipMemcpyHostToDevice, st));
+    tile_norms_kernel<<<(n + kEThreads / 4 - 1) / (kEThreads / 4), kEThreads, 0, st>>>(
+        d_tiles, n, C, d_norm);
+    atom_norms_kernel<<<(K + kEThreads / 8 - 1) / (kEThreads / 8), kEThreads, 0, st>>>(
+        d_tiles, d_src, K, C, d_sq);
+    CSDR_LAUNCH_CHECK("hsdr_compress norms");
+    std::vector<double> norm(n);
+    std::vector<float> sq(K), unit(K);
+    CSDR_HIP_CHECK(hipMemcpyAsync(norm.data(), d_norm, (size_t)n * 8, hipMemcpyDeviceToHost, st));
+    CSDR_HIP_CHECK(hipMemcpyAsync(sq.data(), d_sq, (size_t)K * 4, hipMemcpyDeviceToHost, st));
+    CSDR_HIP_CHECK(hipStreamSynchronize(st));
+    double sum = 0.0;
+    for (double v : norm) sum += std::sqrt(v);
+    *mean_norm = sum / (double)std::max<uint32_t>(1u, n);
+    const float scale = csdr::hsdr_init_scales(sq.data(), K, slots, *mean_norm, unit.data());
+    CSDR_HIP_CHECK(hipMemcpyAsync(d_unit, unit.data(), (size_t)K * 4, hipMemcpyHostToDevice, st));
+    init_atoms_kernel<<<K, kEThreads, 0, st>>>(d_tiles, d_src, d_unit, scale, C, d_D);
+    CSDR_LAUNCH_CHECK("hsdr_compress atoms");
+    CSDR_HIP_CHECK(hipStreamSynchronize(st));  // the factors and the workspace are this frame's
+    return CSDR_OK;
+}
+
+// fitHierarchicalKSVD (HierarchicalSDRStrategy.cpp:494-607) over tiles (n x tile_dim) in host
+// memory: the dictionary initialisation from the fit's generator (mt19937(0xC0DE), :513),
+// matching pursuit, then ksvd_iters atom-update passes each followed by matching pursuit again
+// (:570-573); D (K x tile_dim, non-finite values zeroed as :592-601) and, when codes is not
+// null, the final codes.
 int fit_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t K,
               uint8_t S, uint8_t k, uint8_t ksvd_iters, const std::vector<float>& gamma,
-              std::vector<float>& D, std::vector<uint16_t>* codes_out, hipStream_t st) {
+              float* D, uint16_t* codes, hipStream_t st) {
     Geometry g{};
     g.n_tiles = n_tiles;
     g.tile_dim = tile_dim;
@@ -1128,20 +1244,20 @@ int fit_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t 
                          "hsdr_compress: K-SVD refinement takes tiles of at most 32768 values");
     int rc = check_mp_shape(n_tiles, (int)tile_dim, K, S, k);
     if (rc != CSDR_OK) return rc;
-    D.assign((size_t)K * tile_dim, 0.0f);
-    std::mt19937 rng(0xC0DE);  // the fit's generator (:513), through init and every pass
-    const double mean_norm = csdr::hsdr_init_dictionary(tiles, n_tiles, tile_dim, K,
-                                                        (uint32_t)S * k, D.data(), &rng);
-    const size_t ncodes = (size_t)n_tiles * S * k;
+    const size_t ncodes = (size_t)n_tiles * S * k, kc = (size_t)K * tile_dim;
     DevBuf d_tiles, d_D, d_codes, d_gram;
     if (gram_pays(n_tiles, (int)tile_dim, K, S, k))
         CSDR_HIP_CHECK(hipMalloc(&d_gram.p, gram_ws_bytes(n_tiles, K)));
     CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, (size_t)n_tiles * tile_dim * 4));
-    CSDR_HIP_CHECK(hipMalloc(&d_D.p, D.size() * 4));
+    CSDR_HIP_CHECK(hipMalloc(&d_D.p, kc * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_tiles.p, tiles, (size_t)n_tiles * tile_dim * 4,
                                   hipMemcpyHostToDevice, st));
-    CSDR_HIP_CHECK(hipMemcpyAsync(d_D.p, D.data(), D.size() * 4, hipMemcpyHostToDevice, st));
+    std::mt19937 rng(0xC0DE);  // the fit's generator (:513), through init and every pass
+    double mean_norm = 0.0;
+    rc = init_dictionary_device(d_tiles.f(), n_tiles, tile_dim, K, (uint32_t)S * k, rng, d_D.f(),
+                                &mean_norm, st);
+    if (rc != CSDR_OK) return rc;
     rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
                    d_codes.u16(), d_gram.p, st);
     if (rc != CSDR_OK) return rc;
@@ -1156,16 +1272,13 @@ int fit_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t 
                            d_codes.u16(), d_gram.p, st);
             if (rc != CSDR_OK) return rc;
         }
-        CSDR_HIP_CHECK(hipMemcpyAsync(D.data(), d_D.p, D.size() * 4, hipMemcpyDeviceToHost, st));
     }
-    if (codes_out) {
-        codes_out->resize(ncodes);
-        CSDR_HIP_CHECK(hipMemcpyAsync(codes_out->data(), d_codes.p, ncodes * 2,
-                                      hipMemcpyDeviceToHost, st));
-    }
+    CSDR_HIP_CHECK(hipMemcpyAsync(D, d_D.p, kc * 4, hipMemcpyDeviceToHost, st));
+    if (codes)
+        CSDR_HIP_CHECK(hipMemcpyAsync(codes, d_codes.p, ncodes * 2, hipMemcpyDeviceToHost, st));
     CSDR_HIP_CHECK(hipStreamSynchronize(st));
-    for (float& x : D)  // the fit's final sanitisation (:592-601)
-        if (!std::isfinite(x)) x = 0.0f;
+    for (size_t i = 0; i < kc; ++i)  // the fit's final sanitisation (:592-601)
+        if (!std::isfinite(D[i])) D[i] = 0.0f;
     return CSDR_OK;
 }
 
@@ -1268,7 +1381,7 @@ CSDR_API int csdr_hsdr_init_dictionary(const float* tiles, uint32_t n_tiles, uin
         k_per_stage == 0)
         return set_error(CSDR_E_INVALID, "hsdr_init_dictionary: bad argument");
     csdr::hsdr_init_dictionary(tiles, n_tiles, tile_dim, n_atoms,
-                               (uint32_t)n_stages * k_per_stage, D, nullptr);
+                               (uint32_t)n_stages * k_per_stage, D);
     return CSDR_OK;
 }
 
@@ -1301,10 +1414,11 @@ CSDR_API int csdr_hsdr_compress(const float* w, uint32_t rows, uint32_t cols, ui
     std::vector<float> copied;
     if (!(g.tr == 1 && g.tc == g.C)) copied = extract_tiles(w, g.R_full, g.C, g.tr, g.tc);
     const float* tiles = copied.empty() ? w : copied.data();
-    std::vector<float> gamma(g.S), D;
+    std::vector<float> gamma(g.S), D((size_t)g.K * g.tile_dim);
     for (uint32_t l = 0; l < g.S; ++l) gamma[l] = std::pow(stage_decay, (float)l);
-    std::vector<uint16_t> codes;
-    rc = fit_tiles(tiles, g.n_tiles, g.tile_dim, g.K, g.S, g.k, ksvd_iters, gamma, D, &codes, st);
+    std::vector<uint16_t> codes((size_t)g.n_tiles * g.S * g.k);
+    rc = fit_tiles(tiles, g.n_tiles, g.tile_dim, g.K, g.S, g.k, ksvd_iters, gamma, D.data(),
+                   codes.data(), st);
     if (rc != CSDR_OK) return rc;
 
     // serialisation (:1197-1237): header, stage scales, D, packed codes, edge strips
@@ -1450,8 +1564,9 @@ CSDR_API int csdr_hsda_build(int n, const char* const* names, const float* const
             }
             Dict d;
             d.key = key;
-            int rc = fit_tiles(pool.data(), fill, tile_dim, key.n_atoms, key.n_stages, key.k, ksvd_iters,
-                               gamma, d.atoms, nullptr, st);
+            d.atoms.resize((size_t)key.n_atoms * tile_dim);
+            int rc = fit_tiles(pool.data(), fill, tile_dim, key.n_atoms, key.n_stages, key.k,
+                               ksvd_iters, gamma, d.atoms.data(), nullptr, st);
             if (rc != CSDR_OK) return rc;
             const size_t di = dicts.size();
             dicts.push_back(std::move(d));

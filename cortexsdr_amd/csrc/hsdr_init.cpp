@@ -32,17 +32,9 @@
 #include <cstdint>
 #include <cstring>
 #include <random>
+#include <vector>
 
 #pragma clang fp contract(off)
-
-// The norms' loops call std::fma per element; a CPU with FMA runs it as one instruction and the
-// lanes as vectors (the values are the same), else it is a library call. The mean norm of a
-// 4864 x 896 matrix and its 512 initial atoms: 9.3 -> 2.4 ms on a Xeon host.
-#if defined(__HIP_DEVICE_COMPILE__)  // hipcc's device pass over this file
-#define CSDR_HOST_FMA
-#else
-#define CSDR_HOST_FMA __attribute__((target_clones("arch=x86-64-v3", "default")))
-#endif
 
 namespace csdr {
 
@@ -70,7 +62,7 @@ float rsqrt_newton(float s) {
     return t * h;
 }
 
-CSDR_HOST_FMA float squared_norm(const float* d, uint32_t C) {
+float squared_norm(const float* d, uint32_t C) {
     float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     uint32_t c = 0;
     for (; c + 8 <= C; c += 8)
@@ -92,7 +84,7 @@ CSDR_HOST_FMA float squared_norm(const float* d, uint32_t C) {
 }
 
 // sum_c (double)t[c]^2 in the order of the reference's vectorised loop (header)
-CSDR_HOST_FMA double squared_norm_d(const float* t, uint32_t C) {
+double squared_norm_d(const float* t, uint32_t C) {
     double total = 0.0;
     uint32_t c = 0;
     if (C >= 8) {
@@ -125,25 +117,38 @@ double mean_tile_norm(const float* tiles, uint32_t n, uint32_t C) {
 
 }  // namespace
 
-// Returns the mean tile norm, which the refinement's target norm (atomUpdateStep) takes too.
-double hsdr_init_dictionary(const float* tiles, uint32_t n, uint32_t C, uint16_t K,
-                            uint32_t slots, float* D, std::mt19937* rng_io) {
-    std::mt19937 local(0xC0DE);
-    std::mt19937& rng = rng_io ? *rng_io : local;  // the fit's generator, seeded 0xC0DE
+// The initial atoms' tiles (:513-519): n_atoms picks from the fit's generator.
+void hsdr_init_picks(uint32_t n, uint16_t K, std::mt19937& rng, uint32_t* src) {
     std::uniform_int_distribution<uint32_t> pick(0, n - 1);
-    for (uint32_t j = 0; j < K; ++j) {
-        const uint32_t src = pick(rng);
-        float* d = D + (size_t)j * C;
-        std::memcpy(d, tiles + (size_t)src * C, sizeof(float) * C);
-        const float r = rsqrt_newton(std::max(squared_norm(d, C), 1e-24f));
-        for (uint32_t c = 0; c < C; ++c) d[c] = d[c] * r;
-    }
-    const double mean_norm = mean_tile_norm(tiles, n, C);
+    for (uint32_t j = 0; j < K; ++j) src[j] = pick(rng);
+}
+
+// Atom j is its tile times unit[j], then times the returned scale; sq: the tiles' squared norms
+// (squared_norm's order).
+float hsdr_init_scales(const float* sq, uint16_t K, uint32_t slots, double mean_norm,
+                       float* unit) {
+    for (uint32_t j = 0; j < K; ++j) unit[j] = rsqrt_newton(std::max(sq[j], 1e-24f));
     float scale = (float)mean_norm;
     const float s = (float)slots;
     if (s > 1.0f) scale = scale * rsqrt_newton(s);
-    for (size_t i = 0; i < (size_t)K * C; ++i) D[i] = D[i] * scale;
-    return mean_norm;
+    return scale;
+}
+
+// The whole initialisation on the host.
+void hsdr_init_dictionary(const float* tiles, uint32_t n, uint32_t C, uint16_t K,
+                          uint32_t slots, float* D) {
+    std::mt19937 rng(0xC0DE);  // the fit's generator
+    std::vector<uint32_t> src(K);
+    std::vector<float> sq(K), unit(K);
+    hsdr_init_picks(n, K, rng, src.data());
+    for (uint32_t j = 0; j < K; ++j) sq[j] = squared_norm(tiles + (size_t)src[j] * C, C);
+    const float scale =
+        hsdr_init_scales(sq.data(), K, slots, mean_tile_norm(tiles, n, C), unit.data());
+    for (uint32_t j = 0; j < K; ++j)
+        for (uint32_t c = 0; c < C; ++c) {
+            const float d = tiles[(size_t)src[j] * C + c] * unit[j];
+            D[(size_t)j * C + c] = d * scale;
+        }
 }
 
 // atomUpdateStep's re-seed of atom j (:411-425 for an atom nobody uses, seed constant
