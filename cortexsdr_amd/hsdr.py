@@ -35,18 +35,32 @@ def _check(rc: int) -> None:
         raise CompressionError(rc, msg.decode() if msg else "")
 
 
-def _torch():
-    import torch
+_ready = None  # torch, once it has found a device
 
-    if not torch.cuda.is_available():
-        raise RuntimeError("cortexsdr_amd needs a HIP device (no CPU fallback)")
-    return torch
+
+def _torch():
+    global _ready
+    if _ready is None:
+        import torch
+
+        if not torch.cuda.is_available():
+            raise RuntimeError("cortexsdr_amd needs a HIP device (no CPU fallback)")
+        torch.cuda.init()
+        _ready = torch
+    return _ready
 
 
 def _stream_ptr(stream=None) -> int:
+    """The hipStream_t of `stream`, or of the current device's current stream: torch's own raw
+    accessor where it has one (0.2 us; building a Stream object for it takes 2.8, a third of a
+    small product's call)."""
+    if stream is not None:
+        return int(stream.cuda_stream)
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return int(s.cuda_stream)
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return int(torch.cuda.current_stream().cuda_stream)
+    return int(raw(torch.cuda.current_device()))
 
 
 class HsdbSegment:
