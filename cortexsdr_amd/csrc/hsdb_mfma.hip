@@ -2,18 +2,16 @@
 //
 // Path (cortexSDR tree): HierarchicalSDRStrategy::matmulRowMajor with batch > 1
 // (strategies/HierarchicalSDRStrategy.cpp:1257-1338), block-coded as in research
-// exp_c_kernel/benchmark.py:106-130. W is never stored: each 64-column tile of a 128-row
-// strip is decoded into registers straight in the MFMA A-operand layout and multiplied
-// against the matching 64 x M slice of X.
+// exp_c_kernel/benchmark.py:106-130. W is never stored: 64-column tiles of a row strip are
+// decoded to fp16, in LDS or in registers, and multiplied against the matching 64 x M slice of X.
 //
 // Decode: W[r][k] = g0 * sum_j (c_j * g_j / g0) * D[idx_j][k] over the row's slots (g0 the
-// largest stage gain), with the
-// dictionary held in LDS as fp16 (K <= 1024 atoms: 128 KiB): packed fp16 fused multiply-adds
-// (v_pk_fma_f16, two weights per lane instruction) accumulate each lane's 16 weights of a
-// row straight in the A-operand registers of the matrix-core step (v_mfma_f32_16x16x32_f16,
-// fp32 accumulation; gfx950 runs it at full rate), and g0 scales the fp32 result. X is fp16 as given, or split into fp16 hi + lo parts for fp32 input (two
-// MFMAs). The fp16 dictionary and the fp16 accumulation over the slots keep the product
-// within ~5e-4 relative L2 of the fp32 decode (the path's bar is 1e-3).
+// largest stage gain), with the dictionary held in LDS as fp16 (K <= 1024 atoms: 128 KiB):
+// packed fp16 fused multiply-adds (v_pk_fma_f16, two weights per lane instruction) over the
+// slots in order, fp32 accumulation on the matrix cores (v_mfma_f32_16x16x32_f16; gfx950 runs it
+// at full rate), and g0 scales the fp32 result. X is fp16 as given, or split into fp16 hi + lo
+// parts for fp32 input (two MFMAs). The fp16 dictionary and the fp16 accumulation over the slots
+// keep the product within ~5e-4 relative L2 of the fp32 decode (the path's bar is 1e-3).
 //
 // Layout. Every 64-long k range (one block column) is stored permuted (kperm64), in both the
 // LDS dictionary and the transposed X, so that lane l (q = l/16) reads 16 consecutive
@@ -23,15 +21,13 @@
 // 4(l/16) + i (i = 0..3) of column l % 16.
 //
 // Launches: an init kernel (Y = bias (+ Y when accumulating) + the fp32 edge strip times X,
-// and X transposed to fp16 [m][k] with the permutation, in the workspace), then one
-// persistent kernel: workgroup = 8 or 16 waves x 16 rows; the (row strip, block column) units
-// of all matrices are split in contiguous ranges over the workgroups, and each strip's
-// partial sums are added into Y with device-scope float atomics. A unit's X slice is staged
-// in LDS by the workgroup (two barriers per unit), or, for a single 16-column tile, each wave
-// loads its X operands from the workspace one unit ahead and the waves run without barriers.
-// At M <= 16 with fp16 X and 4 or 8 slots the persistent kernel is the dictionary route
-// instead (qroute_kernel): no weight is decoded; each unit's Q_b = D . X_b is formed on the
-// matrix cores and every row gathers its slots' rows of Q_b from LDS.
+// and X transposed to fp16 operand granules with the permutation, in the workspace), then one
+// persistent kernel: the (row strip, block column) units of all matrices are split in
+// contiguous ranges over one workgroup per CU, and each strip's partial sums are added into Y
+// with device-scope float atomics. Two or more 16-column tiles: mfma_dec_kernel. One (M <= 16):
+// with fp16 X and 4 or 8 slots the dictionary route (qroute_kernel: no weight is decoded, each
+// unit's Q_b = D . X_b is formed on the matrix cores and every row gathers its slots' rows of Q_b
+// from LDS), else mfma_kernel.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -85,47 +81,84 @@ __device__ __forceinline__ float xget(const MParams& p, const MDesc& d, int k, i
                    : static_cast<const float*>(d.x)[i];
 }
 
-// ---- init: Y start values, and X transposed to [m][k] fp16 in 16-byte granules of the
-// permuted k order (threads run along m, so the X reads coalesce).
-__global__ __launch_bounds__(kThreads) void mfma_init_kernel(MParams p) {
+// Transposed X: 16-byte granule g (8 permuted k positions) of block column b and column m, in the
+// order in which a wave loads a 16-column operand: [b][m / 16][g % 2][g / 2][m % 16], so that
+// one load instruction reads 1 KiB in a row. In halves from xt (the lo part xt_part on).
+__device__ __forceinline__ size_t xt_granule(const MParams& p, int b, int m, int g) {
+    return ((((size_t)b * (p.Mpad >> 4) + (m >> 4)) * 2 + (g & 1)) * 64 + (g >> 1) * 16 + (m & 15)) * 8;
+}
+__device__ __forceinline__ size_t xt_part(const MParams& p, const MDesc& d) {
+    return (size_t)p.Mpad * d.C_full;
+}
+
+// ---- init: Y start values, and X transposed into operand granules. blockIdx.x below xwgs: one
+// block column and up to 64 columns of X through LDS (read along X's rows, written granule by
+// granule; straight from X to the granules each lane's 8 values were 8 separate 2-byte loads
+// and its 16-byte store a line of its own). The others: Y.
+__global__ __launch_bounds__(kThreads) void mfma_init_kernel(MParams p, int xwgs) {
+    __shared__ float tile[64][65];
     const MDesc& d = p.m[blockIdx.y];
-    const int M = p.M;
-    const size_t ny = (size_t)d.R * M;
-    const size_t ngr = (size_t)p.Mpad * d.NB * 8;
-    const size_t nx = (size_t)p.Mpad * d.C_full;
-    const size_t stride = (size_t)gridDim.x * kThreads;
-    for (size_t t = (size_t)blockIdx.x * kThreads + threadIdx.x; t < ny + ngr; t += stride) {
-        if (t < ny) {
-            const int r = p.tm ? (int)(t % d.R) : (int)(t / M);
-            const int m = p.tm ? (int)(t / d.R) : (int)(t - (size_t)r * M);
-            float v = p.accumulate ? d.y[t] : 0.0f;
-            if (d.bias) v += d.bias[r];
-            if (d.Ce > 0) {
-                const float* e = d.edge + (size_t)r * d.Ce;
-                float s = 0.0f;
-                for (int cc = 0; cc < d.Ce; ++cc)
-                    s = fmaf(e[cc], xget(p, d, d.C_full + cc, m), s);
-                v += s;
+    const int M = p.M, tid = threadIdx.x;
+    if ((int)blockIdx.x < xwgs) {
+        const int mw = min(64, p.Mpad);        // columns of a tile: 16, 32 or 64
+        const int nmt = p.Mpad / mw;
+        const int b = blockIdx.x / nmt, m0 = (blockIdx.x - b * nmt) * mw;
+        if (b >= d.NB) return;
+        const int n = 64 * mw;
+        // feature-major: threads along a feature's columns; token-major: along a column's features
+        // (four loads in flight per thread, at clamped columns)
+        for (int i0 = tid; i0 < n; i0 += 4 * kThreads) {  // n is a multiple of 4 kThreads
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = i0 + e * kThreads;
+                const int k = p.tm ? (i & 63) : i / mw, c = p.tm ? (i >> 6) : i & (mw - 1);
+                v[e] = xget(p, d, b * 64 + k, min(m0 + c, M - 1));
             }
-            d.y[t] = v;
-        } else {
-            const size_t u = t - ny;
-            const int m = (int)(u % p.Mpad);
-            const size_t bg = u / p.Mpad;
-            const int b = (int)(bg >> 3), g = (int)(bg & 7);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int i = i0 + e * kThreads;
+                const int k = p.tm ? (i & 63) : i / mw, c = p.tm ? (i >> 6) : i & (mw - 1);
+                tile[k][c] = m0 + c < M ? v[e] : 0.0f;
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < mw * 8; i += kThreads) {
+            const int c = i & (mw - 1), g = i / mw;
             _Float16 hi[8], lo[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
-                const int k = b * 64 + csdr::kperm64(g * 8 + j);
-                const float xv = (m < M) ? xget(p, d, k, m) : 0.0f;
+                const float xv = tile[csdr::kperm64(g * 8 + j)][c];
                 hi[j] = (_Float16)xv;
                 lo[j] = (_Float16)(xv - (float)hi[j]);
             }
-            const size_t o = (size_t)m * d.C_full + (size_t)b * 64 + g * 8;
+            const size_t o = xt_granule(p, b, m0 + c, g);
             *reinterpret_cast<u32x4*>(d.xt + o) = __builtin_bit_cast(u32x4, hi);
             if (!p.x_f16)
-                *reinterpret_cast<u32x4*>(d.xt + nx + o) = __builtin_bit_cast(u32x4, lo);
+                *reinterpret_cast<u32x4*>(d.xt + xt_part(p, d) + o) = __builtin_bit_cast(u32x4, lo);
         }
+        return;
+    }
+    if (p.accumulate && !d.bias && d.Ce == 0) return;  // Y stays as it is
+    const size_t ny = (size_t)d.R * M;
+    const size_t stride = (size_t)(gridDim.x - xwgs) * kThreads;
+    if (!p.accumulate && !d.bias && d.Ce == 0) {
+        for (size_t t = (size_t)(blockIdx.x - xwgs) * kThreads + tid; t < ny; t += stride)
+            d.y[t] = 0.0f;
+        return;
+    }
+    for (size_t t = (size_t)(blockIdx.x - xwgs) * kThreads + tid; t < ny; t += stride) {
+        const int r = p.tm ? (int)(t % d.R) : (int)(t / M);
+        const int m = p.tm ? (int)(t / d.R) : (int)(t - (size_t)r * M);
+        float v = p.accumulate ? d.y[t] : 0.0f;
+        if (d.bias) v += d.bias[r];
+        if (d.Ce > 0) {
+            const float* e = d.edge + (size_t)r * d.Ce;
+            float s = 0.0f;
+            for (int cc = 0; cc < d.Ce; ++cc) s = fmaf(e[cc], xget(p, d, d.C_full + cc, m), s);
+            v += s;
+        }
+        d.y[t] = v;
     }
 }
 
@@ -136,27 +169,22 @@ __device__ __forceinline__ int find_matrix(const MParams& p, int u, int g) {
     return g;
 }
 
-// ---- main: persistent; NT = 16-column tiles of this launch, XS = fp32-X split, W waves of
-// 32 rows (strip = 32 W rows). The codes and X slice of unit u + 1 are loaded into registers
-// while unit u is decoded and multiplied. One workgroup per CU (the dictionary fills most of
-// the LDS), so latency is hidden by the W waves of that workgroup.
-// XR: each wave loads its X operands straight from the transposed X (global memory, L1/L2
-// hits: the workgroup's waves all take the same unit sequence) one unit ahead, so the units
-// need no X staging and no barriers; the waves run apart and one's LDS reads overlap
-// another's arithmetic. Else the unit's X slice is staged in LDS by the whole workgroup.
-// LB: slots whose dictionary reads are issued together before their multiply-adds.
-template <int NT, bool XS, int W, int RT, int SLOTS, bool XR>
-__global__ __launch_bounds__(W * 64) void mfma_kernel(MParams p) {
+// ---- main, one 16-column tile (M <= 16) where the dictionary route below does not run (fp32 X,
+// 16 slots): 16 waves, each decoding its own 16-row strips' tiles into the A operands of the
+// matrix-core steps. XS: fp32-X split. The codes and X operands of unit u + 1 are loaded into
+// registers while unit u is decoded and multiplied (X straight from the transposed X: global
+// memory, L1 / L2 hits, as the waves all take the same unit sequence), so the units need no
+// barriers. The slots' dictionary reads are issued four at a time before their multiply-adds.
+template <bool XS, int SLOTS>
+__global__ __launch_bounds__(1024) void mfma_kernel(MParams p) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    constexpr int W = 16;
     constexpr int CW = SLOTS / 4;  // 16-byte code pieces per tile
     constexpr int kThreads = W * 64;
-    constexpr int kStripRows = W * 16 * RT;
+    constexpr int kStripRows = W * 16;
     extern __shared__ __attribute__((aligned(16))) _Float16 smem16[];
-    constexpr int MT = NT * 16;
-    constexpr int NGR = MT * 8 * (XS ? 2 : 1);  // 16-byte X granules per unit
-    constexpr int GPT = XR ? 1 : (NGR + kThreads - 1) / kThreads;
     constexpr int NP = XS ? 2 : 1;           // X parts (fp32 X: hi, lo)
-    constexpr int LB = SLOTS < 4 ? SLOTS : 4;
+    constexpr int LB = 4;
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
     const int q = lane >> 4, rl = lane & 15;
@@ -167,13 +195,11 @@ __global__ __launch_bounds__(W * 64) void mfma_kernel(MParams p) {
     // K x 64; 16-byte granule g of atom a at g ^ ((a >> 1) & 7): rows are 128 bytes, so
     // without it the 16 lanes of one k segment would meet in two bank groups
     _Float16* Ds = smem16;
-    _Float16* Xs = smem16 + (size_t)kMaxAtoms * 64;  // MT x 64 (hi), then MT x 64 (lo)
     const int M = p.M;
 
-    floatx4 acc[RT][NT];
-    u32x4 xr[GPT];   // prefetched X granules of the next unit (staged X)
-    u32x4 xb[XR ? NT : 1][NP][2];  // prefetched X operands of the next unit (XR)
-    u32x4 cr[RT][CW];  // prefetched code words of the next unit (RT row tiles)
+    floatx4 acc;
+    u32x4 xb[NP][2];  // prefetched X operands of the next unit
+    u32x4 cr[CW];     // prefetched code words of the next unit
     int ng = -1, nstrip = 0, nb = 0;  // the prefetched unit
 
     auto prefetch = [&](int u) {
@@ -182,70 +208,40 @@ __global__ __launch_bounds__(W * 64) void mfma_kernel(MParams p) {
         const int lu = u - d.u_base;
         nstrip = lu / d.NB;
         nb = lu - nstrip * d.NB;
-        const size_t nxt = (size_t)p.Mpad * d.C_full;
-        if constexpr (XR) {
-            // lane (column n = 16 nt + rl, group q): granules 2q and 2q + 1 of the block
+        // lane (column rl, group q): granules 2q and 2q + 1 of the block
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+        for (int part = 0; part < NP; ++part)
 #pragma unroll
-                for (int part = 0; part < NP; ++part)
+            for (int c = 0; c < 2; ++c)
+                xb[part][c] = *reinterpret_cast<const u32x4*>(
+                    d.xt + part * xt_part(p, d) + xt_granule(p, nb, p.m0 + rl, 2 * q + c));
+        const int r = min(nstrip * kStripRows + wave * 16 + rl, d.R - 1);
+        const uint32_t* cw = d.codes + csdr::tile_word_offset(r, nb, d.R, d.NB, d.NBc, d.slots);
 #pragma unroll
-                    for (int c = 0; c < 2; ++c)
-                        xb[nt][part][c] = *reinterpret_cast<const u32x4*>(
-                            d.xt + part * nxt + (size_t)(p.m0 + nt * 16 + rl) * d.C_full +
-                            (size_t)nb * 64 + (2 * q + c) * 8);
-        }
-#pragma unroll
-        for (int i = 0; i < (XR ? 0 : GPT); ++i) {
-            const int gi = min(tid + i * kThreads, NGR - 1);
-            const int part = XS ? gi / (MT * 8) : 0;
-            const int gg = gi - part * MT * 8;
-            const int mrow = gg >> 3, gr = gg & 7;
-            xr[i] = *reinterpret_cast<const u32x4*>(
-                d.xt + part * nxt + (size_t)(p.m0 + mrow) * d.C_full + (size_t)nb * 64 + gr * 8);
-        }
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const int r = min(nstrip * kStripRows + wave * 16 * RT + rt * 16 + rl, d.R - 1);
-            const uint32_t* cw =
-                d.codes + csdr::tile_word_offset(r, nb, d.R, d.NB, d.NBc, d.slots);
-#pragma unroll
-            for (int j4 = 0; j4 < CW; ++j4) cr[rt][j4] = *reinterpret_cast<const u32x4*>(cw + j4 * 4);
-        }
+        for (int j4 = 0; j4 < CW; ++j4) cr[j4] = *reinterpret_cast<const u32x4*>(cw + j4 * 4);
     };
 
     auto flush = [&](int g, int strip) {
         const MDesc& d = p.m[g];
+        const int rbase = strip * kStripRows + wave * 16 + q * 4;
+        const int m = p.m0 + rl;
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            const int rbase = strip * kStripRows + wave * 16 * RT + rt * 16 + q * 4;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int m = p.m0 + nt * 16 + rl;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int r = rbase + i;
-                    if (r < d.R && m < M)
-                        __hip_atomic_fetch_add(d.y + (p.tm ? (size_t)m * d.R + r : (size_t)r * M + m),
-                                               acc[rt][nt][i] * d.g0,
-                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-            }
+        for (int i = 0; i < 4; ++i) {
+            const int r = rbase + i;
+            if (r < d.R && m < M)
+                __hip_atomic_fetch_add(d.y + (p.tm ? (size_t)m * d.R + r : (size_t)r * M + m),
+                                       acc[i] * d.g0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
 
     int cur_g = -1, cur_strip = -1;
     prefetch(u0);
     for (int u = u0; u < u1; ++u) {
-        const int g = ng, strip = nstrip, b = nb;
-        (void)b;
+        const int g = ng, strip = nstrip;
         const MDesc& d = p.m[g];
         if (g != cur_g || strip != cur_strip) {
             if (cur_strip >= 0) flush(cur_g, cur_strip);
-#pragma unroll
-            for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[rt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            acc = floatx4{0.f, 0.f, 0.f, 0.f};
             if (g != cur_g) {
                 // the matrix's fp16 dictionary -> LDS (16-byte granules, 8 loads in flight)
                 __syncthreads();
@@ -265,111 +261,70 @@ __global__ __launch_bounds__(W * 64) void mfma_kernel(MParams p) {
                                                       ((gr ^ ((a >> 1) & 7)) * 8)) = v[j];
                     }
                 }
-                if constexpr (XR) __syncthreads();
+                __syncthreads();
             }
             cur_g = g;
             cur_strip = strip;
         }
-        u32x4 xc[XR ? NT : 1][NP][2];
-        if constexpr (XR) {
+        u32x4 xc[NP][2];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
+        for (int part = 0; part < NP; ++part)
 #pragma unroll
-                for (int part = 0; part < NP; ++part)
+            for (int c = 0; c < 2; ++c) xc[part][c] = xb[part][c];
+        u32x4 cc[CW];
 #pragma unroll
-                    for (int c = 0; c < 2; ++c) xc[nt][part][c] = xb[nt][part][c];
-        }
-        // X slice -> LDS; granule index XOR (row & 7) against bank conflicts
-        if constexpr (!XR) __syncthreads();
-#pragma unroll
-        for (int i = 0; i < (XR ? 0 : GPT); ++i) {
-            const int gi = min(tid + i * kThreads, NGR - 1);
-            const int part = XS ? gi / (MT * 8) : 0;
-            const int gg = gi - part * MT * 8;
-            const int mrow = gg >> 3, gr = gg & 7;
-            *reinterpret_cast<u32x4*>(Xs + (size_t)part * MT * 64 + mrow * 64 +
-                                      ((gr ^ (mrow & 7)) * 8)) = xr[i];
-        }
-        u32x4 cc[RT][CW];
-#pragma unroll
-        for (int rt = 0; rt < RT; ++rt)
-#pragma unroll
-            for (int j4 = 0; j4 < CW; ++j4) cc[rt][j4] = cr[rt][j4];
-        if constexpr (!XR) __syncthreads();
+        for (int j4 = 0; j4 < CW; ++j4) cc[j4] = cr[j4];
         if (u + 1 < u1) prefetch(u + 1);
-        // decode this lane's 16 k values of each of its rows: per slot the coefficient as an
-        // fp16 pair (times the slot's gain relative to slot 0) and 8 packed fp16 FMAs over the
-        // atom's two 16-byte granules, accumulated in place as the two 8-value A operands
-        half8 a[RT][2];
+        // decode this lane's 16 k values of its row: per slot the coefficient as an fp16 pair
+        // (times the slot's gain relative to the largest) and 8 packed fp16 FMAs over the atom's
+        // two 16-byte granules, accumulated in place as the two 8-value A operands
+        h2 w[8];
 #pragma unroll
-        for (int rt = 0; rt < RT; ++rt) {
-            h2 w[8];
+        for (int t = 0; t < 8; ++t) w[t] = h2{(_Float16)0.0f, (_Float16)0.0f};
 #pragma unroll
-            for (int t = 0; t < 8; ++t) w[t] = h2{(_Float16)0.0f, (_Float16)0.0f};
+        for (int j0 = 0; j0 < SLOTS; j0 += LB) {
+            // the batch's LB atoms: both 16-byte granules of each read before any is used
+            u32x4 lo[LB], hi[LB];
 #pragma unroll
-            for (int j0 = 0; j0 < SLOTS; j0 += LB) {
-                // the batch's LB atoms: both 16-byte granules of each read before any is used
-                u32x4 lo[LB], hi[LB];
-#pragma unroll
-                for (int jj = 0; jj < LB; ++jj) {
-                    const uint32_t word = cc[rt][(j0 + jj) >> 2][(j0 + jj) & 3];
-                    const uint32_t at = word & 0x7FFFu;
-                    const uint32_t sw = (at >> 1) & 7;
-                    const _Float16* drow = Ds + at * 64;
-                    lo[jj] = *reinterpret_cast<const u32x4*>(drow + (((2 * q) ^ sw) * 8));
-                    hi[jj] = *reinterpret_cast<const u32x4*>(drow + (((2 * q + 1) ^ sw) * 8));
-                }
-#pragma unroll
-                for (int jj = 0; jj < LB; ++jj) {
-                    const int j = j0 + jj;
-                    const uint32_t word = cc[rt][j >> 2][j & 3];
-                    // (c, c): the word's high half in both halves
-                    const h2 c2 =
-                        __builtin_bit_cast(h2, __builtin_amdgcn_perm(word, word, 0x07060706u)) *
-                        __builtin_bit_cast(h2, d.grel[j]);
-                    // (vector elements go through a scalar: bit-casting a subscripted vector
-                    // element directly reads element 0 whatever the subscript)
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) {
-                        const uint32_t el = lo[jj][t], eh = hi[jj][t];
-                        w[t] = __builtin_elementwise_fma(c2, __builtin_bit_cast(h2, el), w[t]);
-                        w[4 + t] = __builtin_elementwise_fma(c2, __builtin_bit_cast(h2, eh), w[4 + t]);
-                    }
-                }
+            for (int jj = 0; jj < LB; ++jj) {
+                const uint32_t word = cc[(j0 + jj) >> 2][(j0 + jj) & 3];
+                const uint32_t at = word & 0x7FFFu;
+                const uint32_t sw = (at >> 1) & 7;
+                const _Float16* drow = Ds + at * 64;
+                lo[jj] = *reinterpret_cast<const u32x4*>(drow + (((2 * q) ^ sw) * 8));
+                hi[jj] = *reinterpret_cast<const u32x4*>(drow + (((2 * q + 1) ^ sw) * 8));
             }
 #pragma unroll
-            for (int c = 0; c < 2; ++c) {
-                const u32x4 v = {__builtin_bit_cast(uint32_t, w[4 * c]),
-                                 __builtin_bit_cast(uint32_t, w[4 * c + 1]),
-                                 __builtin_bit_cast(uint32_t, w[4 * c + 2]),
-                                 __builtin_bit_cast(uint32_t, w[4 * c + 3])};
-                a[rt][c] = __builtin_bit_cast(half8, v);
+            for (int jj = 0; jj < LB; ++jj) {
+                const int j = j0 + jj;
+                const uint32_t word = cc[j >> 2][j & 3];
+                // (c, c): the word's high half in both halves
+                const h2 c2 =
+                    __builtin_bit_cast(h2, __builtin_amdgcn_perm(word, word, 0x07060706u)) *
+                    __builtin_bit_cast(h2, d.grel[j]);
+                // (vector elements go through a scalar: bit-casting a subscripted vector
+                // element directly reads element 0 whatever the subscript)
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const uint32_t el = lo[jj][t], eh = hi[jj][t];
+                    w[t] = __builtin_elementwise_fma(c2, __builtin_bit_cast(h2, el), w[t]);
+                    w[4 + t] = __builtin_elementwise_fma(c2, __builtin_bit_cast(h2, eh), w[4 + t]);
+                }
             }
         }
         // two 32-deep steps over the block column: lane group q holds positions 16 q + 8 c ..
         // + 7 of the permuted k order in step c, in both operands
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            const int n = nt * 16 + rl;
-            const int g0 = (2 * q) ^ (n & 7), g1 = (2 * q + 1) ^ (n & 7);
+        for (int c = 0; c < 2; ++c) {
+            const u32x4 v = {__builtin_bit_cast(uint32_t, w[4 * c]),
+                             __builtin_bit_cast(uint32_t, w[4 * c + 1]),
+                             __builtin_bit_cast(uint32_t, w[4 * c + 2]),
+                             __builtin_bit_cast(uint32_t, w[4 * c + 3])};
 #pragma unroll
-            for (int part = 0; part < (XS ? 2 : 1); ++part) {
-                half8 bs[2];
-                if constexpr (XR) {
-                    bs[0] = __builtin_bit_cast(half8, xc[nt][part][0]);
-                    bs[1] = __builtin_bit_cast(half8, xc[nt][part][1]);
-                } else {
-                    const _Float16* xrow = Xs + (size_t)part * MT * 64 + n * 64;
-                    bs[0] = __builtin_bit_cast(half8, *reinterpret_cast<const u32x4*>(xrow + g0 * 8));
-                    bs[1] = __builtin_bit_cast(half8, *reinterpret_cast<const u32x4*>(xrow + g1 * 8));
-                }
-#pragma unroll
-                for (int c = 0; c < 2; ++c)
-#pragma unroll
-                    for (int rt = 0; rt < RT; ++rt)
-                        acc[rt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                            a[rt][c], bs[c], acc[rt][nt], 0, 0, 0);
-            }
+            for (int part = 0; part < NP; ++part)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    __builtin_bit_cast(half8, v), __builtin_bit_cast(half8, xc[part][c]), acc, 0,
+                    0, 0);
         }
     }
     if (cur_strip >= 0) flush(cur_g, cur_strip);
@@ -474,8 +429,8 @@ __global__ __launch_bounds__(1024) void qroute_kernel(MParams p) {
             const uint32_t w = q == 0 ? a0 : (q == 1 ? a1 : (q == 2 ? a2 : a3));
             gl[j] = __builtin_bit_cast(_Float16, (uint16_t)(w & 0xFFFFu));
         }
-        const _Float16* xt0 = d.xt + (size_t)rl * d.C_full + q * 16;
-        const size_t nxt = (size_t)p.Mpad * d.C_full;
+        const _Float16* xt0 = d.xt + xt_granule(p, 0, rl, 2 * q);
+        const size_t nxt = xt_part(p, d);
         const int K = d.K;
         SegGeom sg;
         sg.NB = d.NB;
@@ -494,12 +449,12 @@ __global__ __launch_bounds__(1024) void qroute_kernel(MParams p) {
         for (int e = 0; e < 16; ++e) ya[e] = 0.0f;
 
         auto load_x = [&](const UnitCursor& c, u32x4 (&dst)[NP][2]) {
-            const _Float16* src = xt0 + (size_t)c.b * 64;
+            const _Float16* src = xt0 + (size_t)c.b * 1024;  // Mpad = 16: 2 KiB a block
 #pragma unroll
             for (int part = 0; part < NP; ++part)
 #pragma unroll
                 for (int cc = 0; cc < 2; ++cc)
-                    dst[part][cc] = *reinterpret_cast<const u32x4*>(src + part * nxt + cc * 8);
+                    dst[part][cc] = *reinterpret_cast<const u32x4*>(src + part * nxt + cc * 512);
         };
         auto load_codes = [&](const UnitCursor& c, cword_t& dst) {
             const int r = min(c.strip * 256 + wave * 16 + rl, sg.R - 1);
@@ -683,6 +638,278 @@ __global__ __launch_bounds__(1024) void qroute_kernel(MParams p) {
     }
 }
 
+// ---- main, two or more 16-column tiles: weights decoded once per workgroup into LDS.
+// A workgroup (8 waves) owns strips of ROWS rows. Per unit (strip, block column) the waves decode
+// the ROWS x 64 tile of W into one of two LDS buffers while the previous unit's tile is multiplied
+// from the other with every column of the launch: one barrier a unit.
+// - Decode: a wave takes rows eight at a time, eight lanes a row, lane g of them the 16-byte
+//   granule g of every slot's atom (8 weights): a read covers eight whole 128-byte atom rows,
+//   which no bank conflict can slow (a row per lane and granules apart, as the A operands would
+//   have it, measured 13.7 LDS cycles a read against 9.6), and the slots' packed fp16 FMAs run
+//   in the same order as mfma_kernel's. The tile's granules lie at g ^ (row % 8), so the A
+//   operand reads (16 rows, one granule) spread over all banks.
+// - Product: waves RG x CG, each ROWS / RG rows by CT 16-column tiles; A from the LDS tile, B
+//   straight from the transposed X (1 KiB a load, issued before the unit's decode, used after
+//   it), so that X takes no LDS: where each wave decoded its own rows and read all of X from LDS
+//   for them, the X reads were twice the decode's at 256 columns.
+// - Code words two units ahead in a register ring; every load unconditional (clamped rows, units
+//   past the range's end wrap), as in qroute_kernel.
+// Bound by the LDS at many columns (per 64-row unit of 8 slots and 256 columns 136 KiB read or
+// written, about 1,350 of its 2,000 cycles; matrix cores 512, vector ALU 560), and by the chain of
+// a unit's reads, multiply-adds and writes at few; beside the units a 256-column call of 68 us
+// spends 9 in the init launch, 8 before the first unit and 9 in the atomics into Y.
+// 4096 x 11008, K = 1024, 8 slots, us per call before (each wave decoding its own rows, X through
+// LDS) and after: fp16 X M = 32 40.2 -> 34, 64 48.2 -> 41.4, 128 63.7 -> 54.5, 256 90.7 -> 68;
+// fp32 X M = 32 41.6 -> 35.5, 64 53 -> 48.5, 128 78 -> 69, 256 156 -> 88.
+constexpr int kDecWaves = 8;
+
+template <int ROWS, int RG, int CG, int CT, bool XS, int SLOTS>
+__global__ __launch_bounds__(kDecWaves * 64) void mfma_dec_kernel(MParams p) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    static_assert(RG * CG == kDecWaves, "waves");
+    constexpr int RT = ROWS / 16 / RG;  // 16-row tiles of a wave's product
+    constexpr int NP = XS ? 2 : 1;          // X parts (fp32 X: hi, lo)
+    constexpr int CW = SLOTS / 4;           // 16-byte code pieces per tile
+    constexpr int DG = ROWS / kDecWaves / 8;  // groups of 8 rows that a wave decodes
+    constexpr int TB = ROWS * 64;             // halves of a tile buffer
+    // A unit's atoms read during the unit before, so that they and the A operands' reads keep the
+    // LDS busy through the arithmetic (256 columns 70.8 -> 68.2 us a call, 128 56.0 -> 54.5);
+    // waves without a barrier between their units drift apart and gain nothing by it.
+    constexpr bool AHEAD = CG > 1 && DG * SLOTS <= 16;
+    extern __shared__ __attribute__((aligned(16))) _Float16 smem16[];
+    _Float16* Wt = smem16;           // two tile buffers
+    _Float16* Ds = smem16 + 2 * TB;  // K x 64
+    const int tid = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int q = lane >> 4, rl = lane & 15;
+    const int dr = lane >> 3, dg = lane & 7;  // decode: row of the group, granule
+    const int wr = wave / CG, wc = wave % CG;
+    const int U = p.total_units;
+    const int u0 = (int)((long long)U * blockIdx.x / gridDim.x);
+    const int u1 = (int)((long long)U * (blockIdx.x + 1) / gridDim.x);
+    if (u0 >= u1) return;
+
+    for (int s0 = u0; s0 < u1;) {  // the units of one matrix at a time
+        const int g = find_matrix(p, s0, -1);
+        const MDesc& d = p.m[g];
+        const int s1 = min(u1, d.u_base + d.u_count);
+        SegGeom sg;
+        sg.NB = d.NB;
+        sg.NBc = d.NBc;
+        sg.R = d.R;
+        sg.nstrips = (d.R + ROWS - 1) / ROWS;
+        sg.nfull = d.NB & ~(d.NBc - 1);
+        const uint32_t* codes = d.codes;
+        float* y = d.y;
+        const float g0 = d.g0;
+        uint32_t grel[SLOTS];
+#pragma unroll
+        for (int j = 0; j < SLOTS; ++j) grel[j] = d.grel[j];
+        const size_t nxt = xt_part(p, d), xblk = (size_t)p.Mpad * 64;
+        const _Float16* xt0 = d.xt + xt_granule(p, 0, p.m0 + wc * CT * 16 + rl, 2 * q);
+
+        u32x4 cr[2][DG][CW];
+        auto load_codes = [&](const UnitCursor& c, u32x4 (&dst)[DG][CW]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int e = 0; e < DG; ++e) {
+                const int r = min(c.strip * ROWS + (wave * DG + e) * 8 + dr, sg.R - 1);
+                const uint32_t* w =
+                    codes + ((size_t)c.b0 * sg.R + (size_t)r * c.nbc + (c.b - c.b0)) * SLOTS;
+#pragma unroll
+                for (int j = 0; j < CW; ++j) dst[e][j] = *reinterpret_cast<const u32x4*>(w + 4 * j);
+            }
+        };
+        // the slots' granules of rows group e, all issued before the first is used (left to itself
+        // the compiler keeps three or four in flight)
+        auto atoms = [&](const u32x4 (&cw)[CW], u32x4 (&at)[SLOTS]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int j = 0; j < SLOTS; ++j) {
+                const uint32_t word = cw[j >> 2][j & 3];
+                at[j] = *reinterpret_cast<const u32x4*>(Ds + (word & 0x7FFFu) * 64 + dg * 8);
+            }
+        };
+        auto weights = [&](const u32x4 (&cw)[CW], const u32x4 (&at)[SLOTS], int e,
+                           int buf) __attribute__((always_inline)) {
+            h2 w[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) w[t] = h2{(_Float16)0.0f, (_Float16)0.0f};
+#pragma unroll
+            for (int j = 0; j < SLOTS; ++j) {
+                const uint32_t word = cw[j >> 2][j & 3];
+                const h2 c2 =
+                    __builtin_bit_cast(h2, __builtin_amdgcn_perm(word, word, 0x07060706u)) *
+                    __builtin_bit_cast(h2, grel[j]);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) {
+                    const uint32_t v = at[j][t];
+                    w[t] = __builtin_elementwise_fma(c2, __builtin_bit_cast(h2, v), w[t]);
+                }
+            }
+            const int row = (wave * DG + e) * 8 + dr;
+            const u32x4 v = {__builtin_bit_cast(uint32_t, w[0]), __builtin_bit_cast(uint32_t, w[1]),
+                             __builtin_bit_cast(uint32_t, w[2]), __builtin_bit_cast(uint32_t, w[3])};
+            *reinterpret_cast<u32x4*>(Wt + buf * TB + row * 64 + ((dg ^ (row & 7)) * 8)) = v;
+        };
+        floatx4 acc[RT][CT];
+        auto clear = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int x = 0; x < RT; ++x)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) acc[x][c] = floatx4{0.f, 0.f, 0.f, 0.f};
+        };
+        auto flush = [&](int strip) __attribute__((always_inline)) {
+#pragma unroll
+            for (int x = 0; x < RT; ++x) {
+                const int rbase = strip * ROWS + (wr * RT + x) * 16 + q * 4;
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const int m = p.m0 + (wc * CT + c) * 16 + rl;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int r = rbase + i;
+                        if (r < sg.R && m < p.M)
+                            __hip_atomic_fetch_add(
+                                y + (p.tm ? (size_t)m * sg.R + r : (size_t)r * p.M + m),
+                                acc[x][c][i] * g0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    }
+                }
+            }
+        };
+        // cursors: the unit multiplied, its successor, and the unit whose codes are loaded next
+        UnitCursor cg;
+        {
+            const int lu = s0 - d.u_base;
+            cg.strip = lu / sg.NB;
+            cg.b = lu - cg.strip * sg.NB;
+            cursor_chunk(sg, cg);
+        }
+        UnitCursor cc = cg;
+        load_codes(cc, cr[1]);  // unit s0: ring slot of unit s0 + i is (i + 1) % 2
+        cursor_next(sg, cc);
+        load_codes(cc, cr[0]);
+        cursor_next(sg, cc);
+        {
+            // the matrix's fp16 dictionary -> LDS (16-byte granules, 8 loads in flight)
+            __syncthreads();
+            const int n = d.K * 8;
+            for (int i0 = 0; i0 < n; i0 += kDecWaves * 64 * 8) {
+                u32x4 v[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    v[j] = *reinterpret_cast<const u32x4*>(
+                        d.dict16p + (size_t)min(i0 + j * kDecWaves * 64 + tid, n - 1) * 8);
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    *reinterpret_cast<u32x4*>(
+                        Ds + (size_t)min(i0 + j * kDecWaves * 64 + tid, n - 1) * 8) = v[j];
+            }
+            __syncthreads();
+        }
+        clear();
+#pragma unroll
+        for (int e = 0; e < DG; ++e) {
+            u32x4 at[SLOTS];
+            atoms(cr[1][e], at);
+            weights(cr[1][e], at, e, 0);
+        }
+        load_codes(cc, cr[1]);
+        cursor_next(sg, cc);
+        u32x4 cw[DG][CW], at[AHEAD ? DG : 1][SLOTS];  // unit v + 1's words, and its atoms' granules
+        if constexpr (AHEAD) {
+#pragma unroll
+            for (int e = 0; e < DG; ++e) {
+                atoms(cr[0][e], at[e]);
+#pragma unroll
+                for (int j = 0; j < CW; ++j) cw[e][j] = cr[0][e][j];
+            }
+            load_codes(cc, cr[0]);
+            cursor_next(sg, cc);
+        }
+        auto step = [&](int v, auto S) __attribute__((always_inline)) {
+            constexpr int sl = decltype(S)::value;  // ring slot and target buffer of unit v + 1
+            // unit v's tile is whole, unit v - 1's has been read (with one column group a wave
+            // multiplies the rows that it decoded: nothing to wait for)
+            if constexpr (CG > 1) __syncthreads();
+            u32x4 xb[CT][NP][2];
+            const _Float16* xs = xt0 + (size_t)cg.b * xblk;
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int part = 0; part < NP; ++part)
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+                        xb[c][part][h] = *reinterpret_cast<const u32x4*>(
+                            xs + part * nxt + (size_t)c * 1024 + h * 512);
+            const _Float16* wb = Wt + sl * TB + (wr * RT * 16 + rl) * 64;
+            half8 a[2][RT];
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int x = 0; x < RT; ++x)
+                    a[h][x] = __builtin_bit_cast(
+                        half8, *reinterpret_cast<const u32x4*>(
+                                   wb + x * 16 * 64 + (((2 * q + h) ^ (rl & 7)) * 8)));
+            __builtin_amdgcn_sched_barrier(0);  // the loads above go first
+            if constexpr (AHEAD) {
+                // unit v + 1 from the granules read during the last unit's products, then unit
+                // v + 2's reads, in flight during this unit's
+#pragma unroll
+                for (int e = 0; e < DG; ++e) weights(cw[e], at[e], e, 1 - sl);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < DG; ++e) {
+                    atoms(cr[1 - sl][e], at[e]);
+#pragma unroll
+                    for (int j = 0; j < CW; ++j) cw[e][j] = cr[1 - sl][e][j];
+                }
+                load_codes(cc, cr[1 - sl]);
+                __builtin_amdgcn_sched_barrier(0);
+            } else if constexpr (DG * SLOTS <= 16) {
+                u32x4 ag[DG][SLOTS];
+#pragma unroll
+                for (int e = 0; e < DG; ++e) atoms(cr[sl][e], ag[e]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int e = 0; e < DG; ++e) weights(cr[sl][e], ag[e], e, 1 - sl);
+                load_codes(cc, cr[sl]);
+            } else {  // a group at a time: two groups of 16 slots' reads would spill
+#pragma unroll
+                for (int e = 0; e < DG; ++e) {
+                    u32x4 ag[SLOTS];
+                    atoms(cr[sl][e], ag);
+                    weights(cr[sl][e], ag, e, 1 - sl);
+                }
+                load_codes(cc, cr[sl]);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+#pragma unroll
+                    for (int part = 0; part < NP; ++part)
+#pragma unroll
+                        for (int x = 0; x < RT; ++x)
+                            acc[x][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                                a[h][x], __builtin_bit_cast(half8, xb[c][part][h]), acc[x][c], 0, 0,
+                                0);
+            const int strip = cg.strip;
+            cursor_next(sg, cg);
+            cursor_next(sg, cc);
+            if (v + 1 == s1 || cg.strip != strip) {
+                flush(strip);
+                clear();
+            }
+        };
+        int v = s0;
+        for (; v + 1 < s1; v += 2) {
+            step(v, std::integral_constant<int, 0>{});
+            step(v + 1, std::integral_constant<int, 1>{});
+        }
+        if (v < s1) step(v, std::integral_constant<int, 0>{});
+        s0 = s1;
+    }
+}
+
 // Columns of X the kernels see: M rounded up to a power of two >= 16 (<= 256), beyond 256 to
 // a multiple of 256, so every launch covers a power-of-two tile of 16 NT columns.
 int padded_m(int M) {
@@ -697,21 +924,6 @@ size_t xt_bytes(const csdr_hsdb* s, int M) {
     return csdr::align_up(2 * mpad * s->C_full * sizeof(_Float16), 256);
 }
 
-// Waves per workgroup and 16-row tiles per wave for a column tile of 16 NT: more waves hide
-// more load latency and let one wave's decode run beside another's matrix-core steps; the
-// register budget (accumulators grow with NT and RT) caps them. Measured on cfg2 against two
-// row tiles per wave (16 waves to 16 columns, 8 to 64, 4 beyond): one row tile, 16 waves to
-// 64 columns and 8 beyond: M = 32 / 64 / 128 / 256 at 4096 x 11008: 47.1 -> 44.0, 58.6 ->
-// 52.2, 78.2 -> 68.7, 105.5 -> 98.6 us (M = 16 unchanged).
-constexpr int waves_for(int nt) { return nt <= 4 ? 16 : 8; }
-// (two 16-row tiles per wave from 64 columns up, so that each X operand read from LDS feeds
-// two matrix-core steps, measured slower: cfg2 M = 64 44.3 -> 56.6 us, M = 256 88.0 -> 104.8)
-constexpr int rows_for(int) { return 1; }
-// X operands from global memory (no X staging) for one 16-column tile: cfg2 4096 x 11008 at
-// M = 16 36.2 -> 33.3 us per call; at two tiles (M = 32) slower, 40.4 -> 44.0; at four the
-// prefetched operands spill
-constexpr bool x_in_regs(int nt, bool) { return nt == 1; }
-
 // The dictionary route for one 16-column tile (M <= 16); CSDR_HSDB_QROUTE=0 keeps the
 // weight-decoding kernel there.
 bool qroute_enabled() {
@@ -719,30 +931,41 @@ bool qroute_enabled() {
     return !(e && *e && std::atoi(e) == 0);
 }
 
-template <int NT, bool XS, int SLOTS>
-int launch_one(const MParams& p, int grid, size_t lds, hipStream_t st) {
-    constexpr int W = waves_for(NT), RT = rows_for(NT);
-    constexpr bool XR = x_in_regs(NT, XS);
-    const void* fn = reinterpret_cast<const void*>(&mfma_kernel<NT, XS, W, RT, SLOTS, XR>);
-    (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-    mfma_kernel<NT, XS, W, RT, SLOTS, XR><<<grid, W * 64, lds, st>>>(p);
+template <typename F>
+int launch_lds(F kern, const MParams& p, int grid, int threads, size_t lds, hipStream_t st) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    kern<<<grid, threads, lds, st>>>(p);
     CSDR_LAUNCH_CHECK("hsdb mfma");
     return CSDR_OK;
 }
 
-template <int NT, bool XS>
-int launch_slots(const MParams& p, int slots, int grid, size_t lds, hipStream_t st) {
-    switch (slots) {
-        case 4: return launch_one<NT, XS, 4>(p, grid, lds, st);
-        case 8: return launch_one<NT, XS, 8>(p, grid, lds, st);
-        default: return launch_one<NT, XS, 16>(p, grid, lds, st);
+// Rows of a strip by column tiles of the launch: each strip's partial sums are added into Y once
+// per workgroup that has units of it, as float atomics in memory, so R x M times the strips'
+// share of 256 workgroups: at 128 rows and 256 columns those were 19 us of a 61 us launch (13 of
+// 48 at 128 columns), half of that at 64 rows, where the X loads (per unit) count double. With
+// fewer columns the decode counts more, and 128 rows give each wave its own 16.
+constexpr int dec_rows(int nt) { return nt >= 8 ? 64 : 128; }
+
+template <bool XS, int SLOTS>
+int launch_main(const MParams& p, int nt, int grid, size_t lds, hipStream_t st) {
+    constexpr int kT = kDecWaves * 64;
+    switch (nt) {
+        case 16: return launch_lds(&mfma_dec_kernel<64, 1, 8, 2, XS, SLOTS>, p, grid, kT, lds, st);
+        case 8: return launch_lds(&mfma_dec_kernel<64, 2, 4, 2, XS, SLOTS>, p, grid, kT, lds, st);
+        case 4: return launch_lds(&mfma_dec_kernel<128, 8, 1, 4, XS, SLOTS>, p, grid, kT, lds, st);
+        case 2: return launch_lds(&mfma_dec_kernel<128, 8, 1, 2, XS, SLOTS>, p, grid, kT, lds, st);
+        default: return launch_lds(&mfma_kernel<XS, SLOTS>, p, grid, 1024, lds, st);
     }
 }
 
-template <int NT>
-int launch_main(const MParams& p, bool xs, int slots, int grid, size_t lds, hipStream_t st) {
-    return xs ? launch_slots<NT, true>(p, slots, grid, lds, st)
-              : launch_slots<NT, false>(p, slots, grid, lds, st);
+template <bool XS>
+int launch_slots(const MParams& p, int nt, int slots, int grid, size_t lds, hipStream_t st) {
+    switch (slots) {
+        case 4: return launch_main<XS, 4>(p, nt, grid, lds, st);
+        case 8: return launch_main<XS, 8>(p, nt, grid, lds, st);
+        default: return launch_main<XS, 16>(p, nt, grid, lds, st);
+    }
 }
 
 }  // namespace
@@ -786,7 +1009,9 @@ int mfma_matmul(int n, const csdr_hsdb* const* segs, const void* const* xs, int 
     p.tm = token_major;
     char* ws = static_cast<char*>(workspace);
     size_t off = csdr::kWsHead;
-    size_t max_elems = 0;
+    size_t max_y = 0;
+    int max_nb = 0;
+    bool any_edge = false;
     for (int i = 0; i < n; ++i) {
         const csdr_hsdb* s = segs[i];
         MDesc& d = p.m[i];
@@ -816,7 +1041,9 @@ int mfma_matmul(int n, const csdr_hsdb* const* segs, const void* const* xs, int 
             const uint32_t h = __builtin_bit_cast(uint16_t, (_Float16)rel);
             d.grel[j] = h << 16 | h;
         }
-        max_elems = std::max(max_elems, (size_t)d.R * M + (size_t)p.Mpad * d.NB * 8);
+        max_y = std::max(max_y, (size_t)d.R * M);
+        max_nb = std::max(max_nb, d.NB);
+        any_edge = any_edge || d.Ce > 0;
     }
     int dev = 0, ncu = 256, lds_max = 65536;
     if (hipGetDevice(&dev) == hipSuccess) {
@@ -830,28 +1057,22 @@ int mfma_matmul(int n, const csdr_hsdb* const* segs, const void* const* xs, int 
             lds_max = v;
     }
     {
-        const int gx = (int)std::min<size_t>(2048, (max_elems + kThreads - 1) / kThreads);
-        mfma_init_kernel<<<dim3(std::max(gx, 1), n), kThreads, 0, st>>>(p);
+        // a workgroup per block column and 64 columns of X, and some for Y
+        const size_t yper = any_edge ? kThreads : 4 * kThreads;  // edge strips: a sum per value
+        const int xwgs = max_nb * (p.Mpad / std::min(64, p.Mpad));
+        const int ywgs = (int)std::min<size_t>(1024, (max_y + yper - 1) / yper);
+        mfma_init_kernel<<<dim3(xwgs + std::max(ywgs, 1), n), kThreads, 0, st>>>(p, xwgs);
         CSDR_LAUNCH_CHECK("hsdb mfma init");
     }
     const bool xsplit = !p.x_f16;
-    const size_t dict_lds = (size_t)kMaxAtoms * 64 * sizeof(_Float16);
-    // widest power-of-two column tile whose X slice fits next to the dictionary
-    int mt = std::min(p.Mpad, kMaxMTile);
-    while (mt > 16 && dict_lds + (size_t)mt * 64 * 2 * (xsplit ? 2 : 1) > (size_t)lds_max)
-        mt /= 2;
-    const size_t lds = dict_lds + (size_t)mt * 64 * 2 * (xsplit ? 2 : 1);
+    const int mt = std::min(p.Mpad, kMaxMTile), nt = mt / 16;  // columns of a launch
+    uint32_t kmax = 0;
+    for (int i = 0; i < n; ++i) kmax = std::max(kmax, segs[i]->K);
+    const size_t lds = (size_t)kmax * 64 * sizeof(_Float16) +
+                       (nt > 1 ? (size_t)2 * dec_rows(nt) * 64 * sizeof(_Float16) : 0);
     if (lds > (size_t)lds_max)
         return set_error(CSDR_E_UNSUPPORTED, "hsdb_matmul: LDS too small for the MFMA path");
-    const int nt = mt / 16;
-    int strip_rows = 16 * 2 * waves_for(1);
-    switch (nt) {
-        case 16: strip_rows = 16 * rows_for(16) * waves_for(16); break;
-        case 8: strip_rows = 16 * rows_for(8) * waves_for(8); break;
-        case 4: strip_rows = 16 * rows_for(4) * waves_for(4); break;
-        case 2: strip_rows = 16 * rows_for(2) * waves_for(2); break;
-        default: strip_rows = 16 * rows_for(1) * waves_for(1); break;
-    }
+    const int strip_rows = nt > 1 ? dec_rows(nt) : 256;
     int units = 0;
     for (int i = 0; i < n; ++i) {
         MDesc& d = p.m[i];
@@ -878,17 +1099,9 @@ int mfma_matmul(int n, const csdr_hsdb* const* segs, const void* const* xs, int 
         return CSDR_OK;
     }
     for (int m0 = 0; m0 < p.Mpad; m0 += mt) {
-        MParams q = p;
-        q.m0 = m0;
-        int rc;
-        const int slots = (int)segs[0]->slots;
-        switch (nt) {
-            case 16: rc = launch_main<16>(q, xsplit, slots, grid, lds, st); break;
-            case 8: rc = launch_main<8>(q, xsplit, slots, grid, lds, st); break;
-            case 4: rc = launch_main<4>(q, xsplit, slots, grid, lds, st); break;
-            case 2: rc = launch_main<2>(q, xsplit, slots, grid, lds, st); break;
-            default: rc = launch_main<1>(q, xsplit, slots, grid, lds, st); break;
-        }
+        p.m0 = m0;
+        const int rc = xsplit ? launch_slots<true>(p, nt, slots0, grid, lds, st)
+                              : launch_slots<false>(p, nt, slots0, grid, lds, st);
         if (rc != CSDR_OK) return rc;
     }
     return CSDR_OK;

@@ -168,3 +168,30 @@ def test_mfma_and_p_path_agree(gpu):
     ref = oracle.hsdb_matmul(stream, x.astype(np.float32))
     assert rel_l2(y_p, ref) <= 1e-5
     assert rel_l2(y_mfma, ref) <= TOL
+
+
+# The kernel that decodes W once per workgroup, at its edges: each column tile (32, 64, 128, 256
+# columns, and a second launch past 256) with its smallest and largest M, rows around the 64- and
+# 128-row strips, fewer units than workgroups, odd atom counts, both layouts, accumulation with
+# and without a bias, and a group of two matrices whose units share a workgroup.
+@pytest.mark.parametrize("M", [17, 32, 33, 65, 128, 129, 257])
+@pytest.mark.parametrize("R,Cc,K,s,dtype", [
+    (65, 192, 77, 4, np.float16), (127, 450, 300, 8, np.float32), (257, 64, 1024, 16, np.float16),
+])
+def test_decoded_tile_edges(gpu, M, R, Cc, K, s, dtype):
+    from test_hsdb_multicol_gpu import ACCUMULATE, TOKEN_MAJOR, run_group
+
+    streams = [layer(R, Cc, K, s, 5), layer(2 * R + 1, Cc, K, s, 6)]
+    x = synth.activations(Cc, M, seed=3, dtype=dtype)
+    refs = [oracle.hsdb_matmul(st, x.astype(np.float32)) for st in streams]
+    rng = np.random.default_rng(M)
+    for flags in (0, TOKEN_MAJOR):
+        for y, ref in zip(run_group(gpu, streams, x, dtype, M, flags), refs):
+            assert rel_l2(y, ref) <= TOL
+        y0 = [rng.normal(size=r.shape).astype(np.float32) for r in refs]
+        bias = [rng.normal(size=r.shape[0]).astype(np.float32) for r in refs]
+        for b in (None, bias):
+            ys = run_group(gpu, streams, x, dtype, M, flags | ACCUMULATE, bias=b, y0=y0)
+            for i, (y, ref) in enumerate(zip(ys, refs)):
+                want = ref + y0[i] + (b[i][:, None] if b else 0)
+                assert rel_l2(y, want) <= TOL
