@@ -18,14 +18,11 @@
 //     16 blocks, and a wave keeps up to 2 steps in flight. x is staged once per workgroup in a
 //     lane-major LDS layout with the sub-block sums of x. Per group:
 //     y += d*sc*(sum q*x) - dmin*m*(sum x), the products exact and summed in fp32.
-//   q4k_mm_kernel (M > 1): 8 waves own 32 rows, up to 64 columns and a range of
-//     super-blocks (split K in at most 8 parts, each on its own XCDs). Wave w takes quant
-//     group w % 4 of every other super-block; per super-block a lane forms q * sc for 8 values
-//     of each of its two sub-blocks as exact fp16 subnormals, and v_mfma_f32_16x16x32_f16
-//     multiplies them with fp16 X (loaded straight into the A operands in the matching k
-//     order) into an fp32 tile scaled by d; the dmin * m term is a second small product with
-//     the sub-block sums of X. No rounding of W: the product is within about 1e-6 (relative
-//     L2) of fp32. The waves' tiles meet in LDS and each output is written once per split.
+//   q4k_sw_kernel and q4k_mm_kernel (M > 1): q * sc of 8 values of a sub-block as exact fp16
+//     subnormals, multiplied with fp16 X by v_mfma_f32_16x16x32_f16 into an fp32 tile scaled by d;
+//     the dmin * m term is a second product with m in every k position. No rounding of W: the
+//     product is within about 1e-6 (relative L2) of fp32. The first takes 16 rows and all of K per
+//     workgroup, the second 64 rows and a part of K (sw_pays).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -455,6 +452,26 @@ __device__ __forceinline__ half8 mm_scale(uint32_t p0, uint32_t p1, uint32_t p2,
     return __builtin_bit_cast(half8, v);
 }
 
+// 8 consecutive values of a sub-block as q * sc * 2^-24. ggml order: nibble `odd` of the 8 bytes
+// (ga, gb) of its group; interleaved: value 2i the low nibble of byte i of wi, 2i + 1 its high one
+template <int ORDER>
+__device__ __forceinline__ half8 mm_weights(uint32_t ga, uint32_t gb, uint32_t wi, int odd,
+                                            uint32_t sc2) {
+    if constexpr (ORDER == 0) {
+        const uint32_t ta = (ga >> (4 * odd)) & 0x0F0F0F0Fu, tb = (gb >> (4 * odd)) & 0x0F0F0F0Fu;
+        return mm_scale(__builtin_amdgcn_perm(ta, ta, 0x0c010c00u),
+                        __builtin_amdgcn_perm(ta, ta, 0x0c030c02u),
+                        __builtin_amdgcn_perm(tb, tb, 0x0c010c00u),
+                        __builtin_amdgcn_perm(tb, tb, 0x0c030c02u), sc2);
+    } else {
+        const uint32_t lo = wi & 0x0F0F0F0Fu, hi = (wi >> 4) & 0x0F0F0F0Fu;
+        return mm_scale(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u),
+                        __builtin_amdgcn_perm(hi, lo, 0x0c050c01u),
+                        __builtin_amdgcn_perm(hi, lo, 0x0c060c02u),
+                        __builtin_amdgcn_perm(hi, lo, 0x0c070c03u), sc2);
+    }
+}
+
 // the 4 scales and 4 mins of sub-blocks 4h .. 4h + 3 (h uniform across the wave), one per
 // byte, from the 12 scale bytes (header words y, z, w), as scale_min unpacks them one at a time
 __device__ __forceinline__ void scale_min_quad(const u32x4& hdr, int h, uint32_t& sc4,
@@ -554,24 +571,9 @@ __global__ __launch_bounds__(kMmThreads) void q4k_mm_kernel(const uint8_t* __res
             const uint32_t sel = 0x0c000c00u + 0x00010001u * (uint32_t)u;
             const uint32_t sc2 = __builtin_amdgcn_perm(sc4, sc4, sel);
             const uint32_t m2 = __builtin_amdgcn_perm(mn4, mn4, sel);
-            half8 bq;
-            if (ORDER == 0) {
-                // group 2h + u / 2, nibble u % 2 of its 8 bytes
-                const int sh = 4 * (u & 1);
-                const uint32_t ta = (w.q[2 * (u >> 1)] >> sh) & 0x0F0F0F0Fu;
-                const uint32_t tb = (w.q[2 * (u >> 1) + 1] >> sh) & 0x0F0F0F0Fu;
-                bq = mm_scale(__builtin_amdgcn_perm(ta, ta, 0x0c010c00u),
-                              __builtin_amdgcn_perm(ta, ta, 0x0c030c02u),
-                              __builtin_amdgcn_perm(tb, tb, 0x0c010c00u),
-                              __builtin_amdgcn_perm(tb, tb, 0x0c030c02u), sc2);
-            } else {
-                // value 2i: low nibble of byte i; 2i + 1: its high nibble
-                const uint32_t lo = w.q[u] & 0x0F0F0F0Fu, hi = (w.q[u] >> 4) & 0x0F0F0F0Fu;
-                bq = mm_scale(__builtin_amdgcn_perm(hi, lo, 0x0c040c00u),
-                              __builtin_amdgcn_perm(hi, lo, 0x0c050c01u),
-                              __builtin_amdgcn_perm(hi, lo, 0x0c060c02u),
-                              __builtin_amdgcn_perm(hi, lo, 0x0c070c03u), sc2);
-            }
+            // (ggml: group 2h + u / 2 of the wave's two)
+            const half8 bq =
+                mm_weights<ORDER>(w.q[2 * (u >> 1)], w.q[2 * (u >> 1) + 1], w.q[u], u & 1, sc2);
             const half8 bm = __builtin_bit_cast(half8, u32x4{m2, m2, m2, m2});
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
@@ -640,6 +642,236 @@ __global__ __launch_bounds__(kMmThreads) void q4k_mm_kernel(const uint8_t* __res
             }
         }
     }
+}
+
+// ---------------------------------------------------------------- M > 1, one pass over W
+//
+// A workgroup owns 16 rows, 16 NT columns and all of K, so nothing is added into Y, W is read
+// once and there is no launch that clears Y. Every load is made of whole runs: as the matrix
+// cores want them, consecutive lanes hold different rows or columns, and each such load costs
+// the memory pipeline a cycle or more per lane (64 rows a workgroup, both operands loaded that
+// way, spent about 2,600 of a super-block's 3,000 cycles on it). The waves have roles, because
+// a wave's loads complete in order and X (L2) would wait behind W (memory):
+//   * kSwWw waves stream W: chunks of kSwSb super-blocks of the 16 rows (576 bytes a row),
+//     kSwAhead chunks in flight in registers;
+//   * kSwXw waves copy X: a chunk's 2 KiB of each column, one chunk ahead in registers, placed in
+//     LDS as the A operands are read. Slot 16 j + c of a sub-block's tile (column c, k-slice j)
+//     is moved to 16 j + (c ^ (4 u + j) % 8), so that a column's pieces, which consecutive lanes
+//     write, meet all bank groups;
+//   * 8 waves take half a super-block of the chunk each (4 sub-blocks); the arithmetic is exact
+//     as described above.
+// Two LDS buffers, one barrier a chunk; the waves' tiles meet in LDS at the end. Per chunk at 32
+// columns: 64 KiB of X through L1 (1,024 cycles), as much written to and read from LDS (1,024),
+// vector ALU about 1,100 a SIMD; a chunk takes some 2,300,
+// as every role's reads, arithmetic and writes run one after the other between two barriers.
+constexpr int kSwRows = 16;
+constexpr int kSwSb = 4;    // super-blocks of a chunk
+constexpr int kSwWaves = 2 * kSwSb;
+constexpr int kSwXw = 4, kSwWw = 2;
+constexpr int kSwThreads = 64 * (kSwWaves + kSwXw + kSwWw);
+constexpr int kSwRowBytes = kSwSb * kBlockBytes;  // of a chunk
+constexpr int kSwPitch = kSwRowBytes + 16;  // 37 16-byte pieces: 16 rows' headers on distinct banks
+constexpr int kSwWBuf = kSwRows * kSwPitch;
+constexpr int kSwAhead = 4;
+constexpr int kSwPieces = kSwRows * (kSwRowBytes / 16);                  // of a chunk of W
+constexpr int kSwLoads = (kSwPieces + 64 * kSwWw - 1) / (64 * kSwWw);    // per lane
+template <int NT>
+constexpr int sw_xbuf() { return kSwSb * NT * 8 * 64 * 16; }
+template <int NT>
+constexpr int sw_lds_bytes() { return 2 * (sw_xbuf<NT>() + kSwWBuf); }
+
+template <int ORDER, int NT>
+__global__ __launch_bounds__(kSwThreads) void q4k_sw_kernel(const uint8_t* __restrict__ W, int R,
+                                                            int nblk, const _Float16* __restrict__ X,
+                                                            int M, float* __restrict__ Y) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char sw_smem[];
+    static_assert(sizeof(floatx4) * kSwWaves * NT * 64 <= sw_lds_bytes<NT>(), "the tiles meet there");
+    u32x4* xl = reinterpret_cast<u32x4*>(sw_smem);          // [2][super-block][NT][8 u][64 slots]
+    unsigned char* wl = sw_smem + 2 * sw_xbuf<NT>();        // [2][16 rows][pitch]
+    constexpr int kXBuf = sw_xbuf<NT>() / 16;               // u32x4 per X buffer
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int r0 = blockIdx.x * kSwRows, n0 = blockIdx.y * 16 * NT;
+    const int nch = (nblk + kSwSb - 1) / kSwSb;
+    const int rl = lane & 15, j = lane >> 4;
+    floatx4 acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) acc[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    // Every role fills chunk 0 before the loop; in iteration k, between its barrier and the next,
+    // the producers fill chunk k + 1 (its buffer was last read in iteration k - 1).
+    if (wave >= kSwWaves + kSwXw) {
+        // ---- W: piece i of a chunk is 16 bytes of row i / 36
+        const int pt = (wave - kSwWaves - kSwXw) * 64 + lane;
+        const size_t rowb = (size_t)nblk * kBlockBytes;
+        const uint8_t* src[kSwLoads];
+        int dst[kSwLoads], at[kSwLoads];
+#pragma unroll
+        for (int q = 0; q < kSwLoads; ++q) {
+            const int i = min(pt + q * 64 * kSwWw, kSwPieces - 1);
+            const int row = i / (kSwRowBytes / 16);
+            at[q] = (i - row * (kSwRowBytes / 16)) * 16;
+            src[q] = W + (size_t)min(r0 + row, R - 1) * rowb;
+            dst[q] = row * kSwPitch + at[q];
+        }
+        u32x4 ring[kSwAhead][kSwLoads];
+        const long long last = (long long)rowb - 16;  // past a row's end: its last piece again
+        auto load = [&](int k, u32x4 (&v)[kSwLoads]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < kSwLoads; ++q)
+                v[q] = *reinterpret_cast<const u32x4*>(
+                    src[q] + min((long long)k * kSwRowBytes + at[q], last));
+        };
+        auto store = [&](int k, const u32x4 (&v)[kSwLoads]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int q = 0; q < kSwLoads; ++q)
+                *reinterpret_cast<u32x4*>(wl + (k & 1) * kSwWBuf + dst[q]) = v[q];
+        };
+#pragma unroll
+        for (int s = 0; s < kSwAhead; ++s) load(s, ring[s]);
+        store(0, ring[0]);
+        load(kSwAhead, ring[0]);
+        for (int k0 = 0; k0 < nch; k0 += kSwAhead) {
+#pragma unroll
+            for (int s = 0; s < kSwAhead; ++s) {
+                const int k = k0 + s;
+                if (k >= nch) break;
+                __syncthreads();
+                store(k + 1, ring[(s + 1) % kSwAhead]);
+                load(k + 1 + kSwAhead, ring[(s + 1) % kSwAhead]);
+            }
+        }
+    } else if (wave >= kSwWaves) {
+        // ---- X: lane t takes piece t % 128 (16 bytes) of the chunk of columns t / 128, + 2, ...
+        constexpr int kCols = 16 * NT / 2;  // columns per lane
+        const int t = (wave - kSwWaves) * 64 + lane, c0 = t >> 7, pc = t & 127;
+        const int sb = pc >> 5, u = (pc >> 2) & 7, pj = pc & 3;
+        const size_t C = (size_t)nblk * 256;
+        const int sw = (4 * u + pj) & 7;
+        u32x4 v[kCols];
+        auto load1 = [&](const _Float16* src, int e) __attribute__((always_inline)) {
+            v[e] = *reinterpret_cast<const u32x4*>(src + (size_t)min(n0 + c0 + 2 * e, M - 1) * C);
+        };
+        auto source = [&](int k) __attribute__((always_inline)) {
+            return X + (size_t)min(k * kSwSb + sb, nblk - 1) * 256 + (pc & 31) * 8;
+        };
+        // piece by piece into the chunk's buffer, each register's next load right behind: the
+        // copy then runs at the rate of its loads, not at their latency a chunk
+        auto pass = [&](int k) __attribute__((always_inline)) {
+            const _Float16* src = source(k + 1);
+#pragma unroll
+            for (int e = 0; e < kCols; ++e) {
+                const int c = c0 + 2 * e;
+                xl[(k & 1) * kXBuf + ((sb * NT + (c >> 4)) * 8 + u) * 64 + 16 * pj +
+                   ((c & 15) ^ sw)] = v[e];
+                load1(src, e);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        };
+        {
+            const _Float16* src = source(0);
+#pragma unroll
+            for (int e = 0; e < kCols; ++e) load1(src, e);
+        }
+        pass(0);
+        for (int k = 0; k < nch; ++k) {
+            __syncthreads();
+            pass(k + 1);
+        }
+    } else {
+        const int sb = wave >> 1, half = wave & 1;
+        for (int k = 0; k < nch; ++k) {
+            __syncthreads();
+            const unsigned char* wb = wl + (k & 1) * kSwWBuf + rl * kSwPitch + sb * kBlockBytes;
+            const u32x4* xb = xl + (k & 1) * kXBuf + (sb * NT * 8 + 4 * half) * 64 + 16 * j;
+            const u32x4 hdr = *reinterpret_cast<const u32x4*>(wb);
+            uint32_t w[4];
+            if (ORDER == 0) {
+                // groups 2h, 2h + 1: bytes 8j .. 8j + 7 (low nibbles: sub-block 2g, high: 2g + 1)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) {
+                    const uint2 v =
+                        *reinterpret_cast<const uint2*>(wb + 16 + 32 * (2 * half + g) + 8 * j);
+                    w[2 * g] = v.x;
+                    w[2 * g + 1] = v.y;
+                }
+            } else {
+                // sub-blocks 4h .. 4h + 3: bytes 4j .. 4j + 3 (two values per byte)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    w[u] = *reinterpret_cast<const uint32_t*>(wb + 16 + 16 * (4 * half + u) + 4 * j);
+            }
+            u32x4 x[4][NT];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+                    x[u][nt] = xb[(nt * 8 + u) * 64 + (rl ^ ((4 * u + j) & 7))];
+            floatx4 D[NT], Dm[NT];
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                D[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+                Dm[nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+            }
+            uint32_t sc4, mn4;
+            scale_min_quad(hdr, half, sc4, mn4);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const uint32_t sel = 0x0c000c00u + 0x00010001u * (uint32_t)u;
+                const uint32_t sc2 = __builtin_amdgcn_perm(sc4, sc4, sel);
+                const uint32_t m2 = __builtin_amdgcn_perm(mn4, mn4, sel);
+                const half8 bq =
+                    mm_weights<ORDER>(w[2 * (u >> 1)], w[2 * (u >> 1) + 1], w[u], u & 1, sc2);
+                const half8 bm = __builtin_bit_cast(half8, u32x4{m2, m2, m2, m2});
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    const half8 a = __builtin_bit_cast(half8, x[u][nt]);
+                    D[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bq, D[nt], 0, 0, 0);
+                    Dm[nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bm, Dm[nt], 0, 0, 0);
+                }
+            }
+            if (k * kSwSb + sb < nblk) {
+                const float d24 = hdr_d(hdr) * 16777216.0f, dm24 = hdr_dmin(hdr) * 16777216.0f;
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) acc[nt][i] += d24 * D[nt][i] - dm24 * Dm[nt][i];
+            }
+        }
+    }
+    __syncthreads();
+    floatx4* red = reinterpret_cast<floatx4*>(sw_smem);  // [wave][NT][64 lanes]
+    if (wave < kSwWaves) {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) red[(wave * NT + nt) * 64 + lane] = acc[nt];
+    }
+    __syncthreads();
+    // output o of the tile: row o % 16, column o / 16 (lane rl + 16 (col / 4) holds column % 4 of it)
+    const float* rf = reinterpret_cast<const float*>(sw_smem);
+    for (int o = threadIdx.x; o < 256 * NT; o += kSwThreads) {
+        const int row = o & 15, col = o >> 4, nt = col >> 4, c = col & 15;
+        float sum = 0.f;
+#pragma unroll
+        for (int v = 0; v < kSwWaves; ++v)
+            sum += rf[((v * NT + nt) * 64 + (c >> 2) * 16 + row) * 4 + (c & 3)];
+        if (r0 + row < R && n0 + col < M) Y[(size_t)(n0 + col) * R + r0 + row] = sum;
+    }
+}
+
+// Which of the two M > 1 kernels. Up to 16 columns q4k_sw_kernel (us, q4k_mm_kernel with its
+// clearing launch first: 4096 x 14336 21.2 / 15.9, 4096^2 10.7 / 6.7, 14336 x 4096 24.5 / 21.5,
+// 300 x 14336 12.8 / 11.2, 896 x 1024 6.1 / 3.8). Past that its copy of X per 16 rows grows with
+// the columns, so it takes up to 64 of them while that is at most 14 chunks' time (rounds of
+// 256 workgroups x chunks of K: 4096 x 14336 M = 32 25.9 / 23.3, 4096^2 13.0 / 8.7 and at 64
+// 18.5 / 15.9, 1000 x 1024 at 64 9.8 / 5.0, but 14336 x 4096 M = 20 26 / 28, 4096 x 14336 M = 64
+// 36 / 42), except a long K with too few row tiles for the chip at 17 to 32 columns, where
+// q4k_mm_kernel splits K over the CUs (1024 x 14336 M = 32 15.6 / 17.1).
+bool sw_pays(int R, int nblk, int M) {
+    if (M <= 16) return true;
+    if (M > 64) return false;
+    const long long wgs = (long long)((R + kSwRows - 1) / kSwRows) * (M <= 32 ? 1 : 2);
+    const long long nch = (nblk + kSwSb - 1) / kSwSb;
+    if (M <= 32 && wgs < 128 && nch > 8) return false;
+    return (wgs + 255) / 256 * nch <= 14;
 }
 
 // ---------------------------------------------------------------- dequant to fp32
@@ -736,6 +968,25 @@ CSDR_API int csdr_q4k_linear(const void* w, int R, int C, int order, const void*
             return set_error(CSDR_E_UNSUPPORTED, "q4k_linear: M > 1 takes fp16 x");
         if (reinterpret_cast<uintptr_t>(x) % 16 || C % 8)
             return set_error(CSDR_E_INVALID, "q4k_linear: x must be 16-byte aligned");
+        if (sw_pays(R, nblk, M)) {
+            const auto* wq = static_cast<const uint8_t*>(w);
+            const auto* xq = static_cast<const _Float16*>(x);
+            const int nt = M <= 16 ? 1 : 2;
+            const dim3 grid((unsigned)((R + kSwRows - 1) / kSwRows),
+                            (unsigned)((M + 16 * nt - 1) / (16 * nt)));
+            auto go = [&](auto kern) {
+                const int lds = nt == 1 ? sw_lds_bytes<1>() : sw_lds_bytes<2>();
+                (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                          hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+                kern<<<grid, kSwThreads, lds, st>>>(wq, R, nblk, xq, M, y);
+            };
+            if (order == CSDR_Q4K_GGML)
+                nt == 1 ? go(&q4k_sw_kernel<0, 1>) : go(&q4k_sw_kernel<0, 2>);
+            else
+                nt == 1 ? go(&q4k_sw_kernel<1, 1>) : go(&q4k_sw_kernel<1, 2>);
+            CSDR_LAUNCH_CHECK("q4k_linear");
+            return CSDR_OK;
+        }
         // 64-row tiles of up to 64 columns; the super-blocks split in S parts (S a power of
         // two up to 8) so that the grid holds at least 256 workgroups where the row tiles
         // alone do not

@@ -67,6 +67,24 @@ def test_linear(gpu, R, C, M, order, xdt):
     assert err <= 1e-5
 
 
+# The one-pass kernel at its edges: fewer super-blocks than a chunk, a partial last chunk, more
+# chunks than are in flight, rows and columns off the 16s, both column tiles and two groups of
+# them; and the shapes on either side of the rule that chooses it (same bar as above: exact
+# products, fp32 sums).
+@pytest.mark.parametrize("order", ["ggml", "interleaved"])
+@pytest.mark.parametrize("R,nblk,M", [(16, 1, 2), (17, 2, 16), (33, 4, 17), (50, 5, 15),
+                                      (15, 9, 31), (130, 23, 9), (100, 13, 32), (48, 33, 33),
+                                      (2050, 36, 20), (65, 3, 64), (40, 57, 20), (40, 57, 64)])
+def test_linear_one_pass(gpu, R, nblk, M, order):
+    from cortexsdr_amd import q4k
+
+    blob = weights(R, 256 * nblk, order)
+    x = synth.activations(256 * nblk, M, seed=11).T.copy().astype(np.float16)
+    y = q4k.linear(q4k.upload(blob), R, 256 * nblk, gpu.from_numpy(x).cuda(), ORDERS[order])
+    ref = oracle.q4k_linear(blob, R, 256 * nblk, x.astype(np.float32), ORDERS[order])
+    assert rel_l2(y.cpu().numpy(), ref) <= 1e-5
+
+
 def test_kat_blocks_through_gpu(gpu):
     # the reference's known-answer block (test_hsdr_kquants.cpp:106-122) through the GPU
     # dequant in the interleaved order: 26, -4
