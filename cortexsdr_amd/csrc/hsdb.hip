@@ -1545,8 +1545,9 @@ __global__ __launch_bounds__(kThreads) void gatherg_kernel(Params p) {
     csdr::chunk_span((uint32_t)c, (uint32_t)d.NB, (uint32_t)d.NBc, b0u, nbcu);
     const int b0 = (int)b0u, nbc = (int)nbcu;
     const int r0 = sidx * d.Rt, rend = min(r0 + d.Rt, d.R);
-    float* Ps = smem;                           // nbc * K * MC
-    float* gs = smem + (size_t)d.NBc * d.K * MC;  // slot gains
+    float* Ps = smem;                                 // nbc * K * MC
+    const int zero = d.NBc * d.K * MC;                // MC zeros behind it
+    float* gs = Ps + zero + MC;                       // slot gains
     const bool gl = d.slots <= kGgGammaLds;
     const int sg = tid & 3, mg = TPR == 8 ? (tid >> 2 & 1) : 0;
     const int W = nbc * d.slots;  // words of a row
@@ -1579,29 +1580,35 @@ __global__ __launch_bounds__(kThreads) void gatherg_kernel(Params p) {
                 for (int j = 0; j < kStageBatch; ++j) Ps[min(i0 + j * kThreads + tid, np - 1)] = v[j];
             }
         }
+        if (tid < MC) Ps[zero + tid] = 0.0f;
         if (gl)
             for (int i = tid; i < d.slots; i += kThreads) gs[i] = d.slot_gamma[i];
     }
     __syncthreads();
     const bool last_chunk = (c == d.nchunks - 1);
-    // gain (0 past the last word) and P offset of each of the lane's words from q0 on
+    // gain and P offset of each of the lane's words from q0 on; past the last word a zero word
+    // on the zeros (an infinite P or coefficient of the repeated word would make 0 * inf of it)
     float gm[kGgWords];
     int po[kGgWords];
+    uint32_t keep[kGgWords];
     auto place = [&](int q0) {
 #pragma unroll
         for (int j = 0; j < kGgWords; ++j) {
             const int q = min(q0 + 4 * j + sg, W - 1);
             const int bb = nbc == 1 ? 0 : q / d.slots, sl = q - bb * d.slots;
-            gm[j] = q0 + 4 * j + sg >= W ? 0.0f : gl ? gs[sl] : d.slot_gamma[sl];
-            po[j] = bb * d.K * MC + 4 * mg;
+            const bool in = q0 + 4 * j + sg < W;
+            gm[j] = !in ? 0.0f : gl ? gs[sl] : d.slot_gamma[sl];
+            po[j] = (in ? bb * d.K * MC : zero) + 4 * mg;
+            keep[j] = in ? 0xFFFFFFFFu : 0u;
         }
     };
     float acc[CPT];
     auto add = [&](const uint32_t (&w)[kGgWords]) {
 #pragma unroll
         for (int j = 0; j < kGgWords; ++j) {
-            const float cf = gm[j] * csdr::h2f(w[j] >> 16);
-            const float* pv = Ps + po[j] + (w[j] & 0x7FFFu) * MC;
+            const uint32_t wd = w[j] & keep[j];
+            const float cf = gm[j] * csdr::h2f(wd >> 16);
+            const float* pv = Ps + po[j] + (wd & 0x7FFFu) * MC;
             if constexpr (CPT == 4) {
                 const float4 v = *reinterpret_cast<const float4*>(pv);
                 acc[0] = fmaf(cf, v.x, acc[0]);
@@ -2417,7 +2424,7 @@ int matmul_group(int n, const csdr_hsdb* const* segs, const void* const* xs, int
             d.Rt = rows * passes;
             d.splits = (d.R + d.Rt - 1) / d.Rt;
             lds_g = std::max(lds_g, (size_t)d.NBc * d.K * gmc * 4 +
-                                        (size_t)std::min(d.slots, kGgGammaLds) * 4);
+                                        (size_t)(gmc + std::min(d.slots, kGgGammaLds)) * 4);
             d.g_base = base;
             d.g_count = d.nchunks * d.splits;
             base += d.g_count;

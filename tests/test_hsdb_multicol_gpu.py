@@ -182,3 +182,24 @@ def test_any_block_length_and_slots(gpu, B, slots, M, flags, dtype):
     ys = run_group(gpu, streams, x, dtype, M, flags | ACCUMULATE, bias=bias, y0=y0)
     for y, w, b, a in zip(ys, want, bias, y0):
         assert rel_l2(y, a + w + b[:, None]) <= (1e-3 if B == 64 and M > 8 else 1e-5)
+
+
+# An infinite x makes P infinite for every atom: with positive atoms and coefficients all of Y is
+# +inf, and a lane's slots past the row's last word (24 of a round of 32) add nothing to it.
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 9])
+@pytest.mark.parametrize("B,slots", [(130, 24), (48, 5), (130, 40)])
+def test_any_slots_infinite_input(gpu, B, slots, M):
+    from cortexsdr_amd import formats
+
+    rng = np.random.default_rng(B + slots)
+    K, R, nb = 75, 37, 2
+    D = np.abs(synth.dictionary(K, B, 11)) + np.float32(0.01)
+    idx = rng.integers(0, K, (R * nb, slots))
+    coef = rng.uniform(0.5, 1.0, (R * nb, slots))
+    stream = formats.pack_hsdb(R, nb * B, D, idx, coef, gamma=(1.0,))
+    x = np.abs(synth.activations(nb * B, M, seed=5, dtype=np.float32))
+    want = oracle.hsdb_matmul(stream, x)
+    x[[3, B + 4], M - 1] = np.inf
+    (y,) = run_group(gpu, [stream], x, np.float32, M)
+    assert (y[:, M - 1] == np.inf).all()
+    assert M == 1 or rel_l2(y[:, :-1], want[:, :-1]) <= 1e-5
