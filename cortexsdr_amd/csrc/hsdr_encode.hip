@@ -623,9 +623,17 @@ size_t gram_ws_bytes(long long n, int K) {
            ((size_t)K + chunk + 1) * 4;
 }
 
-// The Gram path does 2 (n + K) K C operations where mp_kernel does 2 n picks K C.
+// mp_gram_kernel's LDS: the residual, the picks with their gains, the atoms left.
+size_t gram_lds_bytes(int C, int S, int k) {
+    const size_t slots = (size_t)S * k;
+    return ((size_t)C + slots) * 4 + (((slots + 1) & ~(size_t)1) + kGramMaxCand) * 2;
+}
+
+// The Gram path does 2 (n + K) K C operations where mp_kernel does 2 n picks K C. It keeps every
+// pick in LDS, mp_kernel none: more of them than fit in 64 KiB stay with that.
 bool gram_pays(long long n, int C, int K, int S, int k) {
     return K <= kGramMaxK && C <= kGramMaxC && 2 * n * S * k >= n + K &&
+           gram_lds_bytes(C, S, k) <= 64 * 1024 &&
            !std::getenv("CSDR_HSDR_TILES_PER_WG");  // that override names mp_kernel's form
 }
 
@@ -668,7 +676,7 @@ int launch_mp_gram(const float* tiles, long long n, int C, const float* D, int K
     b.count = count;
     b.list = count + 1;
     for (int l = 0; l < S; ++l) a.gamma[l] = b.gamma[l] = gamma[l];
-    const size_t lds = (size_t)(C + S * k) * 4 + (size_t)(((S * k + 1) & ~1) + kGramMaxCand) * 2;
+    const size_t lds = gram_lds_bytes(C, S, k);
     const size_t list_lds = mp_lds_bytes(1, C, K);
     for (long long t0 = 0; t0 < n; t0 += chunk) {
         const long long nt = std::min(chunk, n - t0);

@@ -108,6 +108,16 @@ def test_encode_ties_and_odd_tiles_match_oracle(gpu, monkeypatch, n, C, K, S, k)
     assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), oracle.hsdr_mp(t, D, g, S, k))
 
 
+def test_encode_more_picks_than_the_gram_form_holds(gpu, monkeypatch):
+    # 32 x 345 picks and their gains are past 64 KiB of LDS: mp_kernel, which keeps none
+    monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
+    rng = np.random.default_rng(32)
+    t = (rng.standard_normal((4, 8)) * 0.02).astype(np.float32)
+    D = (rng.standard_normal((512, 8)) * 0.01).astype(np.float32)
+    g = (0.5 ** np.arange(32)).astype(np.float32)
+    assert np.array_equal(gpu_codes(gpu, t, D, g, 32, 345), oracle.hsdr_mp(t, D, g, 32, 345))
+
+
 def test_encode_large_tile_falls_back_to_one_per_workgroup(gpu, monkeypatch):
     # 2 x (C + K) x 4 bytes > 64 KiB: the natural choice is one tile per workgroup
     monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
