@@ -828,8 +828,14 @@ __global__ __launch_bounds__(kDecWaves * 64) void mfma_dec_kernel(MParams p) {
         auto step = [&](int v, auto S) __attribute__((always_inline)) {
             constexpr int sl = decltype(S)::value;  // ring slot and target buffer of unit v + 1
             // unit v's tile is whole, unit v - 1's has been read (with one column group a wave
-            // multiplies the rows that it decoded: nothing to wait for)
-            if constexpr (CG > 1) __syncthreads();
+            // multiplies the rows that it decoded: its own LDS order does, which the fence, no
+            // instruction, keeps the compiler to)
+            if constexpr (CG > 1) {
+                __syncthreads();
+            } else {
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
             u32x4 xb[CT][NP][2];
             const _Float16* xs = xt0 + (size_t)cg.b * xblk;
 #pragma unroll
