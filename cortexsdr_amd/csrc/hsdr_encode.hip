@@ -848,41 +848,70 @@ __global__ __launch_bounds__(kEThreads) void users_scan_kernel(FitArgs a) {
     }
 }
 
+// Bound by the codes' way from L2: 64 of them (a 128-byte line) are in flight per thread and the
+// first walk keeps its finds in LDS, so that the second one is needed only by a thread with more
+// than kFillHits of them (4864 x 896, 24 slots, K = 512: 66 us with one 16-byte load in flight and
+// two walks, 31 here; eight reads at a time for the sum of gamma^2 changed
+// nothing).
+constexpr int kFillHits = 8;
+
 __global__ __launch_bounds__(kEThreads) void users_fill_kernel(FitArgs a) {
     __shared__ double gm_s[kEThreads];
+    __shared__ uint32_t hit_s[kFillHits][kEThreads];  // 2 x position in the run + sign
     const int j = blockIdx.x, tid = threadIdx.x;
     const int u0 = a.off[j], u1 = a.off[j + 1];
     const int slots = a.S * a.k;
-    const uint16_t want = (uint16_t)j;
+    const uint32_t want = (uint32_t)j;
     // runs of a multiple of 8 codes, read 16 bytes at a time (codes is 16-byte aligned)
     const long long run = (a.ncodes + (long long)kEThreads * 8 - 1) / (kEThreads * 8) * 8;
-    const long long i0 = min(tid * run, a.ncodes), i1 = min(i0 + run, a.ncodes);
+    const long long i0 = min(tid * run, a.ncodes);
+    const int len = (int)(min(i0 + run, a.ncodes) - i0);
+    const uint16_t* cd = a.codes + i0;
     auto walk = [&](auto&& use) {
-        long long i = i0;
-        for (; i + 8 <= i1; i += 8) {
-            const uint4 w = *reinterpret_cast<const uint4*>(a.codes + i);
-            const uint32_t ws[4] = {w.x, w.y, w.z, w.w};
+        const int len8 = len & ~7;
+        for (int i = 0; i < len8; i += 64) {  // pieces past the last one: that one, not looked at
+            uint4 w[8];
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                if ((ws[q] & 0x7FFF) == want) use(i + 2 * q, (uint16_t)ws[q]);
-                if ((ws[q] >> 16 & 0x7FFF) == want) use(i + 2 * q + 1, (uint16_t)(ws[q] >> 16));
+            for (int q = 0; q < 8; ++q)
+                w[q] = *reinterpret_cast<const uint4*>(cd + min(i + 8 * q, len8 - 8));
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                uint32_t found = 0;
+#pragma unroll
+                for (int q = 0; q < 16; ++q) {
+                    const uint4& v = w[4 * h + q / 4];
+                    const uint32_t x = q % 4 == 0 ? v.x : q % 4 == 1 ? v.y : q % 4 == 2 ? v.z : v.w;
+                    found |= (x & 0x7FFF) == want ? 1u << (2 * q) : 0u;
+                    found |= (x >> 16 & 0x7FFF) == want ? 2u << (2 * q) : 0u;
+                }
+                const int left = len8 - i - 32 * h;
+                if (left < 32) found &= left > 0 ? (1u << left) - 1 : 0u;
+                for (; found; found &= found - 1) use(i + 32 * h + __ffs(found) - 1);
             }
         }
-        for (; i < i1; ++i)
-            if ((a.codes[i] & 0x7FFF) == want) use(i, a.codes[i]);
+        for (int i = len8; i < len; ++i)
+            if ((cd[i] & 0x7FFFu) == want) use(i);
     };
     int mine = 0;
-    if (u1 > u0) walk([&](long long, uint16_t) { ++mine; });
+    if (u1 > u0)
+        walk([&](int i) {
+            if (mine < kFillHits) hit_s[mine][tid] = 2u * i + (cd[i] >> 15);
+            ++mine;
+        });
     int total;
     int p = u0 + block_scan(mine, &total);
-    if (mine)
-        walk([&](long long i, uint16_t v) {
-            const long long tile = i / slots;
-            const double gm = (double)a.gamma[(int)(i - tile * slots) / a.k];
-            a.utile[p] = (uint32_t)tile;
-            a.ucoef[p] = (v & 0x8000) ? -gm : gm;
-            ++p;
-        });
+    auto put_user = [&](int i, bool neg) {
+        const long long tile = (i0 + i) / slots;
+        const double gm = (double)a.gamma[(int)(i0 + i - tile * slots) / a.k];
+        a.utile[p] = (uint32_t)tile;
+        a.ucoef[p] = neg ? -gm : gm;
+        ++p;
+    };
+    if (mine <= kFillHits) {
+        for (int q = 0; q < mine; ++q) put_user(hit_s[q][tid] >> 1, hit_s[q][tid] & 1);
+    } else {
+        walk([&](int i) { put_user(i, cd[i] >> 15); });
+    }
     __syncthreads();
     double w = 0.0;  // thread 0
     for (int b = u0; b < u1; b += kEThreads) {

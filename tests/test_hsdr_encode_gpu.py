@@ -176,6 +176,35 @@ def test_compress_refined_matches_reference(gpu, enc):
         assert np.array_equal(gpu_codes(gpu, t, rD, rg, S, k), rcodes), f"case {i}"
 
 
+# One refinement pass from the initial dictionary and codes, against its sums in numpy. The
+# device's residuals hold sqrt(S k) 2^-24 of a tile's norm in fp32 roundings, an atom's share of
+# which its users' mean takes to under 2e-6 of its length. Users of few atoms, more than a thread keeps from
+# one walk over the codes; code counts off the 8-code pieces; runs past one round of 64 codes.
+@pytest.mark.parametrize("n,C,K,S,k", [(1003, 24, 3, 2, 3), (3001, 40, 40, 2, 5),
+                                       (2800, 16, 64, 3, 8), (61, 24, 5, 1, 5)])
+def test_one_refinement_pass(gpu, n, C, K, S, k):
+    from cortexsdr_amd import encode
+
+    w = (np.random.default_rng(n).standard_normal((n, C)) * 0.02).astype(np.float32)
+    _, D0, g, c0 = stream_parts(encode.compress(w, 1, C, K, S, k, ksvd_iters=0))
+    _, D1, _, c1 = stream_parts(encode.compress(w, 1, C, K, S, k, ksvd_iters=1))
+    c0 = c0.reshape(n, S * k)
+    idx, coef = c0 & 0x7FFF, np.where(c0 & 0x8000, -1.0, 1.0) * np.repeat(g, k)
+    assert len(np.unique(idx)) == K  # no atom is re-seeded
+    res = w.astype(np.float64)
+    for j in range(S * k):
+        res -= coef[:, j:j + 1] * D0[idx[:, j]].astype(np.float64)
+    target = np.linalg.norm(w.astype(np.float64), axis=1).mean() / np.sqrt(S * k)
+    for a in range(K):
+        tile, slot = np.nonzero(idx == a)
+        cf = coef[tile, slot]
+        new = D0[a] + 0.5 * (cf[:, None] * res[tile]).sum(0) / (cf * cf).sum()
+        if np.linalg.norm(new) > 1.5 * target:
+            new *= target / np.linalg.norm(new)
+        assert np.linalg.norm(D1[a] - new) <= 2e-6 * np.linalg.norm(new), f"atom {a}"
+    assert np.array_equal(c1.reshape(n, -1), oracle.hsdr_mp(w, D1, g, S, k).reshape(n, -1))
+
+
 def test_compress_rejects(gpu):
     from cortexsdr_amd import _lib, encode
 
