@@ -172,6 +172,8 @@ struct csdr_decoder {
     float *pf_a = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_w = nullptr;
     float* pf_s = nullptr;          // the split form's token planes, row scales and partial sums
     int* pf_tok = nullptr;
+    bool pf_eligible = false;       // the blocks took the split form when the buffers were made
+    bool pf_split = false;          // the buffers hold it
     // on-demand layer streaming (blocks of host-resident segments)
     bool prefetch = true;           // copy block j + 2 while block j + 1 runs (else j + 1 after j)
     bool stage_ready = false;       // staging buffers, views, copy stream and events built
@@ -415,6 +417,7 @@ void free_prefill(csdr_decoder* d) {
         d->pf_s = nullptr;
     d->pf_tok = nullptr;
     d->pf_rows = 0;
+    d->pf_split = false;
 }
 
 constexpr int kMinSplitRows = 8;  // fewer: a row of W per wave (csdr_dense_linear_ex)
@@ -443,14 +446,17 @@ size_t split_x_floats(const csdr_decoder_config& c, int rows) {
     return (size_t)rows * (widest + 1) + 16 + split_part_rows(c, rows) * c.hidden;
 }
 
-// Buffers of a prefill pass over `rows` token rows (kept for later passes of up to as many).
+// Buffers of a prefill pass over `rows` token rows, kept for later passes of up to as many while
+// the blocks take the same form (csdr_decoder_set_layer may replace one by a block that does not,
+// or the last that did not by one that does); passes read the form from pf_split.
 int ensure_prefill(csdr_decoder* d, int rows) {
-    if (rows <= d->pf_rows) return CSDR_OK;
+    const bool eligible = prefill_split(d);
+    if (rows <= d->pf_rows && eligible == d->pf_eligible) return CSDR_OK;
     free_prefill(d);
     const csdr_decoder_config& c = d->cfg;
     const size_t n = (size_t)rows, H = c.hidden, F = c.ffn;
     const size_t kvw = (size_t)c.n_kv_heads * c.head_dim;
-    const bool split = prefill_split(d);
+    const bool split = eligible && rows >= kMinSplitRows;
     const size_t wmax =
         std::max({H * H, kvw * H, F * H, split ? split_w_floats(c) : (size_t)0});
     const std::pair<float**, size_t> bufs[] = {
@@ -474,6 +480,8 @@ int ensure_prefill(csdr_decoder* d, int rows) {
     }
     d->pf_tok = static_cast<int*>(p);
     d->pf_rows = rows;
+    d->pf_eligible = eligible;
+    d->pf_split = split;
     return CSDR_OK;
 }
 
@@ -579,7 +587,7 @@ int prefill_pass(csdr_decoder* d, int p0, int T, hipStream_t st) {
     CSDR_LAUNCH_CHECK("decoder pass tokens");
     RC(csdr_hsdb_decode_rows(d->emb, d->pf_tok, M, d->pf_x, st));
     RC(stream_begin(d, st));
-    if (M >= kMinSplitRows && prefill_split(d)) {
+    if (M >= kMinSplitRows && d->pf_split) {
         RC(prefill_layers_split(d, p0, T, st));
         return stream_end(d, st);
     }

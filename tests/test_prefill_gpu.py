@@ -229,6 +229,60 @@ def test_prefill_product_edges(gpu, layers, heads, ffn, nnz, n_prompt):
     _compare(runs, 3, 1e-4)
 
 
+def test_prefill_after_a_layer_changes_form(gpu, monkeypatch):
+    """The pass's buffers are sized for the form that the blocks take (the split planes need
+    64-long coded blocks everywhere): replacing the one block of another width by a 64-long one,
+    and back, between prefills of the same length gives the scores of decoders built that way.
+    (The fused step refuses such blocks; the one-launch-per-op step takes them.) Within 1e-4, as
+    the other forms of the passes."""
+    from cortexsdr_amd import synth
+    from cortexsdr_amd.decoder import LINEARS, Decoder, DecoderSpec, DecoderWeights
+    from cortexsdr_amd.decoder import _fptr, synthetic_weights
+    from cortexsdr_amd.hsdr import HsdbSegment
+
+    monkeypatch.setenv("CSDR_DECODER_FUSED", "0")
+    L, lib = _lib()
+    spec = DecoderSpec(2, 256, 4, 2, 64, 320, 300, 64, kv_dtype="f16")
+    w64 = synthetic_weights(spec, n_atoms=128, nnz=8, seed=17, sigma=0.1)
+    narrow = dict(w64.layers[0])
+    for i, (name, (R, Cc)) in enumerate(spec.shapes().items()):
+        narrow[name] = synth.hsdb_layer(R, Cc, 64, 4, seed_dict=5, seed_codes=30 + i, sigma=0.1,
+                                        B=32)
+    w32 = DecoderWeights(spec, [narrow, w64.layers[1]], w64.lm_head, w64.final_norm)
+    prompt = ((np.arange(40) * 7919 + 11) % spec.vocab).astype(np.int32)
+
+    def scores(dec):
+        dec.prefill(prompt, 0.0, 0.0)
+        return dec.logits()
+
+    def set_first(dec, layer):
+        segs = [HsdbSegment(layer[n]) for n in LINEARS]
+        vecs = [layer["attn_norm"], layer["ffn_norm"], None, None, None]
+        L.check(lib.csdr_decoder_set_layer(dec._h, 0, *[s._h for s in segs],
+                                           *[_fptr(v) for v in vecs]))
+        return segs
+
+    want = {}
+    for n, w in (("64", w64), ("32", w32)):
+        dec = Decoder(w)
+        want[n] = scores(dec)
+        dec.close()
+    assert rel_l2(want["32"], want["64"]) > 1e-2  # two models
+    dec = Decoder(w32)
+    keep = []
+    try:
+        assert rel_l2(scores(dec), want["32"]) < 1e-4
+        keep.append(set_first(dec, w64.layers[0]))
+        assert rel_l2(scores(dec), want["64"]) < 1e-4
+        keep.append(set_first(dec, narrow))
+        assert rel_l2(scores(dec), want["32"]) < 1e-4
+    finally:
+        dec.close()
+        for segs in keep:
+            for sg in segs:
+                sg.free()
+
+
 def test_cfg4_full_model_long_prompt(gpu):
     """configs[3] at full size with a 160-token prompt: one multi-token pass (and passes of 64)
     against the token-at-a-time prefill."""
