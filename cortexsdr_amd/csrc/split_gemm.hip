@@ -2,14 +2,17 @@
 // decoder's batched prefill: W decoded from its codes once per pass, X the prompt's rows.
 //
 // The fp32 matrix-core rate (157 TFLOP/s dense) bounds the fp32 product (gemm_f32.hip), a
-// sixteenth of the fp16 one. Here each value is hi + lo, two fp16 numbers after scaling its row
-// by a power of two that puts the row's largest magnitude in [2^14, 2^15): hi has 11 bits, lo
-// the next 11 (or all down to 2^-24, 2^-39 of the row's largest), so hi + lo is the value to
-// about 2^-23, and
-//   x . w = hi hi + (hi lo + lo hi) + lo lo
-// with the last term (2^-22 of the first) left out: three 16x16x32 products, exact in fp32 and
-// summed in fp32, the cross terms in accumulators of their own. Logits after four Qwen2-0.5B-shaped
-// blocks are 6.8e-6 from a 64-bit forward pass this way, 6.9e-6 with the fp32 matrix cores.
+// sixteenth of the fp16 one. Here each value is hi + 2^-12 lo, two fp16 numbers after scaling its
+// row by a power of two that puts the row's largest magnitude in [2^14, 2^15): hi has 11 bits, lo
+// the next 11. lo is stored 2^12 times its size, as large as hi can be, so that it keeps its bits
+// where the value is small: the pair is the value to 2^-23 of it down to 2^-27 of the row's
+// largest, and to 2^-51 of that below (stored at its size lo ran out at 2^-39, and a row with one
+// value 2^24 times the rest lost 2^-16 of the rest). Then
+//   x . w = hi hi + 2^-12 (hi lo + lo hi) + 2^-24 lo lo
+// with the last term (at most 2^-22 of a product) left out: three 16x16x32 products, exact in fp32
+// and summed in fp32, the cross terms in accumulators of their own. Against 64 bits the product
+// is 1.4e-7 to 6.9e-7 off (relative L2, 896 to 16384 columns), the fp32 matrix cores' 5.0e-7 to
+// 2.3e-6 (their longer chains of rounded sums).
 // A 511-token pass of such a block: 410 -> 245 us (products 245 -> 110, decodes 134 -> 50).
 // Rows with a NaN or an infinity are marked (inv < 0) and their outputs recomputed from the
 // planes' values in plain fp32, so that they come out as an fp32 product's.
@@ -60,18 +63,27 @@ __device__ __forceinline__ float block_sum(float v) {
 }
 
 // The power of two that takes a finite magnitude mx into [2^14, 2^15) (1 for a zero row; at
-// most 2^100, so that it and its inverse are normal numbers), and its inverse.
+// most 2^126, so that it and its inverse are normal numbers), and its inverse.
 __device__ __forceinline__ void row_scale(float mx, float& up, float& down) {
     int e = 0;
-    if (mx > 0.f) e = min(14 - ilogbf(mx), 100);
+    if (mx > 0.f) e = min(14 - ilogbf(mx), 126);
     up = ldexpf(1.0f, e);
     down = ldexpf(1.0f, -e);
 }
 
+constexpr float kLoUp = 4096.f, kLoDown = 1.f / 4096.f;  // |s - hi| <= 2^3: lo to 2^15
+
 __device__ __forceinline__ void split1(float v, float up, _Float16& hi, _Float16& lo) {
     const float s = v * up;
     hi = (_Float16)s;
-    lo = fabsf(s) < INFINITY ? (_Float16)(s - (float)hi) : (_Float16)0.f;
+    lo = fabsf(s) < INFINITY ? (_Float16)((s - (float)hi) * kLoUp) : (_Float16)0.f;
+}
+
+// v times the row scales a and b (powers of two, signs aside): by their exponents' sum, since
+// one of the two alone may take v out of range on the way to a result that is in it.
+__device__ __forceinline__ float unscale(float v, float a, float b) {
+    const auto ex = [](float f) { return (int)(__builtin_bit_cast(uint32_t, f) >> 23 & 0xFF) - 127; };
+    return __builtin_amdgcn_ldexpf(v, ex(a) + ex(b));
 }
 
 // A magnitude for the row's largest: 0 for a value that is not finite (noted in `odd`).
@@ -370,7 +382,7 @@ __global__ __launch_bounds__(kThreads) void split_gemm_kernel(GemmArgs a) {
             for (int v = 0; v < 4; ++v) {
                 if (r + v >= mat.R) continue;
                 const float wi = mat.w.inv[r + v];
-                out[v] = (acc[x][y][v] + cross[x][y][v]) * fabsf(wi) * fabsf(xi);
+                out[v] = unscale(fmaf(cross[x][y][v], kLoDown, acc[x][y][v]), wi, xi);
                 if (wi < 0.f || xi < 0.f) {  // a NaN or an infinity in the row: plain fp32
                     const _Float16 *wh2 = mat.w.hi + (size_t)(r + v) * mat.w.ld,
                                    *wl2 = mat.w.lo + (size_t)(r + v) * mat.w.ld;
@@ -378,9 +390,9 @@ __global__ __launch_bounds__(kThreads) void split_gemm_kernel(GemmArgs a) {
                                    *xl2 = a.x.lo + (size_t)m * a.x.ld;
                     float sum = 0.f;
                     for (int k = s0 * kBK; k < s1 * kBK; ++k)
-                        sum = fmaf((float)wh2[k] + (float)wl2[k], (float)xh2[k] + (float)xl2[k],
-                                   sum);
-                    out[v] = sum * fabsf(wi) * fabsf(xi);
+                        sum = fmaf(fmaf((float)wl2[k], kLoDown, (float)wh2[k]),
+                                   fmaf((float)xl2[k], kLoDown, (float)xh2[k]), sum);
+                    out[v] = unscale(sum, wi, xi);
                 }
                 if (mat.bias && a.parts == 1) out[v] += mat.bias[r + v];
             }

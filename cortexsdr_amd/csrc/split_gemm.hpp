@@ -6,7 +6,7 @@
 
 namespace csdr {
 
-// Rows of fp32 values as two fp16 planes: value = (hi + lo) * inv[row], ld values per row
+// Rows of fp32 values as two fp16 planes: value = (hi + 2^-12 lo) * inv[row], ld values per row
 // (zeros past the row's end). inv < 0 marks a row holding a NaN or an infinity.
 struct SplitPlanes {
     _Float16* hi = nullptr;
