@@ -446,39 +446,47 @@ size_t split_x_floats(const csdr_decoder_config& c, int rows) {
     return (size_t)rows * (widest + 1) + 16 + split_part_rows(c, rows) * c.hidden;
 }
 
-// Buffers of a prefill pass over `rows` token rows, kept for later passes of up to as many while
-// the blocks take the same form (csdr_decoder_set_layer may replace one by a block that does not,
-// or the last that did not by one that does); passes read the form from pf_split.
-int ensure_prefill(csdr_decoder* d, int rows) {
-    const bool eligible = prefill_split(d);
-    if (rows <= d->pf_rows && eligible == d->pf_eligible) return CSDR_OK;
-    free_prefill(d);
+// The buffers of a pass over `rows` token rows in one of its forms; nothing where one of them
+// cannot be had.
+bool alloc_prefill(csdr_decoder* d, int rows, bool split) {
     const csdr_decoder_config& c = d->cfg;
     const size_t n = (size_t)rows, H = c.hidden, F = c.ffn;
     const size_t kvw = (size_t)c.n_kv_heads * c.head_dim;
-    const bool split = eligible && rows >= kMinSplitRows;
     const size_t wmax =
         std::max({H * H, kvw * H, F * H, split ? split_w_floats(c) : (size_t)0});
     const std::pair<float**, size_t> bufs[] = {
         {&d->pf_x, n * H},   {&d->pf_h, n * H},   {&d->pf_q, n * H},
         {&d->pf_k, n * kvw}, {&d->pf_v, n * kvw}, {&d->pf_a, n * std::max(H, F)},
         {&d->pf_g, n * F},   {&d->pf_u, n * F},   {&d->pf_w, wmax},
-        {&d->pf_s, split ? split_x_floats(c, rows) : 4}};
+        {&d->pf_s, split ? split_x_floats(c, rows) : 0}};
+    bool ok = true;
     for (const auto& b : bufs) {
         void* p = nullptr;
-        if (hipMalloc(&p, b.second * 4) != hipSuccess) {
-            free_prefill(d);
-            return set_error(CSDR_E_HIP, "decoder_prefill: out of device memory for " +
-                                             std::to_string(rows) + " prefill rows");
-        }
-        *b.first = static_cast<float*>(p);
+        ok = ok && (b.second == 0 || hipMalloc(&p, b.second * 4) == hipSuccess);
+        *b.first = ok ? static_cast<float*>(p) : nullptr;
     }
     void* p = nullptr;
-    if (hipMalloc(&p, n * 4) != hipSuccess) {
+    ok = ok && hipMalloc(&p, n * 4) == hipSuccess;
+    d->pf_tok = ok ? static_cast<int*>(p) : nullptr;
+    if (!ok) {
+        (void)hipGetLastError();  // (the next launch check would report it)
         free_prefill(d);
-        return set_error(CSDR_E_HIP, "decoder_prefill: out of device memory");
     }
-    d->pf_tok = static_cast<int*>(p);
+    return ok;
+}
+
+// Buffers of a prefill pass over `rows` token rows, kept for later passes of up to as many while
+// the blocks take the same form (csdr_decoder_set_layer may replace one by a block that does not,
+// or the last that did not by one that does); passes read the form from pf_split. Where the split
+// form's (about twice the fp32 form's for the weights) cannot be had, the fp32 form's.
+int ensure_prefill(csdr_decoder* d, int rows) {
+    const bool eligible = prefill_split(d);
+    if (rows <= d->pf_rows && eligible == d->pf_eligible) return CSDR_OK;
+    free_prefill(d);
+    const bool split = eligible && rows >= kMinSplitRows && alloc_prefill(d, rows, true);
+    if (!split && !alloc_prefill(d, rows, false))
+        return set_error(CSDR_E_HIP, "decoder_prefill: out of device memory for " +
+                                         std::to_string(rows) + " prefill rows");
     d->pf_rows = rows;
     d->pf_eligible = eligible;
     d->pf_split = split;
