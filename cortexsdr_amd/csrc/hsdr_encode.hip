@@ -1146,6 +1146,15 @@ struct DevBuf {
     uint16_t* u16() const { return static_cast<uint16_t*>(p); }
 };
 
+// The Gram path's workspace; left empty, for mp_kernel and the same codes, where that path does
+// not pay or the memory cannot be had (asked for after what the call cannot do without).
+void alloc_gram(long long n, int C, int K, int S, int k, DevBuf* ws) {
+    if (gram_pays(n, C, K, S, k) && hipMalloc(&ws->p, gram_ws_bytes(n, K)) != hipSuccess) {
+        ws->p = nullptr;
+        (void)hipGetLastError();
+    }
+}
+
 // One atomUpdateStep per pass (HierarchicalSDRStrategy.cpp:281-490): users, residuals and
 // updates on the device, the re-seeds on the host from the fit's generator (base seed :403).
 struct Refine {
@@ -1283,8 +1292,6 @@ int fit_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t 
     if (rc != CSDR_OK) return rc;
     const size_t ncodes = (size_t)n_tiles * S * k, kc = (size_t)K * tile_dim;
     DevBuf d_tiles, d_D, d_codes, d_gram;
-    if (gram_pays(n_tiles, (int)tile_dim, K, S, k))
-        CSDR_HIP_CHECK(hipMalloc(&d_gram.p, gram_ws_bytes(n_tiles, K)));
     CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, (size_t)n_tiles * tile_dim * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_D.p, kc * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
@@ -1295,20 +1302,21 @@ int fit_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t 
     rc = init_dictionary_device(d_tiles.f(), n_tiles, tile_dim, K, (uint32_t)S * k, rng, d_D.f(),
                                 &mean_norm, st);
     if (rc != CSDR_OK) return rc;
+    Refine rf;
+    if (ksvd_iters) {
+        rc = rf.init(g, mean_norm, gamma, d_tiles.f(), d_D.f(), d_codes.u16());
+        if (rc != CSDR_OK) return rc;
+    }
+    alloc_gram(n_tiles, (int)tile_dim, K, S, k, &d_gram);
     rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
                    d_codes.u16(), d_gram.p, st);
     if (rc != CSDR_OK) return rc;
-    if (ksvd_iters) {
-        Refine rf;
-        rc = rf.init(g, mean_norm, gamma, d_tiles.f(), d_D.f(), d_codes.u16());
+    for (int it = 0; it < ksvd_iters; ++it) {  // atom update, then encode again (:570-573)
+        rc = rf.pass(tiles, rng, st);
         if (rc != CSDR_OK) return rc;
-        for (int it = 0; it < ksvd_iters; ++it) {  // atom update, then encode again (:570-573)
-            rc = rf.pass(tiles, rng, st);
-            if (rc != CSDR_OK) return rc;
-            rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
-                           d_codes.u16(), d_gram.p, st);
-            if (rc != CSDR_OK) return rc;
-        }
+        rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
+                       d_codes.u16(), d_gram.p, st);
+        if (rc != CSDR_OK) return rc;
     }
     CSDR_HIP_CHECK(hipMemcpyAsync(D, d_D.p, kc * 4, hipMemcpyDeviceToHost, st));
     if (codes)
@@ -1328,11 +1336,10 @@ int encode_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, const 
     if (rc != CSDR_OK) return rc;
     const size_t ncodes = (size_t)n_tiles * S * k;
     DevBuf d_tiles, d_D, d_codes, d_gram;
-    if (gram_pays(n_tiles, (int)tile_dim, K, S, k))
-        CSDR_HIP_CHECK(hipMalloc(&d_gram.p, gram_ws_bytes(n_tiles, K)));
     CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, std::max<size_t>((size_t)n_tiles * tile_dim, 1) * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_D.p, D.size() * 4));
     CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
+    alloc_gram(n_tiles, (int)tile_dim, K, S, k, &d_gram);
     CSDR_HIP_CHECK(hipMemcpyAsync(d_tiles.p, tiles, (size_t)n_tiles * tile_dim * 4,
                                   hipMemcpyHostToDevice, st));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_D.p, D.data(), D.size() * 4, hipMemcpyHostToDevice, st));

@@ -120,3 +120,30 @@ for budget in (need, 0):
     assert np.linalg.norm(got - want) < 1e-4 * np.linalg.norm(want), budget
 print("OK")
 """)
+
+
+COMPRESS = r"""
+R, C, K, S, k, iters = 2048, 64, 512, 2, 3, %d
+w = synth.normal(7, R * C, sigma=0.02).astype(np.float32).reshape(R, C)
+def go():
+    a = encode.compress(w, 1, C, K, S, k, ksvd_iters=iters)
+    b, skipped = encode.hsda_build({"a": w, "b": w[:600]}, 1, C, K, S, k, ksvd_iters=iters)
+    assert not skipped
+    return a, b
+want = go()
+n = R + 600                       # the archive's pool is the larger of the two
+codes = n * S * k
+need = n * C * 4 + K * C * 4 + codes * 2                   # tiles, dictionary, codes
+init = n * 8 + K * 12                                      # the initialisation's norms
+refine = n * C * 4 + (K + 1) * 4 + codes * 12 + K * 9      # residuals, user lists, flags
+shim.shim_budget(need + (refine if iters else init))
+assert go() == want
+assert shim.shim_live() == 0
+print("OK")
+"""
+
+
+def test_compress_without_room_for_the_scores(shim):
+    """Tiles, dictionary and codes, and no room for the Gram form's scores: the same bytes by
+    projections, for a matrix and for an archive of two."""
+    run(shim, COMPRESS % 0)
