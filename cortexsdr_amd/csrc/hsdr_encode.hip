@@ -772,7 +772,8 @@ int launch_mp(const float* tiles, long long n, int C, const float* D, int K, int
 //    24 slots: a thread per element with a 64-bit division each);
 //  atom_sum_kernel: correction[c] = sum over the atom's users, in order, of sign * gamma *
 //    residual (double, fused: :428-437), the new value atom + correction * (0.5 / sum gamma^2)
-//    rounded to float (:448-458). One thread per element; the users' rows are L2 reads whose
+//    rounded to float (:448-458), in the atom's place (one that is not finite is re-seeded
+//    whole). One thread per element; the users' rows are L2 reads whose
 //    latency bounds it, so a workgroup takes 256 elements of one atom (K x C / 256 of them)
 //    and eight rows are in flight;
 //  atom_finish_kernel: per atom, a non-finite value flags it for the host's re-seed (:461), the
@@ -783,7 +784,6 @@ struct FitArgs {
     const float* tiles;
     const uint16_t* codes;
     float* D;
-    float* nv;      // K x C new values
     float* res;     // n x C
     int* off;       // K + 1
     uint32_t* utile;
@@ -974,7 +974,8 @@ __global__ __launch_bounds__(kEThreads) void atom_sum_kernel(FitArgs a) {
     }
     for (; u < u1; ++u) corr = fma(a.ucoef[u], (double)a.res[(size_t)a.utile[u] * a.C + c], corr);
     // the new value through double; one that float cannot hold comes out infinite
-    a.nv[(size_t)j * a.C + c] = (float)fma(corr, iw, (double)a.D[(size_t)j * a.C + c]);
+    float& d = a.D[(size_t)j * a.C + c];
+    d = (float)fma(corr, iw, (double)d);
 }
 
 __global__ __launch_bounds__(kEThreads) void atom_finish_kernel(FitArgs a) {
@@ -989,7 +990,7 @@ __global__ __launch_bounds__(kEThreads) void atom_finish_kernel(FitArgs a) {
     float* atom = a.D + (size_t)j * C;
     int bad = 0;
     for (int c = tid; c < C; c += kEThreads) {
-        const float vf = a.nv[(size_t)j * C + c];
+        const float vf = atom[c];
         if (!isfinite(vf)) bad = 1;
         nv[c] = vf;
     }
@@ -1011,8 +1012,6 @@ __global__ __launch_bounds__(kEThreads) void atom_finish_kernel(FitArgs a) {
     if (nn > a.cap) {
         const double sc = a.target / nn;
         for (int c = tid; c < C; c += kEThreads) atom[c] = (float)((double)nv[c] * sc);
-    } else {
-        for (int c = tid; c < C; c += kEThreads) atom[c] = nv[c];
     }
 }
 
@@ -1158,15 +1157,13 @@ void alloc_gram(long long n, int C, int K, int S, int k, DevBuf* ws) {
 // One atomUpdateStep per pass (HierarchicalSDRStrategy.cpp:281-490): users, residuals and
 // updates on the device, the re-seeds on the host from the fit's generator (base seed :403).
 struct Refine {
-    DevBuf res, nv, off, utile, ucoef, invw, flag;
+    DevBuf res, off, utile, ucoef, invw, flag;
     FitArgs fa{};
 
     int init(const Geometry& g, double mean_norm, const std::vector<float>& gamma,
              const float* d_tiles, float* d_D, const uint16_t* d_codes) {
         const size_t slots = (size_t)g.S * g.k, ncodes = (size_t)g.n_tiles * slots;
-        const size_t kc = (size_t)g.K * g.tile_dim;
         CSDR_HIP_CHECK(hipMalloc(&res.p, (size_t)g.n_tiles * g.tile_dim * 4));
-        CSDR_HIP_CHECK(hipMalloc(&nv.p, kc * 4));
         CSDR_HIP_CHECK(hipMalloc(&off.p, ((size_t)g.K + 1) * 4));
         CSDR_HIP_CHECK(hipMalloc(&utile.p, std::max<size_t>(ncodes, 1) * 4));
         CSDR_HIP_CHECK(hipMalloc(&ucoef.p, std::max<size_t>(ncodes, 1) * 8));
@@ -1175,7 +1172,6 @@ struct Refine {
         fa.tiles = d_tiles;
         fa.codes = d_codes;
         fa.D = d_D;
-        fa.nv = nv.f();
         fa.res = res.f();
         fa.off = static_cast<int*>(off.p);
         fa.utile = static_cast<uint32_t*>(utile.p);

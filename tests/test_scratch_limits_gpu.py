@@ -147,3 +147,9 @@ def test_compress_without_room_for_the_scores(shim):
     """Tiles, dictionary and codes, and no room for the Gram form's scores: the same bytes by
     projections, for a matrix and for an archive of two."""
     run(shim, COMPRESS % 0)
+
+
+def test_refinement_in_the_memory_of_its_results(shim):
+    """Two refinement passes in the tiles, dictionary, codes, residuals and user lists, the
+    buffers that the passes cannot do without."""
+    run(shim, COMPRESS % 2)
