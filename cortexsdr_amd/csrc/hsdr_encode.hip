@@ -66,8 +66,9 @@ struct MpArgs {
     uint16_t* codes;     // n x S*k, packIndexSign
     long long n;
     int C, K, S, k, tt;
-    const int* list;   // NULL: tiles 0 .. n - 1; else *count tiles by number (TT = 1)
+    const int* list;   // mp_list_kernel: *count tiles by number, up to `few` of them one a workgroup
     const int* count;
+    int few;
     float gamma[kMaxStages];
 };
 
@@ -93,8 +94,9 @@ __device__ __forceinline__ void load_tiles(const float* rc, float* rv) {
     }
 }
 
-template <int TT>
-__device__ __forceinline__ void mp_tiles(const MpArgs& a, long long t0, int nt) {
+// The nt tiles first, first + 1, ... or (LIST) list[first], list[first + 1], ...
+template <int TT, bool LIST>
+__device__ __forceinline__ void mp_tiles(const MpArgs& a, long long first, int nt) {
     extern __shared__ float smem[];
     const int tt = TT, C = a.C, K = a.K;
     float* r = smem;                                                    // C x TT residuals
@@ -102,13 +104,16 @@ __device__ __forceinline__ void mp_tiles(const MpArgs& a, long long t0, int nt) 
     uint8_t* used = reinterpret_cast<uint8_t*>(proj + (size_t)tt * K);  // nt x K
     __shared__ int best_s[TT];
     __shared__ float scale_s[TT];
+    const auto number = [&](int t) {
+        return LIST ? (long long)a.list[first + min(t, nt - 1)] : first + t;
+    };
     const int tid = threadIdx.x, l16 = tid & 15, grp = tid >> 4;
     const int lane = tid & 63, wave = tid >> 6;
     // residuals tile-minor, r[c * TT + t] (one 16-byte LDS read gives four tiles' values of an
     // element); slots past nt hold zeros
     for (int i = tid; i < TT * C; i += kEThreads) {
         const int c = i / TT, t = i - c * TT;
-        r[i] = t < nt ? a.tiles[(t0 + t) * C + c] : 0.f;
+        r[i] = t < nt ? a.tiles[number(t) * C + c] : 0.f;
     }
     // atoms per 16-lane group at a time: 8 with up to 2 tiles (D blocks of 4 chunks), 2 with
     // more (registers; measured 896 x 896 at 2 tiles: 0.60 ms with 2, 0.51 with 4, 0.45 with 8;
@@ -215,7 +220,7 @@ __device__ __forceinline__ void mp_tiles(const MpArgs& a, long long t0, int nt) 
                 }
                 if (lane == 0) {
                     const int sg = proj[t * K + bi] >= 0.0f ? 1 : -1;
-                    a.codes[(size_t)(t0 + t) * slots + l * a.k + st] =
+                    a.codes[(size_t)number(t) * slots + l * a.k + st] =
                         (uint16_t)((bi & 0x7FFF) | (sg < 0 ? 0x8000 : 0));
                     used[t * K + bi] = 1;
                     best_s[t] = bi;
@@ -237,17 +242,42 @@ __device__ __forceinline__ void mp_tiles(const MpArgs& a, long long t0, int nt) 
 template <int TT>
 __global__ __launch_bounds__(kEThreads) void mp_kernel(MpArgs a) {
     const long long t0 = (long long)blockIdx.x * TT;
-    mp_tiles<TT>(a, t0, (int)min((long long)TT, a.n - t0));
+    mp_tiles<TT, false>(a, t0, (int)min((long long)TT, a.n - t0));
 }
 
-// The tiles that mp_gram_kernel leaves (list, count).
+// The tiles that mp_gram_kernel leaves (list, count): up to `few` of them one a workgroup, more
+// of them (a matrix of equal or parallel rows, whose atoms are all alike, leaves every tile) TT at
+// a time as mp_kernel takes them; two kernels, each launched and one of them returning at once,
+// since one with both bodies had neither's registers. (4864 x 896, K = 512, 24 picks, rows of one
+// value each: 9.2 ms with one tile a workgroup throughout, 3.8 here, 3.4 with mp_kernel alone.)
+template <int TT>
 __global__ __launch_bounds__(kEThreads) void mp_list_kernel(MpArgs a) {
     const int n = *a.count;
-    for (int b = blockIdx.x; b < n; b += gridDim.x) mp_tiles<1>(a, a.list[b], 1);
+    if ((TT == 1) != (n <= a.few)) return;
+    if constexpr (TT == 1) {
+        for (int b = blockIdx.x; b < n; b += gridDim.x) mp_tiles<1, true>(a, b, 1);
+    } else {
+        const int first = blockIdx.x * TT;
+        if (first < n) mp_tiles<TT, true>(a, first, min(TT, n - first));
+    }
 }
 
 size_t mp_lds_bytes(int tt, int C, int K) {
     return (size_t)tt * ((size_t)C + K) * 4 + csdr::align_up((size_t)tt * K, 16);
+}
+
+// Tiles per workgroup: about n / 1024, at least 2 (measured on the Qwen2-0.5B shapes, 1-row
+// tiles: 896 x 896 best at 2 (0.93 ms vs 1.00 at 4, 1.31 at 8), 4864 x 896 at 4 (4.5 ms vs 5.0
+// at 8, 7.3 at 2): enough workgroups per CU to hide latency, and every workgroup reads all of
+// D once per pick, so more tiles each is less D traffic), a power of two, at most 8 and what
+// fits under the soft LDS size; else one tile under the hard size; else 0 (too large).
+int mp_tiles_per_wg(long long n, int C, int K) {
+    const char* ev = std::getenv("CSDR_HSDR_TILES_PER_WG");  // tuning override: 1, 2, 4 or 8
+    long long want = std::min<long long>(kMaxTT, std::max<long long>(2, n / 1024));
+    if (ev && std::atoi(ev) >= 1) want = std::min(kMaxTT, std::atoi(ev));
+    for (int tt = kMaxTT; tt >= 1; tt >>= 1)  // a power of two (the kernel's template)
+        if (tt <= want && mp_lds_bytes(tt, C, K) <= kLdsSoft) return tt;
+    return mp_lds_bytes(1, C, K) <= kLdsHard ? 1 : 0;
 }
 
 // ---------------------------------------------------------------- picks through the Gram matrix
@@ -453,7 +483,7 @@ __global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
             const float v = x[c] / mx;
             n2 = fmaf(v, v, n2);
         }
-    const float n0 = mx > 0.f ? mx * __builtin_amdgcn_sqrtf(csdr::wave_sum(n2)) * 1.01f : 0.f;
+    float n0 = mx > 0.f ? mx * __builtin_amdgcn_sqrtf(csdr::wave_sum(n2)) * 1.01f : 0.f;
     const auto leave = [&] {
         if (lane == 0) a.list[atomicAdd(a.count, 1)] = tile;
     };
@@ -461,6 +491,14 @@ __global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
         !(n0 == 0.f || (n0 >= 1e-12f && n0 <= 1e12f))) {
         leave();
         return;
+    }
+    // a zero tile's residual stays exactly zero while its pick, atom 0, is all zeros: n0 of 0 says
+    // so, kZeroNorm that the first pick ends it
+    constexpr float kZeroNorm = 1e-38f;
+    if (n0 == 0.f) {
+        bool live = false;
+        for (int c = lane; c < C; c += 64) live |= a.D[c] != 0.f;
+        if (__any(live)) n0 = kZeroNorm;
     }
     const float u = 1.25f * 5.9604645e-8f * dmax;
     float rn2 = n0 * n0, nmax2 = rn2, len = 0.f;
@@ -510,8 +548,8 @@ __global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
                             __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[i]), src));
                     }
                 sg = sv >= 0.f ? 1 : -1;
-            } else if (n0 == 0.f && t == 0) {
-                // a zero tile: every projection is 0, atom 0 stands
+            } else if (n0 <= kZeroNorm && (t == 0 || n0 == 0.f)) {
+                // a zero residual: every projection is 0, atom 0 stands
             } else if (nc > kGramMaxCand) {
                 leave();
                 return;
@@ -677,7 +715,12 @@ int launch_mp_gram(const float* tiles, long long n, int C, const float* D, int K
     b.list = count + 1;
     for (int l = 0; l < S; ++l) a.gamma[l] = b.gamma[l] = gamma[l];
     const size_t lds = gram_lds_bytes(C, S, k);
-    const size_t list_lds = mp_lds_bytes(1, C, K);
+    // (from 4096 tiles on; below, two tiles a workgroup gain less than the second launch costs)
+    const int tt = mp_tiles_per_wg(n, C, K);
+    b.few = tt >= 4 ? 1024 : 0x7fffffff;
+    const auto list = [&](auto kern, int per, long long most) {
+        kern<<<(unsigned)((most + per - 1) / per), kEThreads, mp_lds_bytes(per, C, K), st>>>(b);
+    };
     for (long long t0 = 0; t0 < n; t0 += chunk) {
         const long long nt = std::min(chunk, n - t0);
         a.tiles = b.tiles = tiles + (size_t)t0 * C;
@@ -690,24 +733,14 @@ int launch_mp_gram(const float* tiles, long long n, int C, const float* D, int K
         else if (K <= 512) mp_gram_kernel<8><<<grid, 64, lds, st>>>(a);
         else if (K <= 1024) mp_gram_kernel<16><<<grid, 64, lds, st>>>(a);
         else mp_gram_kernel<32><<<grid, 64, lds, st>>>(a);
-        mp_list_kernel<<<(unsigned)std::min<long long>(nt, 1024), kEThreads, list_lds, st>>>(b);
+        list(&mp_list_kernel<1>, 1, std::min<long long>(nt, 1024));
+        if (nt > b.few) {
+            if (tt == 8) list(&mp_list_kernel<8>, 8, nt);
+            else list(&mp_list_kernel<4>, 4, nt);
+        }
         CSDR_LAUNCH_CHECK("hsdr_encode");
     }
     return CSDR_OK;
-}
-
-// Tiles per workgroup: about n / 1024, at least 2 (measured on the Qwen2-0.5B shapes, 1-row
-// tiles: 896 x 896 best at 2 (0.93 ms vs 1.00 at 4, 1.31 at 8), 4864 x 896 at 4 (4.5 ms vs 5.0
-// at 8, 7.3 at 2): enough workgroups per CU to hide latency, and every workgroup reads all of
-// D once per pick, so more tiles each is less D traffic), a power of two, at most 8 and what
-// fits under the soft LDS size; else one tile under the hard size; else 0 (too large).
-int mp_tiles_per_wg(long long n, int C, int K) {
-    const char* ev = std::getenv("CSDR_HSDR_TILES_PER_WG");  // tuning override: 1, 2, 4 or 8
-    long long want = std::min<long long>(kMaxTT, std::max<long long>(2, n / 1024));
-    if (ev && std::atoi(ev) >= 1) want = std::min(kMaxTT, std::atoi(ev));
-    for (int tt = kMaxTT; tt >= 1; tt >>= 1)  // a power of two (the kernel's template)
-        if (tt <= want && mp_lds_bytes(tt, C, K) <= kLdsSoft) return tt;
-    return mp_lds_bytes(1, C, K) <= kLdsHard ? 1 : 0;
 }
 
 int check_mp_shape(long long n, int C, int K, int S, int k) {

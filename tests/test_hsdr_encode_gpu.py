@@ -108,6 +108,47 @@ def test_encode_ties_and_odd_tiles_match_oracle(gpu, monkeypatch, n, C, K, S, k)
     assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), oracle.hsdr_mp(t, D, g, S, k))
 
 
+# Tiles left to projections, by the thousand: in the first chunk of tiles (2^24 / K) more than the
+# 1024 that go one a workgroup, a count off the tiles per workgroup (4 at K = 2048, 8 at K = 64),
+# and in a second chunk, whose tiles and codes are at an offset, a few.
+@pytest.mark.parametrize("n,C,K,S,k,n_left", [(8192 + 300, 8, 2048, 2, 2, 1201),
+                                              (9001, 24, 64, 2, 3, 9001)])
+def test_encode_many_tiles_left_match_oracle(gpu, monkeypatch, n, C, K, S, k, n_left):
+    monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
+    rng = np.random.default_rng(n + K)
+    t = (rng.standard_normal((n, C)) * 0.02).astype(np.float32)
+    D = rng.standard_normal((K, C)).astype(np.float32)
+    D *= 0.02 * np.sqrt(C / (S * k)) / np.linalg.norm(D, axis=1, keepdims=True)
+    left = rng.permutation(min(n, 8192) if n_left < n else n)[:n_left]
+    t[left] *= np.where(rng.random((n_left, 1)) < 0.5, 1e-15, 1e15).astype(np.float32)
+    if n_left < n:
+        t[8192 + 17:8192 + 60:3] *= np.float32(1e15)
+    g = (0.5 ** np.arange(S)).astype(np.float32)
+    assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), oracle.hsdr_mp(t, D, g, S, k))
+
+
+@pytest.mark.parametrize("zero_atom", [True, False])
+def test_encode_zero_tiles_match_oracle(gpu, monkeypatch, zero_atom):
+    """Zero tiles where atom 0, their first pick, is all zeros (it then stands at every pick), and
+    where it is not, its values as small as fp32 holds included."""
+    monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
+    n, C, K, S, k = 300, 100, 200, 3, 4
+    rng = np.random.default_rng(5)
+    t = (rng.standard_normal((n, C)) * 0.02).astype(np.float32)
+    t[::2] = 0
+    t[4, 60] = -0.0
+    D = (rng.standard_normal((K, C)) * 0.01).astype(np.float32)
+    D[0] = 0
+    D[9:40] = 0
+    D[12, 99] = 1e-38
+    if not zero_atom:
+        D[0, 70] = 1e-30
+    g = (0.5 ** np.arange(S)).astype(np.float32)
+    want = oracle.hsdr_mp(t, D, g, S, k)
+    assert zero_atom == (not want.reshape(n, -1)[::2].any())
+    assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), want)
+
+
 def test_encode_more_picks_than_the_gram_form_holds(gpu, monkeypatch):
     # 32 x 345 picks and their gains are past 64 KiB of LDS: mp_kernel, which keeps none
     monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
