@@ -1178,14 +1178,43 @@ struct DevBuf {
     uint16_t* u16() const { return static_cast<uint16_t*>(p); }
 };
 
-// The Gram path's workspace; left empty, for mp_kernel and the same codes, where that path does
-// not pay or the memory cannot be had (asked for after what the call cannot do without).
-void alloc_gram(long long n, int C, int K, int S, int k, DevBuf* ws) {
-    if (gram_pays(n, C, K, S, k) && hipMalloc(&ws->p, gram_ws_bytes(n, K)) != hipSuccess) {
-        ws->p = nullptr;
-        (void)hipGetLastError();
+// The buffers of one fit or encode. The Gram path's workspace is asked for first (its allocation
+// and the others' run beside the work already on the device) and left empty, for mp_kernel and
+// the same codes, where that path does not pay or the memory cannot be had; it is given up again
+// where a buffer that the call cannot do without finds no room.
+struct Scratch {
+    DevBuf gram;
+    hipStream_t st;
+
+    Scratch(long long n, int C, int K, int S, int k, hipStream_t stream) : st(stream) {
+        if (gram_pays(n, C, K, S, k) && hipMalloc(&gram.p, gram_ws_bytes(n, K)) != hipSuccess) {
+            gram.p = nullptr;
+            (void)hipGetLastError();
+        }
     }
-}
+
+    int need(DevBuf& b, size_t bytes) {
+        hipError_t e = hipMalloc(&b.p, bytes);
+        if (e != hipSuccess && gram.p) {
+            (void)hipGetLastError();
+            (void)hipStreamSynchronize(st);  // an encode may still be reading it
+            (void)hipFree(gram.p);
+            gram.p = nullptr;
+            e = hipMalloc(&b.p, bytes);
+        }
+        if (e == hipSuccess) return CSDR_OK;
+        b.p = nullptr;
+        (void)hipGetLastError();
+        return set_error(CSDR_E_HIP, "hsdr_compress: out of device memory (" +
+                                         std::to_string(bytes) + " bytes)");
+    }
+};
+
+#define RC(expr)                        \
+    do {                                \
+        const int rc_ = (expr);         \
+        if (rc_ != CSDR_OK) return rc_; \
+    } while (0)
 
 // One atomUpdateStep per pass (HierarchicalSDRStrategy.cpp:281-490): users, residuals and
 // updates on the device, the re-seeds on the host from the fit's generator (base seed :403).
@@ -1194,14 +1223,14 @@ struct Refine {
     FitArgs fa{};
 
     int init(const Geometry& g, double mean_norm, const std::vector<float>& gamma,
-             const float* d_tiles, float* d_D, const uint16_t* d_codes) {
+             const float* d_tiles, float* d_D, const uint16_t* d_codes, Scratch& scratch) {
         const size_t slots = (size_t)g.S * g.k, ncodes = (size_t)g.n_tiles * slots;
-        CSDR_HIP_CHECK(hipMalloc(&res.p, (size_t)g.n_tiles * g.tile_dim * 4));
-        CSDR_HIP_CHECK(hipMalloc(&off.p, ((size_t)g.K + 1) * 4));
-        CSDR_HIP_CHECK(hipMalloc(&utile.p, std::max<size_t>(ncodes, 1) * 4));
-        CSDR_HIP_CHECK(hipMalloc(&ucoef.p, std::max<size_t>(ncodes, 1) * 8));
-        CSDR_HIP_CHECK(hipMalloc(&invw.p, (size_t)g.K * 8));
-        CSDR_HIP_CHECK(hipMalloc(&flag.p, (size_t)g.K));
+        RC(scratch.need(res, (size_t)g.n_tiles * g.tile_dim * 4));
+        RC(scratch.need(off, ((size_t)g.K + 1) * 4));
+        RC(scratch.need(utile, std::max<size_t>(ncodes, 1) * 4));
+        RC(scratch.need(ucoef, std::max<size_t>(ncodes, 1) * 8));
+        RC(scratch.need(invw, (size_t)g.K * 8));
+        RC(scratch.need(flag, (size_t)g.K));
         fa.tiles = d_tiles;
         fa.codes = d_codes;
         fa.D = d_D;
@@ -1269,9 +1298,9 @@ void put(std::vector<uint8_t>& out, const T& v) {
 // (the square roots summed in tile order, as hsdr_init.cpp does).
 int init_dictionary_device(const float* d_tiles, uint32_t n, uint32_t C, uint16_t K,
                            uint32_t slots, std::mt19937& rng, float* d_D, double* mean_norm,
-                           hipStream_t st) {
+                           Scratch& scratch, hipStream_t st) {
     DevBuf ws;  // n squared norms, then K picks, K squared norms, K factors
-    CSDR_HIP_CHECK(hipMalloc(&ws.p, (size_t)n * 8 + (size_t)K * 12));
+    RC(scratch.need(ws, (size_t)n * 8 + (size_t)K * 12));
     double* d_norm = static_cast<double*>(ws.p);
     uint32_t* d_src = reinterpret_cast<uint32_t*>(d_norm + n);
     float* d_sq = reinterpret_cast<float*>(d_src + K);
@@ -1320,32 +1349,29 @@ int fit_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, uint16_t 
     int rc = check_mp_shape(n_tiles, (int)tile_dim, K, S, k);
     if (rc != CSDR_OK) return rc;
     const size_t ncodes = (size_t)n_tiles * S * k, kc = (size_t)K * tile_dim;
-    DevBuf d_tiles, d_D, d_codes, d_gram;
-    CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, (size_t)n_tiles * tile_dim * 4));
-    CSDR_HIP_CHECK(hipMalloc(&d_D.p, kc * 4));
-    CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
+    Scratch scratch(n_tiles, (int)tile_dim, K, S, k, st);
+    DevBuf d_tiles, d_D, d_codes;
+    RC(scratch.need(d_tiles, (size_t)n_tiles * tile_dim * 4));
+    RC(scratch.need(d_D, kc * 4));
+    RC(scratch.need(d_codes, std::max<size_t>(ncodes * 2, 2)));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_tiles.p, tiles, (size_t)n_tiles * tile_dim * 4,
                                   hipMemcpyHostToDevice, st));
     std::mt19937 rng(0xC0DE);  // the fit's generator (:513), through init and every pass
     double mean_norm = 0.0;
-    rc = init_dictionary_device(d_tiles.f(), n_tiles, tile_dim, K, (uint32_t)S * k, rng, d_D.f(),
-                                &mean_norm, st);
-    if (rc != CSDR_OK) return rc;
-    Refine rf;
+    RC(init_dictionary_device(d_tiles.f(), n_tiles, tile_dim, K, (uint32_t)S * k, rng, d_D.f(),
+                              &mean_norm, scratch, st));
+    const auto encode = [&] {
+        return launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
+                         d_codes.u16(), scratch.gram.p, st);
+    };
+    RC(encode());
     if (ksvd_iters) {
-        rc = rf.init(g, mean_norm, gamma, d_tiles.f(), d_D.f(), d_codes.u16());
-        if (rc != CSDR_OK) return rc;
-    }
-    alloc_gram(n_tiles, (int)tile_dim, K, S, k, &d_gram);
-    rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
-                   d_codes.u16(), d_gram.p, st);
-    if (rc != CSDR_OK) return rc;
-    for (int it = 0; it < ksvd_iters; ++it) {  // atom update, then encode again (:570-573)
-        rc = rf.pass(tiles, rng, st);
-        if (rc != CSDR_OK) return rc;
-        rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
-                       d_codes.u16(), d_gram.p, st);
-        if (rc != CSDR_OK) return rc;
+        Refine rf;
+        RC(rf.init(g, mean_norm, gamma, d_tiles.f(), d_D.f(), d_codes.u16(), scratch));
+        for (int it = 0; it < ksvd_iters; ++it) {  // atom update, then encode again (:570-573)
+            RC(rf.pass(tiles, rng, st));
+            RC(encode());
+        }
     }
     CSDR_HIP_CHECK(hipMemcpyAsync(D, d_D.p, kc * 4, hipMemcpyDeviceToHost, st));
     if (codes)
@@ -1364,16 +1390,16 @@ int encode_tiles(const float* tiles, uint32_t n_tiles, uint32_t tile_dim, const 
     int rc = check_mp_shape(n_tiles, (int)tile_dim, K, S, k);
     if (rc != CSDR_OK) return rc;
     const size_t ncodes = (size_t)n_tiles * S * k;
-    DevBuf d_tiles, d_D, d_codes, d_gram;
-    CSDR_HIP_CHECK(hipMalloc(&d_tiles.p, std::max<size_t>((size_t)n_tiles * tile_dim, 1) * 4));
-    CSDR_HIP_CHECK(hipMalloc(&d_D.p, D.size() * 4));
-    CSDR_HIP_CHECK(hipMalloc(&d_codes.p, std::max<size_t>(ncodes * 2, 2)));
-    alloc_gram(n_tiles, (int)tile_dim, K, S, k, &d_gram);
+    Scratch scratch(n_tiles, (int)tile_dim, K, S, k, st);
+    DevBuf d_tiles, d_D, d_codes;
+    RC(scratch.need(d_tiles, std::max<size_t>((size_t)n_tiles * tile_dim, 1) * 4));
+    RC(scratch.need(d_D, D.size() * 4));
+    RC(scratch.need(d_codes, std::max<size_t>(ncodes * 2, 2)));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_tiles.p, tiles, (size_t)n_tiles * tile_dim * 4,
                                   hipMemcpyHostToDevice, st));
     CSDR_HIP_CHECK(hipMemcpyAsync(d_D.p, D.data(), D.size() * 4, hipMemcpyHostToDevice, st));
     rc = launch_mp(d_tiles.f(), n_tiles, (int)tile_dim, d_D.f(), K, S, k, gamma.data(),
-                   d_codes.u16(), d_gram.p, st);
+                   d_codes.u16(), scratch.gram.p, st);
     if (rc != CSDR_OK) return rc;
     codes.resize(ncodes);
     CSDR_HIP_CHECK(hipMemcpyAsync(codes.data(), d_codes.p, ncodes * 2, hipMemcpyDeviceToHost, st));
