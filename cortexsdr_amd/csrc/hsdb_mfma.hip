@@ -74,13 +74,6 @@ struct MParams {
     int m0;  // first column of this launch (the launch covers 16 * NT columns)
 };
 
-// X element (feature k, column m) in the call's layout.
-__device__ __forceinline__ float xget(const MParams& p, const MDesc& d, int k, int m) {
-    const size_t i = p.tm ? (size_t)m * (d.C_full + d.Ce) + k : (size_t)k * p.M + m;
-    return p.x_f16 ? (float)static_cast<const _Float16*>(d.x)[i]
-                   : static_cast<const float*>(d.x)[i];
-}
-
 // Transposed X: 16-byte granule g (8 permuted k positions) of block column b and column m, in the
 // order in which a wave loads a 16-column operand: [b][m / 16][g % 2][g / 2][m % 16], so that
 // one load instruction reads 1 KiB in a row. In halves from xt (the lo part xt_part on).
@@ -92,72 +85,126 @@ __device__ __forceinline__ size_t xt_part(const MParams& p, const MDesc& d) {
 }
 
 // ---- init: Y start values, and X transposed into operand granules. blockIdx.x below xwgs: one
-// block column and up to 64 columns of X through LDS (read along X's rows, written granule by
+// block column and MW columns of X through LDS (read along X's rows, written granule by
 // granule; straight from X to the granules each lane's 8 values were 8 separate 2-byte loads
-// and its 16-byte store a line of its own). The others: Y.
+// and its 16-byte store a line of its own). The others: Y. Bound by round trips where the matrix
+// is small, so all of a thread's X values are loaded before the first is used (896 x 896, 65
+// columns: 8.6 us with four rounds of four loads, 4.0 here), and by the edge strip's operands
+// where there is one, so a thread takes four outputs that share the coalesced operand once there
+// are more than kEdgeWide of them (14336 x 300, 256 columns: 94 us an output a thread and at most
+// 1024 workgroups, 34 here; with fewer, one: 9 columns 18.0 us a call, 24.3 with four).
+constexpr size_t kEdgeWide = 1 << 20;
+
+template <typename XT, int MW>
+__device__ __forceinline__ void init_x(const MParams& p, const MDesc& d, int wg, float (*tile)[65]) {
+    constexpr int kPer = 64 * MW / kThreads;  // values per thread
+    const int tid = threadIdx.x, M = p.M;
+    const int nmt = p.Mpad / MW;
+    const int b = wg / nmt, m0 = (wg - b * nmt) * MW;
+    if (b >= d.NB) return;
+    const XT* x = static_cast<const XT*>(d.x);
+    // feature-major: threads along a feature's columns; token-major: along a column's features
+    // (at clamped columns)
+    const size_t C = d.C_full + d.Ce;
+    float v[kPer];
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+        const int i = tid + e * kThreads;
+        const int k = p.tm ? (i & 63) : i / MW, c = p.tm ? (i >> 6) : i & (MW - 1);
+        const int m = min(m0 + c, M - 1);
+        v[e] = (float)x[p.tm ? (size_t)m * C + b * 64 + k : (size_t)(b * 64 + k) * M + m];
+    }
+#pragma unroll
+    for (int e = 0; e < kPer; ++e) {
+        const int i = tid + e * kThreads;
+        const int k = p.tm ? (i & 63) : i / MW, c = p.tm ? (i >> 6) : i & (MW - 1);
+        tile[k][c] = m0 + c < M ? v[e] : 0.0f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i0 = 0; i0 < MW * 8; i0 += kThreads) {
+        const int i = i0 + tid;
+        if (MW * 8 < kThreads && i >= MW * 8) break;
+        const int c = i & (MW - 1), g = i / MW;
+        _Float16 hi[8], lo[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float xv = tile[csdr::kperm64(g * 8 + j)][c];
+            hi[j] = (_Float16)xv;
+            lo[j] = (_Float16)(xv - (float)hi[j]);
+        }
+        const size_t o = xt_granule(p, b, m0 + c, g);
+        *reinterpret_cast<u32x4*>(d.xt + o) = __builtin_bit_cast(u32x4, hi);
+        if (sizeof(XT) == 4)
+            *reinterpret_cast<u32x4*>(d.xt + xt_part(p, d) + o) = __builtin_bit_cast(u32x4, lo);
+    }
+}
+
+// Y = (Y +) bias + edge . X: OUT rows of a column (row-major Y: threads along the columns) or
+// columns of a row (token-major: along the rows), each sum in feature order.
+template <typename XT, int OUT>
+__device__ __forceinline__ void init_edge(const MParams& p, const MDesc& d, size_t t0,
+                                          size_t stride) {
+    const int M = p.M, R = d.R, Ce = d.Ce;
+    const XT* x = static_cast<const XT*>(d.x);
+    const size_t C = d.C_full + Ce;
+    const int fast = p.tm ? R : M, slow = p.tm ? M : R;
+    const size_t n = (size_t)((slow + OUT - 1) / OUT) * fast;
+    for (size_t t = t0; t < n; t += stride) {
+        const int f = (int)(t % fast), s0 = (int)(t / fast) * OUT;
+        const float* e[OUT];
+        const XT* xv[OUT];
+        float s[OUT];
+#pragma unroll
+        for (int q = 0; q < OUT; ++q) {  // past the end the last one (not stored)
+            const int sq = min(s0 + q, slow - 1), r = p.tm ? f : sq, m = p.tm ? sq : f;
+            e[q] = d.edge + (size_t)r * Ce;
+            xv[q] = x + (p.tm ? (size_t)m * C + d.C_full : (size_t)d.C_full * M + m);
+            s[q] = 0.0f;
+        }
+        const size_t xs = p.tm ? 1 : M;
+#pragma unroll 8
+        for (int cc = 0; cc < Ce; ++cc)
+            if (p.tm) {
+                const float ev = e[0][cc];
+#pragma unroll
+                for (int q = 0; q < OUT; ++q) s[q] = fmaf(ev, (float)xv[q][cc], s[q]);
+            } else {
+                const float x0 = (float)xv[0][cc * xs];
+#pragma unroll
+                for (int q = 0; q < OUT; ++q) s[q] = fmaf(e[q][cc], x0, s[q]);
+            }
+#pragma unroll
+        for (int q = 0; q < OUT; ++q) {
+            if (s0 + q >= slow) break;
+            float& y = d.y[(size_t)(s0 + q) * fast + f];
+            float v = p.accumulate ? y : 0.0f;
+            if (d.bias) v += d.bias[p.tm ? f : s0 + q];
+            y = v + s[q];
+        }
+    }
+}
+
+template <typename XT, int MW>
 __global__ __launch_bounds__(kThreads) void mfma_init_kernel(MParams p, int xwgs) {
     __shared__ float tile[64][65];
     const MDesc& d = p.m[blockIdx.y];
-    const int M = p.M, tid = threadIdx.x;
     if ((int)blockIdx.x < xwgs) {
-        const int mw = min(64, p.Mpad);        // columns of a tile: 16, 32 or 64
-        const int nmt = p.Mpad / mw;
-        const int b = blockIdx.x / nmt, m0 = (blockIdx.x - b * nmt) * mw;
-        if (b >= d.NB) return;
-        const int n = 64 * mw;
-        // feature-major: threads along a feature's columns; token-major: along a column's features
-        // (four loads in flight per thread, at clamped columns)
-        for (int i0 = tid; i0 < n; i0 += 4 * kThreads) {  // n is a multiple of 4 kThreads
-            float v[4];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = i0 + e * kThreads;
-                const int k = p.tm ? (i & 63) : i / mw, c = p.tm ? (i >> 6) : i & (mw - 1);
-                v[e] = xget(p, d, b * 64 + k, min(m0 + c, M - 1));
-            }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int i = i0 + e * kThreads;
-                const int k = p.tm ? (i & 63) : i / mw, c = p.tm ? (i >> 6) : i & (mw - 1);
-                tile[k][c] = m0 + c < M ? v[e] : 0.0f;
-            }
-        }
-        __syncthreads();
-        for (int i = tid; i < mw * 8; i += kThreads) {
-            const int c = i & (mw - 1), g = i / mw;
-            _Float16 hi[8], lo[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float xv = tile[csdr::kperm64(g * 8 + j)][c];
-                hi[j] = (_Float16)xv;
-                lo[j] = (_Float16)(xv - (float)hi[j]);
-            }
-            const size_t o = xt_granule(p, b, m0 + c, g);
-            *reinterpret_cast<u32x4*>(d.xt + o) = __builtin_bit_cast(u32x4, hi);
-            if (!p.x_f16)
-                *reinterpret_cast<u32x4*>(d.xt + xt_part(p, d) + o) = __builtin_bit_cast(u32x4, lo);
-        }
+        init_x<XT, MW>(p, d, blockIdx.x, tile);
         return;
     }
     if (p.accumulate && !d.bias && d.Ce == 0) return;  // Y stays as it is
-    const size_t ny = (size_t)d.R * M;
+    const size_t ny = (size_t)d.R * p.M;
     const size_t stride = (size_t)(gridDim.x - xwgs) * kThreads;
-    if (!p.accumulate && !d.bias && d.Ce == 0) {
-        for (size_t t = (size_t)(blockIdx.x - xwgs) * kThreads + tid; t < ny; t += stride)
-            d.y[t] = 0.0f;
+    const size_t t0 = (size_t)(blockIdx.x - xwgs) * kThreads + threadIdx.x;
+    if (d.Ce > 0) {
+        if (ny > kEdgeWide) init_edge<XT, 4>(p, d, t0, stride);
+        else init_edge<XT, 1>(p, d, t0, stride);
         return;
     }
-    for (size_t t = (size_t)(blockIdx.x - xwgs) * kThreads + tid; t < ny; t += stride) {
-        const int r = p.tm ? (int)(t % d.R) : (int)(t / M);
-        const int m = p.tm ? (int)(t / d.R) : (int)(t - (size_t)r * M);
+    for (size_t t = t0; t < ny; t += stride) {
         float v = p.accumulate ? d.y[t] : 0.0f;
-        if (d.bias) v += d.bias[r];
-        if (d.Ce > 0) {
-            const float* e = d.edge + (size_t)r * d.Ce;
-            float s = 0.0f;
-            for (int cc = 0; cc < d.Ce; ++cc) s = fmaf(e[cc], xget(p, d, d.C_full + cc, m), s);
-            v += s;
-        }
+        if (d.bias) v += d.bias[p.tm ? t % d.R : t / p.M];
         d.y[t] = v;
     }
 }
@@ -1063,11 +1110,21 @@ int mfma_matmul(int n, const csdr_hsdb* const* segs, const void* const* xs, int 
             lds_max = v;
     }
     {
-        // a workgroup per block column and 64 columns of X, and some for Y
-        const size_t yper = any_edge ? kThreads : 4 * kThreads;  // edge strips: a sum per value
-        const int xwgs = max_nb * (p.Mpad / std::min(64, p.Mpad));
-        const int ywgs = (int)std::min<size_t>(1024, (max_y + yper - 1) / yper);
-        mfma_init_kernel<<<dim3(xwgs + std::max(ywgs, 1), n), kThreads, 0, st>>>(p, xwgs);
+        // a workgroup per block column and MW columns of X, and some for Y
+        const int mw = std::min(64, p.Mpad);
+        const size_t yper = any_edge && max_y <= kEdgeWide ? kThreads : 4 * kThreads;
+        const int xwgs = max_nb * (p.Mpad / mw);
+        const int ywgs = (int)std::min<size_t>(any_edge ? 4096 : 1024, (max_y + yper - 1) / yper);
+        const dim3 grid(xwgs + std::max(ywgs, 1), n);
+        auto go = [&](auto kern) { kern<<<grid, kThreads, 0, st>>>(p, xwgs); };
+        auto pick = [&](auto xt) {
+            using XT = decltype(xt);
+            if (mw == 64) go(&mfma_init_kernel<XT, 64>);
+            else if (mw == 32) go(&mfma_init_kernel<XT, 32>);
+            else go(&mfma_init_kernel<XT, 16>);
+        };
+        if (p.x_f16) pick(_Float16{});
+        else pick(float{});
         CSDR_LAUNCH_CHECK("hsdb mfma init");
     }
     const bool xsplit = !p.x_f16;

@@ -195,3 +195,29 @@ def test_decoded_tile_edges(gpu, M, R, Cc, K, s, dtype):
             for i, (y, ref) in enumerate(zip(ys, refs)):
                 want = ref + y0[i] + (b[i][:, None] if b else 0)
                 assert rel_l2(y, want) <= TOL
+
+
+# What the first launch writes: Y = (Y +) bias + edge strip . X in fp32, four outputs a thread
+# (rows of a column, or token-major columns of a row), with every code's coefficient zero so that
+# the matrix-core launch adds zeros only. Up to 63 products summed in fp32: 1e-6.
+@pytest.mark.parametrize("M,dtype", [(9, np.float32), (17, np.float16), (34, np.float32),
+                                     (101, np.float16), (259, np.float32)])
+@pytest.mark.parametrize("R,Ce", [(1, 63), (66, 1), (131, 7), (300, 44)])
+def test_edge_strip_alone(gpu, M, dtype, R, Ce):
+    from cortexsdr_amd import formats
+    from test_hsdb_multicol_gpu import ACCUMULATE, TOKEN_MAJOR, run_group
+
+    rng = np.random.default_rng(R + M)
+    edge = rng.standard_normal((R, Ce)).astype(np.float32)
+    D = synth.dictionary(32, 64, 1)
+    stream = formats.pack_hsdb(R, 64 + Ce, D, rng.integers(0, 32, (R, 4)), np.zeros((R, 4)),
+                               edge=edge)
+    x = rng.standard_normal((64 + Ce, M)).astype(dtype)
+    ref = edge.astype(np.float64) @ x[64:].astype(np.float64)
+    y0 = [rng.standard_normal((R, M)).astype(np.float32)]
+    bias = [rng.standard_normal(R).astype(np.float32)]
+    for flags in (0, TOKEN_MAJOR):
+        y = run_group(gpu, [stream], x, dtype, M, flags)[0]
+        assert rel_l2(y, ref) <= 1e-6
+        y = run_group(gpu, [stream], x, dtype, M, flags | ACCUMULATE, bias=bias, y0=y0)[0]
+        assert rel_l2(y, ref + y0[0] + bias[0][:, None]) <= 1e-6
