@@ -857,21 +857,64 @@ __global__ __launch_bounds__(kSwThreads) void q4k_sw_kernel(const uint8_t* __res
     }
 }
 
-// Which of the two M > 1 kernels. Up to 16 columns q4k_sw_kernel (us, q4k_mm_kernel with its
-// clearing launch first: 4096 x 14336 21.2 / 15.9, 4096^2 10.7 / 6.7, 14336 x 4096 24.5 / 21.5,
-// 300 x 14336 12.8 / 11.2, 896 x 1024 6.1 / 3.8). Past that its copy of X per 16 rows grows with
-// the columns, so it takes up to 64 of them while that is at most 14 chunks' time (rounds of
-// 256 workgroups x chunks of K: 4096 x 14336 M = 32 25.9 / 23.3, 4096^2 13.0 / 8.7 and at 64
-// 18.5 / 15.9, 1000 x 1024 at 64 9.8 / 5.0, but 14336 x 4096 M = 20 26 / 28, 4096 x 14336 M = 64
-// 36 / 42), except a long K with too few row tiles for the chip at 17 to 32 columns, where
-// q4k_mm_kernel splits K over the CUs (1024 x 14336 M = 32 15.6 / 17.1).
-bool sw_pays(int R, int nblk, int M) {
-    if (M <= 16) return true;
+int device_cus() {
+    int dev = 0, n = 0;
+    return hipGetDevice(&dev) == hipSuccess &&
+                   hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) ==
+                       hipSuccess &&
+                   n > 0
+               ? n
+               : 256;
+}
+
+// q4k_mm_kernel's launch: 64-row tiles of up to 64 columns; the super-blocks split in S parts (S
+// a power of two up to 8) so that the grid holds at least 256 workgroups where the row tiles alone
+// do not.
+struct MmLaunch {
+    MmGrid g;
+    int NT, gz;
+    long long nwg;
+};
+MmLaunch mm_launch(int R, int nblk, int M) {
+    MmLaunch l;
+    l.NT = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
+    l.gz = (M + 16 * l.NT - 1) / (16 * l.NT);
+    l.g.nrt = (R + kMmRows - 1) / kMmRows;
+    l.g.S = 1;
+    while (l.g.S < 8 && l.g.S < nblk && (long long)l.g.nrt * l.g.S * l.gz < 256) l.g.S *= 2;
+    l.g.KB = (nblk + l.g.S - 1) / l.g.S;
+    const int pad = 8 / l.g.S;
+    l.g.nrt_p = (l.g.nrt + pad - 1) / pad * pad;
+    l.nwg = (long long)l.g.nrt_p * l.g.S * l.gz;
+    return l;
+}
+
+// Which of the two M > 1 kernels: the one with the smaller estimate, from times of both over R 64
+// to 57344, 1 to 160 super-blocks a row and 2 to 64 columns (2,360 shapes; us a call).
+//   q4k_sw_kernel: one workgroup a CU, each with its start and its chunks of K: 7 + rounds x (1.95
+//     + 0.57 chunks), at two column tiles (2.73 + 0.84 chunks).
+//   q4k_mm_kernel: 7.4, or with S > 1 14 for the launch that clears Y and 3.6 per million values
+//     added into it; per super-block of a part 0.36 + 0.009 M, 1.5 times that where W's rows are a
+//     multiple of 1152 bytes apart (its row-per-lane loads meet in few memory channels), 2.56 times
+//     that per round of two workgroups a CU once there are more of them than CUs.
+// The choice costs 0.4% against always knowing the better one (at most 1.14 times mm's time, 14336 x
+// 20480 M = 64). A long K of few rows (1024 x 28672
+// M = 4: 16.8 us with mm, 18.6 with sw) and many rows of a short K (28672 x 1024 M = 32 13.7 /
+// 25.4, 14336 x 256 M = 48 7.7 / 25.8) go to mm; 4096 x 14336 M = 16 20.6 / 12.9 and M = 32 25.4 /
+// 18.4, 4096^2 M = 32 13 / 9, 5000 x 1024 M = 64 20.6 / 12.9 to sw. Past 64 columns sw's copy of
+// X per 16 rows is too much.
+bool sw_pays(int R, int nblk, int M, int ncu) {
     if (M > 64) return false;
-    const long long wgs = (long long)((R + kSwRows - 1) / kSwRows) * (M <= 32 ? 1 : 2);
-    const long long nch = (nblk + kSwSb - 1) / kSwSb;
-    if (M <= 32 && wgs < 128 && nch > 8) return false;
-    return (wgs + 255) / 256 * nch <= 14;
+    const int nt = M <= 16 ? 1 : 2;
+    const long long wgs = (long long)((R + kSwRows - 1) / kSwRows) * ((M + 16 * nt - 1) / (16 * nt));
+    const double rounds = (double)((wgs + ncu - 1) / ncu), chunks = (nblk + kSwSb - 1) / kSwSb;
+    const double sw = 7 + rounds * (nt == 1 ? 1.95 + 0.57 * chunks : 2.73 + 0.84 * chunks);
+    const MmLaunch l = mm_launch(R, nblk, M);
+    const long long n = (long long)l.g.nrt * l.g.S * l.gz;
+    const double per = (0.36 + 0.009 * M) * (nblk % 8 == 0 ? 1.5 : 1.0);
+    const double crowd = n <= ncu ? 1.0 : 2.56 * (double)((n + 2 * ncu - 1) / (2 * ncu));
+    const double fixed = l.g.S > 1 ? 14 + 3.6e-6 * M * R * l.g.S : 7.4;
+    return sw <= fixed + crowd * l.g.KB * per;
 }
 
 // ---------------------------------------------------------------- dequant to fp32
@@ -968,7 +1011,7 @@ CSDR_API int csdr_q4k_linear(const void* w, int R, int C, int order, const void*
             return set_error(CSDR_E_UNSUPPORTED, "q4k_linear: M > 1 takes fp16 x");
         if (reinterpret_cast<uintptr_t>(x) % 16 || C % 8)
             return set_error(CSDR_E_INVALID, "q4k_linear: x must be 16-byte aligned");
-        if (sw_pays(R, nblk, M)) {
+        if (sw_pays(R, nblk, M, device_cus())) {
             const auto* wq = static_cast<const uint8_t*>(w);
             const auto* xq = static_cast<const _Float16*>(x);
             const int nt = M <= 16 ? 1 : 2;
@@ -987,19 +1030,10 @@ CSDR_API int csdr_q4k_linear(const void* w, int R, int C, int order, const void*
             CSDR_LAUNCH_CHECK("q4k_linear");
             return CSDR_OK;
         }
-        // 64-row tiles of up to 64 columns; the super-blocks split in S parts (S a power of
-        // two up to 8) so that the grid holds at least 256 workgroups where the row tiles
-        // alone do not
-        const int NT = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
-        const int gz = (M + 16 * NT - 1) / (16 * NT);
-        MmGrid g;
-        g.nrt = (R + kMmRows - 1) / kMmRows;
-        g.S = 1;
-        while (g.S < 8 && g.S < nblk && (long long)g.nrt * g.S * gz < 256) g.S *= 2;
-        g.KB = (nblk + g.S - 1) / g.S;
-        const int pad = 8 / g.S;
-        g.nrt_p = (g.nrt + pad - 1) / pad * pad;
-        const long long nwg = (long long)g.nrt_p * g.S * gz;
+        const MmLaunch l = mm_launch(R, nblk, M);
+        const MmGrid& g = l.g;
+        const int NT = l.NT;
+        const long long nwg = l.nwg;
         if (nwg > 0x7fffffffLL)
             return set_error(CSDR_E_UNSUPPORTED, "q4k_linear: too many output tiles");
         if (g.S > 1) {

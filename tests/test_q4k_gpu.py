@@ -74,7 +74,8 @@ def test_linear(gpu, R, C, M, order, xdt):
 @pytest.mark.parametrize("order", ["ggml", "interleaved"])
 @pytest.mark.parametrize("R,nblk,M", [(16, 1, 2), (17, 2, 16), (33, 4, 17), (50, 5, 15),
                                       (15, 9, 31), (130, 23, 9), (100, 13, 32), (48, 33, 33),
-                                      (2050, 36, 20), (65, 3, 64), (40, 57, 20), (40, 57, 64)])
+                                      (2050, 36, 20), (65, 3, 64), (40, 57, 20), (40, 57, 64),
+                                      (30, 112, 4), (20000, 1, 18), (9000, 2, 50), (8200, 5, 2)])
 def test_linear_one_pass(gpu, R, nblk, M, order):
     from cortexsdr_amd import q4k
 
