@@ -802,7 +802,9 @@ int launch_mp(const float* tiles, long long n, int C, const float* D, int K, int
 //    order, each term fused (the reference's r[c] += scale * atom[c], :300-311), then tile -
 //    recon (:316-320). A workgroup per tile: its codes are uniform (scalar loads) and a thread
 //    keeps 4 elements, with the next slots' atom rows in flight (84 -> 24 us at 4864 x 896,
-//    24 slots: a thread per element with a 64-bit division each);
+//    24 slots: a thread per element with a 64-bit division each). Short tiles share one, 16
+//    threads each up to 64 elements and 64 up to 256 (16384 8 x 8 tiles 26 us a thread per
+//    element, 18.6 a workgroup each, 8.3 here; 32768 4 x 4 tiles 14.2, 34.6, 11.6);
 //  atom_sum_kernel: correction[c] = sum over the atom's users, in order, of sign * gamma *
 //    residual (double, fused: :428-437), the new value atom + correction * (0.5 / sum gamma^2)
 //    rounded to float (:448-458), in the atom's place (one that is not finite is re-seeded
@@ -957,17 +959,22 @@ __global__ __launch_bounds__(kEThreads) void users_fill_kernel(FitArgs a) {
     if (tid == 0) a.inv_w[j] = w <= 1e-12 ? 0.0 : 0.5 / w;
 }
 
+template <int LPT>
 __global__ __launch_bounds__(kEThreads) void residual_kernel(FitArgs a) {
     const int slots = a.S * a.k;
-    const uint16_t* cd = a.codes + (size_t)blockIdx.x * slots;
-    const float* x = a.tiles + (size_t)blockIdx.x * a.C;
-    float* out = a.res + (size_t)blockIdx.x * a.C;
-    for (int c0 = threadIdx.x; c0 < a.C; c0 += 4 * kEThreads) {
+    const long long tile =
+        LPT == kEThreads ? blockIdx.x
+                         : (long long)blockIdx.x * (kEThreads / LPT) + threadIdx.x / LPT;
+    if (tile >= a.n) return;
+    const uint16_t* cd = a.codes + (size_t)tile * slots;
+    const float* x = a.tiles + (size_t)tile * a.C;
+    float* out = a.res + (size_t)tile * a.C;
+    for (int c0 = threadIdx.x % LPT; c0 < a.C; c0 += 4 * LPT) {
         int c[4];
         float rec[4];
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            c[e] = min(c0 + e * kEThreads, a.C - 1);
+            c[e] = min(c0 + e * LPT, a.C - 1);
             rec[e] = 0.f;
         }
         int sl = 0;
@@ -984,7 +991,7 @@ __global__ __launch_bounds__(kEThreads) void residual_kernel(FitArgs a) {
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-            if (c0 + e * kEThreads < a.C) out[c0 + e * kEThreads] = x[c[e]] - rec[e];
+            if (c0 + e * LPT < a.C) out[c0 + e * LPT] = x[c[e]] - rec[e];
     }
 }
 
@@ -1267,7 +1274,13 @@ struct Refine {
         users_scan_kernel<<<1, kEThreads, 0, st>>>(fa);
         users_fill_kernel<<<K, kEThreads, 0, st>>>(fa);
         CSDR_LAUNCH_CHECK("hsdr_compress users");
-        residual_kernel<<<(unsigned)fa.n, kEThreads, 0, st>>>(fa);
+        const auto residual = [&](auto kern, int lpt) {
+            const long long per = kEThreads / lpt;
+            kern<<<(unsigned)((fa.n + per - 1) / per), kEThreads, 0, st>>>(fa);
+        };
+        if (C <= 64) residual(&residual_kernel<16>, 16);
+        else if (C <= 256) residual(&residual_kernel<64>, 64);
+        else residual(&residual_kernel<kEThreads>, kEThreads);
         CSDR_LAUNCH_CHECK("hsdr_compress residual");
         atom_sum_kernel<<<dim3(K, (C + kEThreads - 1) / kEThreads), kEThreads, 0, st>>>(fa);
         atom_finish_kernel<<<K, kEThreads, (size_t)C * 4, st>>>(fa);

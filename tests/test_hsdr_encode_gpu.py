@@ -220,9 +220,12 @@ def test_compress_refined_matches_reference(gpu, enc):
 # One refinement pass from the initial dictionary and codes, against its sums in numpy. The
 # device's residuals hold sqrt(S k) 2^-24 of a tile's norm in fp32 roundings, an atom's share of
 # which its users' mean takes to under 2e-6 of its length. Users of few atoms, more than a thread keeps from
-# one walk over the codes; code counts off the 8-code pieces; runs past one round of 64 codes.
+# one walk over the codes; code counts off the 8-code pieces; runs past one round of 64 codes;
+# tile lengths either side of 64 and 256, where 16, 64 or 256 threads take a tile's residual.
 @pytest.mark.parametrize("n,C,K,S,k", [(1003, 24, 3, 2, 3), (3001, 40, 40, 2, 5),
-                                       (2800, 16, 64, 3, 8), (61, 24, 5, 1, 5)])
+                                       (2800, 16, 64, 3, 8), (61, 24, 5, 1, 5),
+                                       (1501, 64, 20, 2, 4), (1103, 65, 20, 2, 4),
+                                       (899, 256, 12, 2, 3), (902, 257, 12, 2, 3)])
 def test_one_refinement_pass(gpu, n, C, K, S, k):
     from cortexsdr_amd import encode
 
