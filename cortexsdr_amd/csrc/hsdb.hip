@@ -513,16 +513,16 @@ __device__ void stage_x_m1(const Params& p, const MatDesc& d, int b0, int nb, fl
 }
 
 // Y initialisation for the gathers' accumulation: 0 or bias, or left as it is (+ bias), by
-// workgroup u of the n that the matrix has in the dx launch (NT threads each).
+// workgroup u of the n that the matrix has in the dx launch (NT threads each); M is p.M.
 template <int NT>
-__device__ __forceinline__ void init_y(const Params& p, const MatDesc& d, int u, int n) {
-    const size_t ytot = (size_t)d.R * p.M;
+__device__ __forceinline__ void init_y(const Params& p, const MatDesc& d, int u, int n, int M) {
+    const size_t ytot = (size_t)d.R * M;
     const size_t yper = (ytot + n - 1) / n;
     const size_t ye = min(ytot, (size_t)(u + 1) * yper);
     // (kept with no bias: nothing to do, and no read of y to wait for)
     if (!p.accumulate || d.bias) {
         for (size_t i = (size_t)u * yper + threadIdx.x; i < ye; i += NT) {
-            const float bv = d.bias ? d.bias[p.tm ? i % d.R : i / p.M] : 0.0f;
+            const float bv = d.bias ? d.bias[M == 1 ? i : p.tm ? i % d.R : i / M] : 0.0f;
             d.y[i] = p.accumulate ? d.y[i] + bv : bv;
         }
     }
@@ -539,7 +539,7 @@ __global__ __launch_bounds__(kThreads) void dx_kernel(Params p) {
     const int u = wg - d.dx_base;
     const int tid = threadIdx.x;
     const int M = p.M;
-    init_y<kThreads>(p, d, u, d.dx_count);
+    init_y<kThreads>(p, d, u, d.dx_count, M);
     {
         // 16 lanes per atom: lane l holds D[a][4l .. 4l+3] (one coalesced 16-byte load; a
         // wave reads 4 whole rows). The x range of this workgroup is staged in LDS in one
@@ -625,7 +625,7 @@ __global__ __launch_bounds__(kThreads) void dxw_kernel(Params p) {
     const MatDesc& d = p.m[g];
     const int u = (int)blockIdx.x - d.dg_base;
     const int lane = threadIdx.x & 63;
-    init_y<kThreads>(p, d, u, d.dg_count);
+    init_y<kThreads>(p, d, u, d.dg_count, 1);
     const long long item = (long long)u * (kThreads / 64) + (threadIdx.x >> 6);  // b * K + a
     if (item >= (long long)d.NB * d.K) return;
     const int b = (int)(item / d.K), a = (int)(item - (long long)b * d.K);
@@ -658,7 +658,7 @@ __global__ __launch_bounds__(kDgThreads) void dxg_kernel(Params p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lg = lane >> 4;
     const int M = p.M;
-    init_y<kDgThreads>(p, d, u, d.dg_count);
+    init_y<kDgThreads>(p, d, u, d.dg_count, M);
     const int na = (d.K + 15) / 16, nm = (M + 15) / 16;
     const int at = u % na, mt = u / na % nm, b = u / na / nm;
     const int a = min(at * 16 + li, d.K - 1), m = min(mt * 16 + li, M - 1);
@@ -728,7 +728,7 @@ __global__ __launch_bounds__(kDgThreads) void dxg_kernel(Params p) {
 // combine is staged for the workgroup's blocks in LDS first (stage_x_m1).
 template <int XOP, int NT>
 __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
-        typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
     constexpr int kAtoms = NT / 4;  // 16 per wave
     int g = 0;
     while (g + 1 < p.G && wg >= p.m[g + 1].dx_base) ++g;
@@ -736,18 +736,7 @@ __device__ __forceinline__ void dx1_body(const Params& p, int wg) {
     const int u = wg - d.dx_base;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int li = lane & 15, lg = lane >> 4;
-    {
-        const size_t ytot = (size_t)d.R;
-        const size_t yper = (ytot + d.dx_count - 1) / d.dx_count;
-        const size_t ye = min(ytot, (size_t)(u + 1) * yper);
-        // (kept with no bias: nothing to do, and no read of y to wait for)
-        if (!p.accumulate || d.bias) {
-            for (size_t i = (size_t)u * yper + tid; i < ye; i += NT) {
-                const float bv = d.bias ? d.bias[i] : 0.0f;
-                d.y[i] = p.accumulate ? d.y[i] + bv : bv;
-            }
-        }
-    }
+    init_y<NT>(p, d, u, d.dx_count, 1);
     const int na = (d.K + kAtoms - 1) / kAtoms;
     const int ag = u % na, bg = u / na;
     const int a = min(ag * kAtoms + wave * 16 + li, d.K - 1);
@@ -897,7 +886,7 @@ constexpr int kXsStride = 68;
 
 template <int XOP, int MC>
 __global__ __launch_bounds__(kThreads) void dxmm_kernel(Params p) {
-        static_assert(MC == 2 || MC == 4 || MC == 8 || MC == 16, "MC");
+    static_assert(MC == 2 || MC == 4 || MC == 8 || MC == 16, "MC");
     static_assert(kThreads == 256, "one X element per thread and pass");
     constexpr int BPT = 16 / MC;  // block columns per N tile
     __shared__ __attribute__((aligned(16))) float xs[16 * kXsStride];
@@ -915,8 +904,8 @@ __global__ __launch_bounds__(kThreads) void dxmm_kernel(Params p) {
     // dictionary operand first (the longest round trip), then the X tile
     f32x4 dv[4];
     {
-        const f32x4* src = reinterpret_cast<const f32x4*>(d.dict + (size_t)min(a0 + li, d.K - 1) * 64 +
-                                                    lg * 16);
+        const f32x4* src = reinterpret_cast<const f32x4*>(
+            d.dict + (size_t)min(a0 + li, d.K - 1) * 64 + lg * 16);
 #pragma unroll
         for (int i = 0; i < 4; ++i) dv[i] = src[i];
     }
@@ -1149,10 +1138,9 @@ __device__ __forceinline__ void gatherw_body(const Params& p, int wg) {
     if constexpr (P4) {
         // nontemporal: the slice was just streamed out by the dx launch (headline step 15.35 ->
         // 14.72 us; a gather that re-reads a slice still in its L2 is slower this way)
-        typedef float f32x4v __attribute__((ext_vector_type(4)));
-        const f32x4v* sv = reinterpret_cast<const f32x4v*>(Pg);
+        const f32x4* sv = reinterpret_cast<const f32x4*>(Pg);
         auto ld = [&](int i) {
-            const f32x4v v = __builtin_nontemporal_load(sv + i);
+            const f32x4 v = __builtin_nontemporal_load(sv + i);
             return make_float4(v.x, v.y, v.z, v.w);
         };
         pv0 = ld(min(tid, np4 - 1));
@@ -1275,7 +1263,7 @@ template <int SLOTS, int MC, int TD, int LPR, bool P16, typename TileFn>
 __device__ __forceinline__ void gatherv_stream(const MatDesc& d, const float* Ps, float* rowt,
                                                u32x4 (*buf)[SLOTS / 4], TileFn tile, int nk,
                                                int wfirst, int ntiles) {
-        typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef float f2 __attribute__((ext_vector_type(2)));
     constexpr int PPB = SLOTS / 4;
     constexpr int G = MC / 4;
     constexpr int kStep = 64;
@@ -1343,7 +1331,8 @@ __device__ __forceinline__ void gatherv_stream(const MatDesc& d, const float* Ps
             if constexpr (MC >= 4) {
 #pragma unroll
                 for (int m4 = 0; m4 < MC; m4 += 4)
-                    *reinterpret_cast<f32x4*>(rt + m4) = f32x4{acc[m4], acc[m4 + 1], acc[m4 + 2], acc[m4 + 3]};
+                    *reinterpret_cast<f32x4*>(rt + m4) =
+                        f32x4{acc[m4], acc[m4 + 1], acc[m4 + 2], acc[m4 + 3]};
             } else {
 #pragma unroll
                 for (int m = 0; m < MC; ++m) rt[m] = acc[m];
@@ -1437,20 +1426,18 @@ void gatherv_kernel(Params p) {
     // the P round trip and the barrier.
     constexpr int NBUF = TD + 1;
     u32x4 buf[NBUF][PPB];
-        if (P16 || (M == MC && (d.K * MC) % 4 == 0)) {
+    if (P16 || (M == MC && (d.K * MC) % 4 == 0)) {
         // P slice: global [block][atom][M] (fp16 P: [block][atom][8] halves) -> LDS, a
         // straight copy of 16-byte pieces (at most 8 per thread: one round trip)
         const f32x4* Pg = P16 ? reinterpret_cast<const f32x4*>(d.P) + (size_t)b0 * d.K
-                           : reinterpret_cast<const f32x4*>(d.P + (size_t)b0 * d.K * M);
+                              : reinterpret_cast<const f32x4*>(d.P + (size_t)b0 * d.K * M);
         f32x4* Pl = reinterpret_cast<f32x4*>(Ps);
         const int n4 = nbc * d.K * (P16 ? 4 : MC) / 4;
         for (int i0 = 0; i0 < n4; i0 += kGThreads * 8) {
             f32x4 v[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) {  // nontemporal, as the M == 1 gather's P slice
-                typedef float f32x4v __attribute__((ext_vector_type(4)));
-                v[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4v*>(Pg) +
-                                                  min(i0 + j * kGThreads + tid, n4 - 1));
+                v[j] = __builtin_nontemporal_load(Pg + min(i0 + j * kGThreads + tid, n4 - 1));
             }
             if (i0 == 0) {
 #pragma unroll
