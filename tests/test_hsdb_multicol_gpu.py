@@ -181,7 +181,7 @@ def test_any_block_length_and_slots(gpu, B, slots, M, flags, dtype):
     assert rel_l2(ys[0], want[0]) <= 1e-5
     ys = run_group(gpu, streams, x, dtype, M, flags | ACCUMULATE, bias=bias, y0=y0)
     for y, w, b, a in zip(ys, want, bias, y0):
-        assert rel_l2(y, a + w + b[:, None]) <= (1e-3 if B == 64 and M > 8 else 1e-5)
+        assert rel_l2(y, a + w + b[:, None]) <= 1e-5
 
 
 # An infinite x makes P infinite for every atom: with positive atoms and coefficients all of Y is
