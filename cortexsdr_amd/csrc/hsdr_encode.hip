@@ -66,9 +66,8 @@ struct MpArgs {
     uint16_t* codes;     // n x S*k, packIndexSign
     long long n;
     int C, K, S, k, tt;
-    const int* list;   // mp_list_kernel: *count tiles by number, up to `few` of them one a workgroup
+    const int* list;   // mp_list_kernel: *count tiles by number
     const int* count;
-    int few;
     float gamma[kMaxStages];
 };
 
@@ -94,10 +93,11 @@ __device__ __forceinline__ void load_tiles(const float* rc, float* rv) {
     }
 }
 
-// The nt tiles first, first + 1, ... or (LIST) list[first], list[first + 1], ...
-template <int TT, bool LIST>
+// The nt tiles first, first + 1, ... or (LIST) list[first], list[first + 1], ...; kNA atoms per
+// 16-lane group at a time.
+template <int TT, bool LIST, int kNA = TT <= 2 ? 8 : 2>
 __device__ __forceinline__ void mp_tiles(const MpArgs& a, long long first, int nt) {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];  // (wide reads, load_tiles)
     const int tt = TT, C = a.C, K = a.K;
     float* r = smem;                                                    // C x TT residuals
     float* proj = r + (size_t)tt * C;                                   // nt x K scores
@@ -115,11 +115,10 @@ __device__ __forceinline__ void mp_tiles(const MpArgs& a, long long first, int n
         const int c = i / TT, t = i - c * TT;
         r[i] = t < nt ? a.tiles[number(t) * C + c] : 0.f;
     }
-    // atoms per 16-lane group at a time: 8 with up to 2 tiles (D blocks of 4 chunks), 2 with
+    // kNA: 8 with up to 2 tiles (D blocks of 4 chunks), 2 with
     // more (registers; measured 896 x 896 at 2 tiles: 0.60 ms with 2, 0.51 with 4, 0.45 with 8;
     // 4864 x 896 at 4 tiles: 3.48 ms with 2, 4.01 with 4)
-    constexpr int kNA = TT <= 2 ? 8 : 2;
-    constexpr int kDB = kNA >= 8 ? 4 : 8;  // chunks of an atom loaded per block
+    constexpr int kDB = kNA >= 4 ? 4 : 8;  // chunks of an atom loaded per block
     const int C16 = C & ~15, C8 = C & ~7;  // end of the 16-element chunks, of the 8-element one
     const int nch = C16 / 16;  // full 16-element chunks (block loads clamp into them)
     const int slots = a.S * a.k;
@@ -245,20 +244,29 @@ __global__ __launch_bounds__(kEThreads) void mp_kernel(MpArgs a) {
     mp_tiles<TT, false>(a, t0, (int)min((long long)TT, a.n - t0));
 }
 
-// The tiles that mp_gram_kernel leaves (list, count): up to `few` of them one a workgroup, more
-// of them (a matrix of equal or parallel rows, whose atoms are all alike, leaves every tile) TT at
-// a time as mp_kernel takes them; two kernels, each launched and one of them returning at once,
-// since one with both bodies had neither's registers. (4864 x 896, K = 512, 24 picks, rows of one
-// value each: 9.2 ms with one tile a workgroup throughout, 3.8 here, 3.4 with mp_kernel alone.)
+// The tiles that mp_gram_kernel leaves (list, count): one a workgroup up to kListFew of them,
+// where a pick is a chain of round trips; past that (equal or parallel rows, whose atoms are all
+// alike) TT at a time as mp_kernel takes them, since every workgroup reads all of D per pick and
+// L2's rate bounds it (4864 x 896, K = 512, 24 picks, rows of one value each: 9.3 ms with one tile a
+// workgroup throughout, 3.7 here, 3.4 with mp_kernel alone). With TT = 2, what mp_kernel takes
+// below 4096 tiles, one at a time stays the faster (600 x 128, K = 512, 4 picks 103 us, 124).
+// Beside the other form single tiles take 4 atoms at a time, and that form has a workgroup for
+// every TT tiles that may be left: with 8, or with a loop, the registers leave it fewer waves (5.3
+// ms).
+constexpr int kListFew = 256;
+
 template <int TT>
 __global__ __launch_bounds__(kEThreads) void mp_list_kernel(MpArgs a) {
     const int n = *a.count;
-    if ((TT == 1) != (n <= a.few)) return;
     if constexpr (TT == 1) {
         for (int b = blockIdx.x; b < n; b += gridDim.x) mp_tiles<1, true>(a, b, 1);
     } else {
-        const int first = blockIdx.x * TT;
-        if (first < n) mp_tiles<TT, true>(a, first, min(TT, n - first));
+        const int b = blockIdx.x;
+        if (n <= kListFew) {
+            if (b < n) mp_tiles<1, true, 4>(a, b, 1);
+        } else if (b * TT < n) {
+            mp_tiles<TT, true>(a, b * TT, min(TT, n - b * TT));
+        }
     }
 }
 
@@ -444,7 +452,7 @@ __device__ __forceinline__ float wave_max(float v) {
 
 template <int KPL>
 __global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
-    extern __shared__ float smem[];
+    extern __shared__ __attribute__((aligned(16))) float smem[];
     const int C = a.C, K = a.K, lane = threadIdx.x, slots = a.S * a.k;
     float* r = smem;                                           // C: the exact residual, when needed
     float* hgam = r + C;                                       // slots: gamma * sign of the picks
@@ -715,12 +723,9 @@ int launch_mp_gram(const float* tiles, long long n, int C, const float* D, int K
     b.list = count + 1;
     for (int l = 0; l < S; ++l) a.gamma[l] = b.gamma[l] = gamma[l];
     const size_t lds = gram_lds_bytes(C, S, k);
-    // (from 4096 tiles on; below, two tiles a workgroup gain less than the second launch costs)
     const int tt = mp_tiles_per_wg(n, C, K);
-    b.few = tt >= 4 ? 1024 : 0x7fffffff;
-    const auto list = [&](auto kern, int per, long long most) {
-        kern<<<(unsigned)((most + per - 1) / per), kEThreads, mp_lds_bytes(per, C, K), st>>>(b);
-    };
+    const int list_tt = tt >= 4 ? tt : 1;
+    const size_t list_lds = mp_lds_bytes(list_tt, C, K);  // (no more than the soft limit)
     for (long long t0 = 0; t0 < n; t0 += chunk) {
         const long long nt = std::min(chunk, n - t0);
         a.tiles = b.tiles = tiles + (size_t)t0 * C;
@@ -733,11 +738,13 @@ int launch_mp_gram(const float* tiles, long long n, int C, const float* D, int K
         else if (K <= 512) mp_gram_kernel<8><<<grid, 64, lds, st>>>(a);
         else if (K <= 1024) mp_gram_kernel<16><<<grid, 64, lds, st>>>(a);
         else mp_gram_kernel<32><<<grid, 64, lds, st>>>(a);
-        list(&mp_list_kernel<1>, 1, std::min<long long>(nt, 1024));
-        if (nt > b.few) {
-            if (tt == 8) list(&mp_list_kernel<8>, 8, nt);
-            else list(&mp_list_kernel<4>, 4, nt);
-        }
+        const long long lgrid = list_tt == 1
+                                    ? std::min<long long>(nt, 1024)
+                                    : std::max<long long>((nt + list_tt - 1) / list_tt,
+                                                          std::min<long long>(nt, kListFew));
+        if (list_tt == 8) mp_list_kernel<8><<<(unsigned)lgrid, kEThreads, list_lds, st>>>(b);
+        else if (list_tt == 4) mp_list_kernel<4><<<(unsigned)lgrid, kEThreads, list_lds, st>>>(b);
+        else mp_list_kernel<1><<<(unsigned)lgrid, kEThreads, list_lds, st>>>(b);
         CSDR_LAUNCH_CHECK("hsdr_encode");
     }
     return CSDR_OK;

@@ -108,11 +108,13 @@ def test_encode_ties_and_odd_tiles_match_oracle(gpu, monkeypatch, n, C, K, S, k)
     assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), oracle.hsdr_mp(t, D, g, S, k))
 
 
-# Tiles left to projections, by the thousand: in the first chunk of tiles (2^24 / K) more than the
-# 1024 that go one a workgroup, a count off the tiles per workgroup (4 at K = 2048, 8 at K = 64),
-# and in a second chunk, whose tiles and codes are at an offset, a few.
+# Tiles left to projections, by the hundred and the thousand: in the first chunk of tiles (2^24 / K)
+# either side of the 256 that go one a workgroup, a count off the tiles per workgroup (4 at K =
+# 2048, 8 at K = 64), and in a second chunk, whose tiles and codes are at an offset, a few.
 @pytest.mark.parametrize("n,C,K,S,k,n_left", [(8192 + 300, 8, 2048, 2, 2, 1201),
-                                              (9001, 24, 64, 2, 3, 9001)])
+                                              (9001, 24, 64, 2, 3, 9001),
+                                              (8192 + 9, 8, 2048, 1, 3, 256),
+                                              (5000, 20, 64, 2, 2, 257)])
 def test_encode_many_tiles_left_match_oracle(gpu, monkeypatch, n, C, K, S, k, n_left):
     monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
     rng = np.random.default_rng(n + K)
@@ -122,7 +124,7 @@ def test_encode_many_tiles_left_match_oracle(gpu, monkeypatch, n, C, K, S, k, n_
     left = rng.permutation(min(n, 8192) if n_left < n else n)[:n_left]
     t[left] *= np.where(rng.random((n_left, 1)) < 0.5, 1e-15, 1e15).astype(np.float32)
     if n_left < n:
-        t[8192 + 17:8192 + 60:3] *= np.float32(1e15)
+        t[8192 + 2:8192 + 60:3] *= np.float32(1e15)
     g = (0.5 ** np.arange(S)).astype(np.float32)
     assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), oracle.hsdr_mp(t, D, g, S, k))
 
