@@ -703,11 +703,11 @@ __global__ __launch_bounds__(1024) void qroute_kernel(MParams p) {
 //   past the range's end wrap), as in qroute_kernel.
 // Bound by the LDS at many columns (per 64-row unit of 8 slots and 256 columns 136 KiB read or
 // written, about 1,350 of its 2,000 cycles; matrix cores 512, vector ALU 560), and by the chain of
-// a unit's reads, multiply-adds and writes at few; beside the units a 256-column call of 68 us
-// spends 9 in the init launch, 8 before the first unit and 9 in the atomics into Y.
+// a unit's reads, multiply-adds and writes at few; beside the units a 256-column call of 63 us
+// spends 4 in the init launch, 8 before the first unit and 9 in the atomics into Y.
 // 4096 x 11008, K = 1024, 8 slots, us per call before (each wave decoding its own rows, X through
-// LDS) and after: fp16 X M = 32 40.2 -> 34, 64 48.2 -> 41.4, 128 63.7 -> 54.5, 256 90.7 -> 68;
-// fp32 X M = 32 41.6 -> 35.5, 64 53 -> 48.5, 128 78 -> 69, 256 156 -> 88.
+// LDS) and after: fp16 X M = 32 40.2 -> 31.4, 64 48.2 -> 35, 128 63.7 -> 49.7, 256 90.7 ->
+// 62.6; fp32 X M = 32 41.6 -> 33.8, 64 53 -> 45.6, 128 78 -> 64.7, 256 156 -> 83.
 constexpr int kDecWaves = 8;
 
 template <int ROWS, int RG, int CG, int CT, bool XS, int SLOTS>
