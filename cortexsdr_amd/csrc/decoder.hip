@@ -172,6 +172,7 @@ struct csdr_decoder {
     float *pf_a = nullptr, *pf_g = nullptr, *pf_u = nullptr, *pf_w = nullptr;
     float* pf_s = nullptr;          // the split form's token planes, row scales and partial sums
     int* pf_tok = nullptr;
+    bool use_split = true;          // CSDR_DECODER_SPLIT=0: passes in the fp32 form only
     bool pf_eligible = false;       // the blocks took the split form when the buffers were made
     bool pf_split = false;          // the buffers hold it
     // on-demand layer streaming (blocks of host-resident segments)
@@ -424,6 +425,7 @@ constexpr int kMinSplitRows = 8;  // fewer: a row of W per wave (csdr_dense_line
 
 // The prefill's split form (split_gemm.hpp) needs every block's matrices in its layout.
 bool prefill_split(const csdr_decoder* d) {
+    if (!d->use_split) return false;
     for (const Layer& L : d->layers)
         for (const csdr_hsdb* w : {L.q, L.k, L.v, L.o, L.gate, L.up, L.down})
             if (!csdr::split_eligible(w)) return false;
@@ -833,6 +835,7 @@ CSDR_API int csdr_decoder_create_batched(const csdr_decoder_config* cfg, int bat
     d->layers.resize(c.n_layers);
     if (const char* e = getenv("CSDR_DECODER_GRAPH")) d->use_graph = atoi(e) != 0;
     if (const char* e = getenv("CSDR_DECODER_FUSED")) d->fused = atoi(e) != 0;
+    if (const char* e = getenv("CSDR_DECODER_SPLIT")) d->use_split = atoi(e) != 0;
     d->attn_splits = csdr_attn_decode_splits_kv(B, c.n_heads, c.n_kv_heads, c.head_dim, c.max_ctx,
                                                 c.kv_dtype);
     int rc = CSDR_OK;

@@ -433,9 +433,9 @@ CSDR_API int csdr_dense_linear(const float* w, int R, int C, const float* x, int
                                void* hip_stream);
 /* As csdr_dense_linear, plus bias (R floats, may be NULL) and flags (CSDR_HSDB_ACCUMULATE:
  * y += x . W^T + bias). M >= 8 (C % 4 == 0, w and x 16-byte aligned) runs on the fp32 matrix
- * cores (v_mfma_f32_16x16x4_f32, fp32 accumulation); smaller M one wave per row of W. The
- * decoder's batched prefill multiplies the prompt rows by each coded weight decoded once with
- * csdr_hsdb_decompress through this call. */
+ * cores (v_mfma_f32_16x16x4_f32, fp32 accumulation); smaller M one wave per row of W. One of
+ * the decoder's two prefill forms multiplies the prompt rows by each coded weight decoded once
+ * with csdr_hsdb_decompress through this call. */
 CSDR_API int csdr_dense_linear_ex(const float* w, int R, int C, const float* x, int M, float* y,
                                   const float* bias, int flags, void* hip_stream);
 /* y = silu(g) * u (silu_mul, cortex_sdk.cpp:1245-1256). */
@@ -679,9 +679,13 @@ CSDR_API int csdr_decoder_set_output(csdr_decoder* dec, const csdr_hsdb* lm_head
 /* Runs the prompt from position 0 (resetting the cache and the generated-token set) and
  * selects the first new token (it lands at position n_prompt). prompt: batch x n_prompt ids.
  * Positions 0 .. n_prompt - 2 run as multi-token passes of up to the prefill chunk tokens per
- * sequence (csdr_decoder_set_prefill_chunk): every weight decoded once per pass to dense fp32
- * and multiplied on the matrix cores for all the pass's tokens, causal prompt attention
- * (csdr_attn_prefill); the last prompt position runs the decode step, which selects. */
+ * sequence (csdr_decoder_set_prefill_chunk): every weight decoded once per pass and multiplied
+ * on the matrix cores for all the pass's tokens, causal prompt attention (csdr_attn_prefill);
+ * the last prompt position runs the decode step, which selects. Passes of 8 rows or more over
+ * blocks of 64-long codes (at most 16384 columns) multiply in pairs of fp16 values, with fp32
+ * sums and an error against exact arithmetic no larger than the fp32 form's; others, decoders
+ * created with CSDR_DECODER_SPLIT=0 in the environment, and passes whose pairs find no device
+ * memory, decode to dense fp32 and multiply in fp32. */
 CSDR_API int csdr_decoder_prefill(csdr_decoder* dec, const int32_t* prompt, int n_prompt,
                                   float temperature, float penalty);
 /* Token choice by the text CLI's lazy HSDR scoring (select_next_token_from_lazy_hsdr,
@@ -693,8 +697,9 @@ CSDR_API int csdr_decoder_prefill(csdr_decoder* dec, const int32_t* prompt, int 
 CSDR_API int csdr_decoder_set_lazy_selection(csdr_decoder* dec, const csdr_lazy_hsdr* emb,
                                              float penalty);
 /* Tokens per sequence in one prefill pass (default 512); 0 runs every prompt position as a
- * decode step instead (the token-at-a-time form). Buffers for B x chunk rows and one dense
- * weight (the largest, F x H fp32) are allocated at the first prefill that needs them. */
+ * decode step instead (the token-at-a-time form). Buffers for B x chunk rows and the decoded
+ * weights of one input (gate and up: 2 F x H fp32 in pairs; the fp32 form's one weight F x H) are
+ * allocated at the first prefill that needs them. */
 CSDR_API int csdr_decoder_set_prefill_chunk(csdr_decoder* dec, int tokens);
 /* n_steps further tokens, one graph replay each; synchronises at the end. */
 CSDR_API int csdr_decoder_decode(csdr_decoder* dec, int n_steps, float temperature,

@@ -208,11 +208,12 @@ def test_decoder_prefill_passes_match_token_at_a_time(gpu, B):
 # tiles per thread of the decode, parts of the contraction, one block only (no product but k
 # and v). Against the token-at-a-time prefill, which sums in fp32 too: two forms of a few
 # blocks' fp32 sums differ by some 1e-6 a product, so 1e-4 as above.
+# With CSDR_DECODER_SPLIT=0 the passes run in the fp32 form: the same bar between the two forms.
 @pytest.mark.parametrize("layers,heads,ffn,nnz,n_prompt", [
     (2, 3, 200, 4, 9), (2, 2, 1100, 6, 71), (2, 1, 2200, 8, 140), (1, 2, 64, 8, 33),
     (3, 14, 136, 16, 66),
 ])
-def test_prefill_product_edges(gpu, layers, heads, ffn, nnz, n_prompt):
+def test_prefill_product_edges(gpu, monkeypatch, layers, heads, ffn, nnz, n_prompt):
     from cortexsdr_amd.decoder import Decoder, DecoderSpec, synthetic_weights
 
     spec = DecoderSpec(layers, 64 * heads, heads, 1, 64, ffn, 333, n_prompt + 8)
@@ -226,6 +227,13 @@ def test_prefill_product_edges(gpu, layers, heads, ffn, nnz, n_prompt):
             runs.append(_run(dec, prompt, 3))
         finally:
             dec.close()
+    monkeypatch.setenv("CSDR_DECODER_SPLIT", "0")
+    dec = Decoder(w, prefill_chunk=512)
+    try:
+        runs.append(_run(dec, prompt, 3))
+    finally:
+        dec.close()
+    assert not np.array_equal(runs[1][0][0], runs[3][0][0])  # another form, not the same one
     _compare(runs, 3, 1e-4)
 
 
