@@ -491,7 +491,7 @@ __global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
             const float v = x[c] / mx;
             n2 = fmaf(v, v, n2);
         }
-    float n0 = mx > 0.f ? mx * __builtin_amdgcn_sqrtf(csdr::wave_sum(n2)) * 1.01f : 0.f;
+    const float n0 = mx > 0.f ? mx * __builtin_amdgcn_sqrtf(csdr::wave_sum(n2)) * 1.01f : 0.f;
     const auto leave = [&] {
         if (lane == 0) a.list[atomicAdd(a.count, 1)] = tile;
     };
@@ -500,13 +500,15 @@ __global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
         leave();
         return;
     }
-    // a zero tile's residual stays exactly zero while its pick, atom 0, is all zeros: n0 of 0 says
-    // so, kZeroNorm that the first pick ends it
-    constexpr float kZeroNorm = 1e-38f;
+    // a zero tile whose first pick, atom 0, is all zeros too stays zero: atom 0 at every pick
     if (n0 == 0.f) {
         bool live = false;
         for (int c = lane; c < C; c += 64) live |= a.D[c] != 0.f;
-        if (__any(live)) n0 = kZeroNorm;
+        for (int l = 0; l < a.S; ++l) live |= !(fabsf(a.gamma[l]) < INFINITY);  // 0 * inf
+        if (!__any(live)) {
+            for (int q = lane; q < slots; q += 64) a.codes[(size_t)tile * slots + q] = 0;
+            return;
+        }
     }
     const float u = 1.25f * 5.9604645e-8f * dmax;
     float rn2 = n0 * n0, nmax2 = rn2, len = 0.f;
@@ -556,8 +558,8 @@ __global__ __launch_bounds__(64) void mp_gram_kernel(GramArgs a) {
                             __builtin_amdgcn_readlane(__builtin_bit_cast(int, s[i]), src));
                     }
                 sg = sv >= 0.f ? 1 : -1;
-            } else if (n0 <= kZeroNorm && (t == 0 || n0 == 0.f)) {
-                // a zero residual: every projection is 0, atom 0 stands
+            } else if (n0 == 0.f && t == 0) {
+                // a zero tile: every projection is 0, atom 0 stands
             } else if (nc > kGramMaxCand) {
                 leave();
                 return;

@@ -129,10 +129,11 @@ def test_encode_many_tiles_left_match_oracle(gpu, monkeypatch, n, C, K, S, k, n_
     assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), oracle.hsdr_mp(t, D, g, S, k))
 
 
-@pytest.mark.parametrize("zero_atom", [True, False])
-def test_encode_zero_tiles_match_oracle(gpu, monkeypatch, zero_atom):
+@pytest.mark.parametrize("zero_atom,scale", [(True, 1.0), (False, 1.0), (True, np.inf)])
+def test_encode_zero_tiles_match_oracle(gpu, monkeypatch, zero_atom, scale):
     """Zero tiles where atom 0, their first pick, is all zeros (it then stands at every pick), and
-    where it is not, its values as small as fp32 holds included."""
+    where it is not, its values as small as fp32 holds included; and with an infinite stage
+    scale, which makes NaN of the zeros."""
     monkeypatch.delenv("CSDR_HSDR_TILES_PER_WG", raising=False)
     n, C, K, S, k = 300, 100, 200, 3, 4
     rng = np.random.default_rng(5)
@@ -145,9 +146,9 @@ def test_encode_zero_tiles_match_oracle(gpu, monkeypatch, zero_atom):
     D[12, 99] = 1e-38
     if not zero_atom:
         D[0, 70] = 1e-30
-    g = (0.5 ** np.arange(S)).astype(np.float32)
+    g = (scale * 0.5 ** np.arange(S)).astype(np.float32)
     want = oracle.hsdr_mp(t, D, g, S, k)
-    assert zero_atom == (not want.reshape(n, -1)[::2].any())
+    assert (zero_atom and scale == 1.0) == (not want.reshape(n, -1)[::2].any())
     assert np.array_equal(gpu_codes(gpu, t, D, g, S, k), want)
 
 
